@@ -65,7 +65,8 @@ int hpd_inverse_lower(int n, double* A, i64 lda, int nb, int* dinfo, void* scrat
         double* A21 = A11 + b;
         double* A20 = A + k0 + b;
         double* A22 = A11 + b + (i64)b * lda;
-        ELEMAMD_HIP_TRY(launch_potrf_unb<double>(b, A11, lda, dinfo, k0, s));
+        ELEMAMD_HIP_TRY(n <= nb ? launch_potrf_unb<double>(b, A11, lda, dinfo, k0, s)
+                                : launch_potrf_block_f64(b, A11, lda, dinfo, k0, s));
         ELEMAMD_HIP_TRY(block_inverse(n <= nb, b, A11, lda, false, Xs, nullptr, dinfo, s));
         if (j > 0)  // W = X11 A10
             ELEMAMD_HIP_TRY(launch_gemm_f64(false, false, b, j, b, 1.0, Xs, kLdX, Lo, A10, lda, F, 0.0, Ws, ldw, 0,

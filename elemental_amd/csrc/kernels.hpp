@@ -15,6 +15,8 @@ constexpr int kNoLimit = 0x7fffffff;
 // global column col_offset (skips if an earlier column failed).
 template <typename T>
 hipError_t launch_potrf_unb(int n, T* A, i64 lda, int* info, int col_offset, hipStream_t s);
+// the diagonal block of a blocked FP64 factorization (LVar3Unb up to rounding order)
+hipError_t launch_potrf_block_f64(int n, double* A, i64 lda, int* info, int col_offset, hipStream_t s);
 
 // trsm_panel.hip -- B := B * inv(L)^T, L nb x nb lower (nb <= 128), B m x nb.
 template <typename T>

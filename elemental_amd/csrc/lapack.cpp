@@ -139,7 +139,9 @@ int cholesky_lower(int n, T* A, i64 lda, int nb, int trailing, int* dinfo, hipSt
                 }
             }
             if constexpr (sizeof(T) == 8) {
-                ELEMAMD_HIP_TRY(launch_potrf_unb<T>(b, Akk, lda, dinfo, k, s));
+                // a single block keeps LVar3Unb's rounding order (bit for bit)
+                ELEMAMD_HIP_TRY(n <= nb ? launch_potrf_unb<T>(b, Akk, lda, dinfo, k, s)
+                                        : launch_potrf_block_f64(b, (double*)Akk, lda, dinfo, k, s));
                 if (n - k - b > 0)
                     ELEMAMD_HIP_TRY(launch_panel_f64(n - k - b, b, (const double*)Akk, lda, (double*)Akk + b, lda,
                                                      dinfo, k + b, s));

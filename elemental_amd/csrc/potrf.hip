@@ -19,6 +19,7 @@
 // Storage may be double or float (the mixed-precision factor keeps its
 // working matrix in float); arithmetic is always double.
 #include "common.hpp"
+#include "diag16_dev.hpp"
 #include "kernels.hpp"
 #include "potrf_dev.hpp"
 
@@ -35,6 +36,26 @@ template <typename T>
 hipError_t launch_potrf_unb(int n, T* A, i64 lda, int* info, int col_offset, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(potrf_unb_kernel<T>, dim3(1), dim3(kPotrfThreads), 0, s, n, A, lda, info, col_offset);
+    return hipGetLastError();
+}
+
+// The diagonal block of a blocked FP64 factorization (diag16_dev.hpp): same
+// result as LVar3Unb up to rounding order.  n = 128: 25 us alone and 44 us
+// beside the trailing update at n = 16384, against 78 and 128 us of
+// potrf_unb_kernel, which stays where the reference's rounding order is kept
+// bit for bit (a single block, n <= nb).
+__global__ __launch_bounds__(diag16::kThreads) void potrf_block_kernel(int n, double* __restrict__ A, i64 lda,
+                                                                       int* __restrict__ info, int col_offset) {
+    __shared__ diag16::Lds sh;
+    __builtin_amdgcn_s_setprio(2);  // chain kernel (see potrf_unb_kernel)
+    if (info != nullptr && *info != 0 && *info <= col_offset) return;
+    diag16::factor_block<double, false>(sh, n, A, lda, nullptr, info, col_offset);
+}
+
+hipError_t launch_potrf_block_f64(int n, double* A, i64 lda, int* info, int col_offset, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    if (n > 128) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(potrf_block_kernel, dim3(1), dim3(diag16::kThreads), 0, s, n, A, lda, info, col_offset);
     return hipGetLastError();
 }
 

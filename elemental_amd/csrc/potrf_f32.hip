@@ -3,12 +3,9 @@
 // (include/elemental/lapack-like/Cholesky/LVar3.hpp:83-123, LVar3Unb at :19-49)
 // and the panel solve L21 := A21 L11^{-T}.  Two kernels:
 //
-// potrf_f32_kernel -- one workgroup, the block in LDS as float, right-looking
-//   in 32-column steps: wave 0 factors the 32 x 32 diagonal piece in FP64;
-//   all waves invert it (recursive doubling, FP64) and multiply the rows
-//   below by the inverse (FP64 MFMA), then apply the rank-32 update to the
-//   rest of the block (FP32 MFMA).  A block narrower than 128 is padded with
-//   the identity.
+// potrf_f32_kernel -- one workgroup, the block in FP64 registers
+//   (diag16_dev.hpp), stored back as float with the inverses of its 32 x 32
+//   diagonal pieces.
 // panel_f32_kernel -- one 64-row slab per workgroup, with the inverses of
 //   the four 32 x 32 diagonal pieces of L11 (by the diagonal-block kernel):
 //   each wave solves its 16 rows block by block,
@@ -19,147 +16,13 @@
 //   preconditions).  With planes requested the result is also written as
 //   bf16 hi/lo planes for the split-BF16x3 updates.
 #include "common.hpp"
+#include "diag16_dev.hpp"
 #include "kernels.hpp"
 #include "solve_dev.hpp"
 
 namespace elemamd {
 
 constexpr int kPiLd = 132;  // LDS row stride (floats): MFMA operand reads are conflict-free
-
-// One wave: factor the 32 x 32 block of sA at (c0, c0) in FP64 into sD
-// (transposed) and back into sA as float, with the reciprocal diagonal in sRd.
-// Returns 0, or the 1-based failing column.
-// Lane (h, i) = (lane / 32, lane % 32) holds columns 16h .. 16h+15 of row i.
-// Column j travels through LDS (the wave's own writes and reads, in order;
-// two buffers by column parity so the next column's write need not wait for
-// this column's reads): its owners publish the entries below the pivot
-// (zeros above it) and the pivot, every lane reads the pivot and the 16
-// entries of its half, and the rank-1 update runs unmasked because the
-// published zeros leave finished entries unchanged.  Each update starts with
-// the next column's entry, so its publication can overlap the rest.  The
-// pivot's reciprocal square root is the hardware estimate refined by one
-// Newton step (error far below the float the factor is stored in) and is
-// kept, so nothing divides.
-__device__ inline int factor32(float (*sA)[kPiLd], double (*sD)[34], double (*sCol)[34], double* sRd, int c0,
-                               int lane) {
-    // an opaque copy of the lane index keeps the compiler from hoisting the
-    // per-lane masks of all four calls out of the caller's loop (it ran out
-    // of registers doing so)
-    int lv = lane;
-    asm volatile("" : "+v"(lv));
-    const int i = lv & 31, hh = lv >> 5;
-    double d[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) d[q] = (double)sA[c0 + i][c0 + 16 * hh + q];
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-        const int jh = j >> 4, jq = j & 15;
-        double* col = sCol[j & 1];
-        int jv = j;  // opaque per column: the lane masks are made here, not all up front
-        asm volatile("" : "+s"(jv));
-        const bool own = hh == (jv >> 4), diag = i == jv;
-        if (own) col[i] = (i > jv) ? d[jq] : 0.0;
-        // the column's readers are other lanes of this wave: the wave
-        // barrier keeps every read below the store (without it the compiler
-        // may read in the non-owners' branch, ahead of the owners' store)
-        __builtin_amdgcn_wave_barrier();
-        // the pivot comes straight from its lane's register (no LDS round
-        // trip on the test); the 16 column entries are read in one batch
-        const int pl = 32 * jh + j;
-        const double piv = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(d[jq]), pl),
-                                            __builtin_amdgcn_readlane(__double2loint(d[jq]), pl));
-        const double cij = col[i];
-        double ck[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) ck[q] = col[16 * hh + q];
-        if (!(piv > 0.0)) return j + 1;
-        double y = __builtin_amdgcn_rsq(piv);
-        y = fma(y, fma(-0.5 * piv * y, y, 0.5), y);
-        const double lij = cij * y;
-        if (own) d[jq] = diag ? piv * y : lij;
-        const double sij = lij * y;  // a_ij / a_jj: one multiplier for the whole row
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int q = (jq + 1 + u) & 15;  // the next column's entry first
-            d[q] = fma(-sij, ck[q], d[q]);
-        }
-        if (lv == 0) sRd[j] = y;
-    }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int k = 16 * hh + q;
-        sD[k][i] = (k <= i) ? d[q] : 0.0;  // transposed: column k of L is a row of sD
-        sA[c0 + i][c0 + k] = (k <= i) ? (float)d[q] : 0.0f;
-    }
-    return 0;
-}
-
-// All threads: X = inv(L) of the piece factored by factor32 (FP64, L in sD
-// transposed, 1/L_kk in sRd) by recursive doubling over diagonal blocks of
-// size b = 1, 2, 4, 8, 16:  for L = [L11 0; L21 L22],
-//     X21 = -X22 (L21 X11)
-// with X11, X22 already inverted; every element of a level is one thread (a
-// dot of length <= b), so the 32-step chain of a substitution becomes 10
-// short steps.  sX: row-major, zero above the diagonal; sT: scratch.
-__device__ inline void invert32(const double (*sD)[34], const double* sRd, double (*sX)[33], double (*sT)[33],
-                                int t) {
-    for (int e = t; e < 1024; e += 256) {
-        const int i = e >> 5, j = e & 31;
-        sX[i][j] = (i == j) ? sRd[i] : 0.0;
-    }
-    __syncthreads();
-    for (int b = 1; b < 32; b *= 2) {
-        const int ne = 16 * b;  // elements of all the level's X21 blocks
-        const int q = t / (b * b), i = (t % (b * b)) / b, j = t % b;
-        const int r0 = 2 * b * q, rb = r0 + b;
-        if (t < ne) {  // T = L21 X11 (X11 lower: m >= j)
-            double acc = 0.0;
-            for (int m = j; m < b; ++m) acc = fma(sD[r0 + m][rb + i], sX[r0 + m][r0 + j], acc);
-            sT[rb + i][r0 + j] = acc;
-        }
-        __syncthreads();
-        if (t < ne) {  // X21 = -X22 T (X22 lower: m <= i)
-            double acc = 0.0;
-            for (int m = 0; m <= i; ++m) acc = fma(sX[rb + i][rb + m], sT[rb + m][r0 + j], acc);
-            sX[rb + i][r0 + j] = -acc;
-        }
-        __syncthreads();
-    }
-}
-
-// All threads: the rows below the piece, r in [c0 + 32, 128), columns
-// c0 .. c0 + 31 of sA := A L^{-T} = A X^T with X = inv(L) (FP64 MFMA
-// 16x16x4, 16 x 16 output tiles dealt to the waves).  Every wave reads its
-// operands, then the workgroup synchronises, then results overwrite sA.
-__device__ inline void below_times_xt(float (*sA)[kPiLd], const double (*sX)[33], int c0, int w, int lane) {
-    const int m = lane & 15, g = lane >> 4;
-    const int ntile = 2 * ((96 - c0) / 16);  // row tiles x 2 column tiles
-    double fa[3][8], fb[3][8];
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-        const int tt = w + 4 * u, rt = tt >> 1, ct = tt & 1;
-        const int ra = tt < ntile ? c0 + 32 + 16 * rt + m : 127;  // clamped when the tile does not exist
-#pragma unroll
-        for (int kb = 0; kb < 8; ++kb) {
-            fa[u][kb] = (double)sA[ra][c0 + 4 * kb + g];  // A[i = m][k = 4 kb + g]
-            fb[u][kb] = sX[16 * ct + m][4 * kb + g];      // B[k][j = m] = X[j][k]
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-        const int tt = w + 4 * u, rt = tt >> 1, ct = tt & 1;
-        if (tt >= ntile) continue;
-        d4_t acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int kb = 0; kb < 8; ++kb) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[u][kb], fb[u][kb], acc, 0, 0, 0);
-        // a dependent zero-operand MFMA right before the accumulator is read
-        // (the wait states between an FP64 MFMA and a read of its result)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(0.0, 0.0, acc, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) sA[c0 + 32 + 16 * rt + g + 4 * v][c0 + 16 * ct + m] = (float)acc[v];
-    }
-}
 
 // acc (16 x 16) += P (16 x 32) Q^T: rows pr.. of P from column pc, rows qr..
 // of Q from column qc, both row-major in LDS; all 16 operand loads are in
@@ -180,77 +43,18 @@ __device__ inline void tile_ab_t(f4_t& acc, const float (*P)[LP], int pr, int pc
 // One b x b (b <= 128) diagonal block at A (float storage): L11 overwrites
 // its lower triangle, the inverses of its four 32 x 32 diagonal pieces go to
 // Xd (4 x 32 x 32 floats, row-major).  A failing pivot records
-// col_offset + column in *info.
-__global__ __launch_bounds__(256) void potrf_f32_kernel(int b, float* __restrict__ A, i64 lda,
-                                                        float* __restrict__ Xd, int* __restrict__ info,
-                                                        int col_offset) {
-    __shared__ float sA[128][kPiLd];
-    __shared__ double sD[32][34];  // the FP64 factor of the current piece, transposed
-    __shared__ double sCol[2][34], sRd[32];
-    __shared__ double sX[32][33], sT[32][33];  // the current piece's inverse, scratch
-    __shared__ int sfail;
+// col_offset + column in *info.  b = 128: 25 us alone, 37 us beside the
+// trailing update at n = 16384; the form before it (the block as float in
+// LDS, 32-column pieces through LDS, 94 KB) took 56 and 70 us.
+__global__ __launch_bounds__(diag16::kThreads) void potrf_f32_kernel(int b, float* __restrict__ A, i64 lda,
+                                                                     float* __restrict__ Xd, int* __restrict__ info,
+                                                                     int col_offset) {
+    __shared__ diag16::Lds sh;
     // the factorization's chain: its waves issue ahead of the trailing
     // update's waves sharing the SIMD (wave priority, not queue priority)
-    __builtin_amdgcn_s_setprio(3);
+    __builtin_amdgcn_s_setprio(2);
     if (info != nullptr && *info != 0 && *info <= col_offset) return;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, m = lane & 15, g = lane >> 4;
-    {
-        // element e = t + 256 q: row e % 128, column e / 128; all 64 loads from
-        // clamped (in-bounds) addresses in flight together, then selected into LDS
-        float v[64];
-        const int r = t & 127;
-        const i64 rr = r < b ? r : b - 1;
-#pragma unroll
-        for (int q = 0; q < 64; ++q) {
-            const int c = (t >> 7) + 2 * q;
-            v[q] = A[rr + (i64)(c < b ? c : b - 1) * lda];
-        }
-#pragma unroll
-        for (int q = 0; q < 64; ++q) {
-            const int c = (t >> 7) + 2 * q;
-            sA[r][c] = (r < b && c < b) ? (c <= r ? v[q] : 0.0f) : (r == c ? 1.0f : 0.0f);
-        }
-    }
-    if (t == 0) sfail = 0;
-    __syncthreads();
-    for (int p = 0; p < 4; ++p) {
-        const int c0 = 32 * p;
-        if (w == 0) {
-            const int f = factor32(sA, sD, sCol, sRd, c0, lane);
-            if (f != 0 && lane == 0) sfail = c0 + f;
-        }
-        __syncthreads();
-        if (sfail != 0) break;
-        invert32(sD, sRd, sX, sT, t);
-        for (int e = t; e < 1024; e += 256) Xd[p * 1024 + e] = (float)sX[e >> 5][e & 31];
-        below_times_xt(sA, sX, c0, w, lane);
-        __syncthreads();
-        // rank-32 update of the rest of the block (lower 16 x 16 tiles)
-        const int nrt = (96 - c0) / 16;
-        const int ntl = nrt * (nrt + 1) / 2;
-        for (int tt = w; tt < ntl; tt += 4) {
-            int ti = 0;
-            while ((ti + 1) * (ti + 2) / 2 <= tt) ++ti;
-            const int tj = tt - ti * (ti + 1) / 2;
-            const int r0 = c0 + 32 + 16 * ti, q0 = c0 + 32 + 16 * tj;
-            f4_t acc = {};
-            tile_ab_t(acc, sA, r0, c0, sA, q0, c0, m, g);
-            mfma_retire();
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int r = r0 + 4 * g + v, q = q0 + m;
-                if (q <= r) sA[r][q] -= acc[v];
-            }
-        }
-        __syncthreads();
-    }
-    const int fail = sfail;
-#pragma unroll 4
-    for (int idx = t; idx < 128 * 128; idx += 256) {
-        const int r = idx & 127, c = idx >> 7;
-        if (r < b && c <= r) A[r + (i64)c * lda] = sA[r][c];
-    }
-    if (fail != 0 && t == 0 && info != nullptr) *info = col_offset + fail;
+    diag16::factor_block<float, true>(sh, b, A, lda, Xd, info, col_offset);
 }
 
 // Rows rw .. rw+15 of a panel slab (staged in sB) -= P_slab P_top^T: the
@@ -527,7 +331,7 @@ __global__ __launch_bounds__(256) void panel_f32_kernel(int m, int b, const floa
 
 hipError_t launch_potrf_f32(int b, float* A, i64 lda, float* Xd, int* info, int col_offset, hipStream_t s) {
     if (b <= 0) return hipSuccess;
-    hipLaunchKernelGGL(potrf_f32_kernel, dim3(1), dim3(256), 0, s, b, A, lda, Xd, info, col_offset);
+    hipLaunchKernelGGL(potrf_f32_kernel, dim3(1), dim3(diag16::kThreads), 0, s, b, A, lda, Xd, info, col_offset);
     return hipGetLastError();
 }
 
