@@ -41,11 +41,13 @@ constexpr int kWaves = 8;             // tile rows of a 128-column block
 constexpr int kThreads = 64 * kWaves;
 constexpr int kXLd = 130;             // LDS column stride of the solved tiles (rows of the block)
 
+template <bool INV>
 struct Lds {
+    static constexpr int kV = INV ? kWaves : 2;  // without the inverses two diagonal tiles alternate
     double X[16][kXLd];        // the piece's solved tiles, [column of the piece][row of the block]
     double D[16][18];          // the diagonal tile before its factorization, by rows
     double M[16][18];          // [c][k]: l_ck / l_kk for c > k, else 0 (the piece's multipliers)
-    double V[kWaves][16][17];  // per wave: its diagonal tile's unscaled columns [column][row]; then its inverse (INV)
+    double V[kV][16][17];      // wave w, [w % kV]: its diagonal tile's unscaled columns [column][row]; then its inverse (INV)
     int bad;
 };
 
@@ -147,7 +149,7 @@ __device__ __forceinline__ void update_cols(double (&d)[16], double l) {
 // column stays in registers once it is applied.
 template <int K>
 struct Column {
-    static __device__ __forceinline__ void run(double (&d)[16], double r, int i, bool& good, Lds& sh,
+    static __device__ __forceinline__ void run(double (&d)[16], double r, int i, bool& good, double (*M)[18],
                                                double (*V)[17]) {
         V[K][i] = d[K];
         if constexpr (K < 15) {
@@ -172,8 +174,8 @@ struct Column {
             update_cols<K + 11, 16>(d, l);
             int k = K;  // opaque: 15 hoisted lane masks would not fit the scalar registers
             asm volatile("" : "+s"(k));
-            sh.M[i][K] = i > k ? lr : 0.0;
-            Column<K + 1>::run(d, rn, i, good, sh, V);
+            M[i][K] = i > k ? lr : 0.0;
+            Column<K + 1>::run(d, rn, i, good, M, V);
         }
     }
 };
@@ -223,7 +225,8 @@ struct InvCol<16> {
 // 0-based failing column of the piece, or 16.  On return sh.X holds the
 // piece's columns (the diagonal tile's rows among them), columns from the
 // failing one on as they stood when it failed.
-__device__ __forceinline__ int piece_careful(Lds& sh, int p, int nrows) {
+template <bool INV>
+__device__ __forceinline__ int piece_careful(Lds<INV>& sh, int p, int nrows) {
 #pragma clang fp contract(off)
     const int t = threadIdx.x, r0 = 16 * p, row = r0 + t;
     if (t < 16)
@@ -251,7 +254,7 @@ __device__ __forceinline__ int piece_careful(Lds& sh, int p, int nrows) {
 // col_offset + column (1-based) in *info.  INV: the inverses of the block's
 // 32 x 32 diagonal pieces also go to Xd (4 x 32 x 32, row-major).
 template <typename T, bool INV>
-__device__ __forceinline__ void factor_block(Lds& sh, int b, T* __restrict__ A, i64 lda, float* __restrict__ Xd,
+__device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict__ A, i64 lda, float* __restrict__ Xd,
                                              int* __restrict__ info, int col_offset) {
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -285,22 +288,30 @@ __device__ __forceinline__ void factor_block(Lds& sh, int b, T* __restrict__ A, 
     }
     // tile (w, q) of the factor, from its rows of sh.X
     auto store_tile = [&](int q) __attribute__((always_inline)) {
+        // (opaque lane: the addresses are made here, not kept in registers
+        // across the loop)
+        int lv = lane;
+        asm volatile("" : "+v"(lv));
+        const int cs = lv & 15, gs = lv >> 4, col = 16 * q + cs;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int row = 16 * w + g + 4 * v, col = 16 * q + c;
-            if (row < b && col < b) A[row + (i64)col * lda] = (T)sh.X[c][row];
+            const int row = 16 * w + gs + 4 * v;
+            if (row < b && col < b) A[row + (i64)col * lda] = (T)sh.X[cs][row];
         }
     };
     int failed = 0;  // 1-based failing column of the block
     for (int p = 0; p < np; ++p) {
         if (w == p) {
             __builtin_amdgcn_s_setprio(3);
+            int lv = lane;  // (opaque, as in store_tile)
+            asm volatile("" : "+v"(lv));
+            const int c = lv & 15;
             double d[16];
 #pragma unroll
             for (int q = 0; q < 16; ++q) d[q] = sh.D[c][q];
             const double piv = bcast<0>(d[0]);
             bool good = __builtin_amdgcn_class(piv, 0x180);
-            Column<0>::run(d, rsqrt_full(piv), c, good, sh, sh.V[w]);
+            Column<0>::run(d, rsqrt_full(piv), c, good, sh.M, sh.V[w % Lds<INV>::kV]);
             if (!good && lane == 0) sh.bad = 1;
             __builtin_amdgcn_s_setprio(2);
         }
@@ -315,7 +326,7 @@ __device__ __forceinline__ void factor_block(Lds& sh, int b, T* __restrict__ A, 
                 double m[16], a[4] = {t[0][0], t[0][1], t[0][2], t[0][3]};
 #pragma unroll
                 for (int k = 0; k < 16; ++k) m[k] = sh.M[c][k];  // (the last one is not used)
-                const double rv = rsqrt_full(sh.V[p][c][c]);
+                const double rv = rsqrt_full(sh.V[p % Lds<INV>::kV][c][c]);
                 // (the copies above end two wait states before the first DPP read)
                 asm volatile("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
                 TileColumn<0>::run(a, m);
@@ -336,7 +347,7 @@ __device__ __forceinline__ void factor_block(Lds& sh, int b, T* __restrict__ A, 
             if (kend < 16) failed = 16 * p + kend + 1;
             if (w == p) {
 #pragma unroll 1
-                for (int q = 0; q < 16; ++q) sh.V[w][q][c] = sh.X[q][16 * w + c];
+                for (int q = 0; q < 16; ++q) sh.V[w % Lds<INV>::kV][q][c] = sh.X[q][16 * w + c];
             }
             if (failed) {
                 if (w > p && w < np) store_tile(p);
@@ -368,7 +379,10 @@ __device__ __forceinline__ void factor_block(Lds& sh, int b, T* __restrict__ A, 
             if (p > 0 && !careful) store_tile(p - 1);
             // the diagonal tile's columns, scaled by the reciprocal roots; l_kk
             // is the root itself, pivot * r with one correction
-            double pv = sh.V[w][c][c], rv = 1.0;
+            int lv = lane;  // (opaque, as in store_tile)
+            asm volatile("" : "+v"(lv));
+            const int c = lv & 15, g = lv >> 4;
+            double pv = sh.V[w % Lds<INV>::kV][c][c], rv = 1.0;
             if (kend == 16 && !careful) {
                 rv = rsqrt_full(pv);
                 const double s = pv * rv;
@@ -378,18 +392,21 @@ __device__ __forceinline__ void factor_block(Lds& sh, int b, T* __restrict__ A, 
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int r = g + 4 * v;
-                l[v] = r == c ? pv : sh.V[w][c][r] * rv;
+                l[v] = r == c ? pv : sh.V[w % Lds<INV>::kV][c][r] * rv;
                 const int row = 16 * p + r, col = 16 * p + c;
                 if (row < b && c <= r) A[row + (i64)col * lda] = (T)l[v];
             }
             if constexpr (INV) {
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int v = 0; v < 4; ++v) sh.V[w][c][g + 4 * v] = l[v];
+                for (int v = 0; v < 4; ++v) sh.V[w % Lds<INV>::kV][c][g + 4 * v] = l[v];
             }
         }
         if (failed) {
             // the rest of the block as the failing column left it
+            int lv = lane;  // (opaque, as in store_tile)
+            asm volatile("" : "+v"(lv));
+            const int c = lv & 15, g = lv >> 4;
             if (w > p && w < np)
 #pragma unroll
                 for (int J = 1; J < kWaves; ++J)

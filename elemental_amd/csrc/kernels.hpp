@@ -55,7 +55,7 @@ hipError_t launch_syrk_ln_f64(int m, int n, int k, double alpha, const double* A
 // float storage; bf16x3 = false: FP32 MFMA, true: split-BF16x3 MFMA with FP32 accumulation.
 hipError_t launch_syrk_ln_f32(bool bf16x3, int m, int n, int k, float alpha, const float* A, i64 lda, const float* B,
                               i64 ldb, float beta, float* C, i64 ldc, const int* info, int kcol0, int nbp,
-                              hipStream_t s);
+                              hipStream_t s, bool beside_chain = false);
 
 // Split-BF16 from pre-split panels: np bf16 planes of the panel (plane p at
 // planes + p*ps, row-major, row stride ldk a multiple of 32), made by

@@ -50,13 +50,15 @@ static hipError_t syrk_launch(int trailing, int m, int n, int k, const T* A, i64
                                   info, kcol0, nbp, s, beside_chain);
     else
         return launch_syrk_ln_f32(trailing == kTrailingBf16x3, m, n, k, -1.0f, (const float*)A, lda, (const float*)A,
-                                  lda, 1.0f, (float*)C, ldc, info, kcol0, nbp, s);
+                                  lda, 1.0f, (float*)C, ldc, info, kcol0, nbp, s, beside_chain);
 }
 
-// update depth (columns per trailing pass)
+// update depth (columns per trailing pass) of a group that starts with `rem`
+// columns left
 template <typename T>
-static int update_depth(int trailing) {
-    return sizeof(T) == 8 ? kUpdateDepthF64 : (trailing == kTrailingF32 ? kUpdateDepthF32 : kUpdateDepthBf16x3);
+static int update_depth(int trailing, int rem) {
+    if (sizeof(T) == 8) return rem > kUpdateDepthF64Rem ? kUpdateDepthF64Large : kUpdateDepthF64;
+    return trailing == kTrailingF32 ? kUpdateDepthF32 : kUpdateDepthBf16x3;
 }
 
 // bf16 planes of the float factor's panels (two alternating sets) and the
@@ -67,7 +69,7 @@ static int plane_count(int nb, int trailing) {
 static size_t plane_region_bytes(int n, int nb, int trailing) {
     const int np = plane_count(nb, trailing);
     if (np == 0 || n <= 0) return 0;
-    const int G = std::max(1, update_depth<float>(trailing) / nb);
+    const int G = std::max(1, update_depth<float>(trailing, n) / nb);
     const i64 gw = std::min<i64>((i64)G * nb, n);
     const i64 ldk = (gw + 31) / 32 * 32;
     return (2 * (size_t)np * (size_t)n * (size_t)ldk * sizeof(unsigned short) + 255) & ~(size_t)255;
@@ -86,9 +88,13 @@ int cholesky_lower(int n, T* A, i64 lda, int nb, int trailing, int* dinfo, hipSt
     if (n == 0) return kOk;
     StreamPair* sp = stream_pair(s);
     if (sp == nullptr) return kErrHip;
-    const int G = std::max(1, update_depth<T>(trailing) / nb);
-    const i64 gw64 = (i64)G * nb;
-    const int gw = (int)std::min<i64>(gw64, n);
+    // columns of the group that starts at column c (the float factor's groups
+    // are all of one width: its planes are laid out for it)
+    auto width = [&](int c) {
+        const int G = std::max(1, update_depth<T>(trailing, n - c) / nb);
+        return (int)std::min<i64>((i64)G * nb, n - c);
+    };
+    const int gw = width(0);
     // split-BF16x3 / x6: the panel solve also writes its result as 2 / 3
     // bf16 planes (row-major, rows from the group's first column down), which
     // every update of the group reads: the in-group block-column updates, the
@@ -115,8 +121,8 @@ int cholesky_lower(int n, T* A, i64 lda, int nb, int trailing, int* dinfo, hipSt
     }
     int group = 0;
     bool rest_pending = false;
-    for (int c0 = 0; c0 < n; c0 += gw, ++group) {
-        const int c1 = (int)std::min<i64>(n, (i64)c0 + gw);
+    for (int c0 = 0, c1; c0 < n; c0 = c1, ++group) {
+        c1 = c0 + width(c0);
         unsigned short* Pl = nullptr;  // this group's planes (stride plane_elems), row 0 = matrix row c0
         if (planes) Pl = pbuf + (size_t)(group & 1) * np * plane_elems;
         // the group's block columns, in order
@@ -163,7 +169,7 @@ int cholesky_lower(int n, T* A, i64 lda, int nb, int trailing, int* dinfo, hipSt
         const int kg = c1 - c0;
         const T* P = A + c1 + (i64)c0 * lda;  // the group's panels below it, m2 x kg
         T* C = A + c1 + (i64)c1 * lda;        // trailing matrix, m2 x m2
-        const int bn = std::min(gw, m2);      // next group's block columns
+        const int bn = width(c1);             // next group's block columns
         if (rest_pending) ELEMAMD_HIP_TRY(hipStreamWaitEvent(s, sp->ev_b, 0));
         if (group == 0 && trailing_ready != nullptr) ELEMAMD_HIP_TRY(hipStreamWaitEvent(s, trailing_ready, 0));
         if (planes) Pl += (i64)(c1 - c0) * ldk;  // rows from c1 on
@@ -750,7 +756,7 @@ int mixed_factor(int n, const double* A, i64 lda, const MixedOpts& o, MixedFacto
     // the float copy: the first group of block columns on the caller's
     // stream, the columns right of it on aux under that group's factor steps
     // (the factorization waits for them before its first trailing update)
-    const int gw = std::min(n, std::max(1, update_depth<float>(o.trailing) / std::max(1, o.nb)) * o.nb);
+    const int gw = std::min(n, std::max(1, update_depth<float>(o.trailing, n) / std::max(1, o.nb)) * o.nb);
     // the solve preparation (diagonal-block inverses, sweep operands) of each
     // 512-column block on aux3 once the factorization has made that block's
     // columns final; it reads only the lower triangle

@@ -16,7 +16,12 @@ enum : int { kRefineIR = 0, kRefineCG = 1 };
 
 // Columns of panels applied per pass over the trailing matrix (a multiple of
 // the block size nb is used: max(1, depth / nb) panels).
-constexpr int kUpdateDepthF64 = 256;
+// FP64: 512 while more than 8192 columns are left (the trailing update sets
+// the pace and runs at 61 TF/s instead of 54), 256 below (the chain sets the
+// pace, and a deeper group has more of it).  n = 16384 solve: 256 throughout
+// 40.2 ms, 512 throughout 39.2, the change at 4096, 6144 or 8192 columns 38.4,
+// at 10240 38.6; n = 2048: 256 1.78 ms, 512 1.85.
+constexpr int kUpdateDepthF64 = 256, kUpdateDepthF64Large = 512, kUpdateDepthF64Rem = 8192;
 constexpr int kUpdateDepthF32 = 512;
 constexpr int kUpdateDepthBf16x3 = 512;
 

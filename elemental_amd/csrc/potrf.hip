@@ -44,9 +44,9 @@ hipError_t launch_potrf_unb(int n, T* A, i64 lda, int* info, int col_offset, hip
 // beside the trailing update at n = 16384, against 78 and 128 us of
 // potrf_unb_kernel, which stays where the reference's rounding order is kept
 // bit for bit (a single block, n <= nb).
-__global__ __launch_bounds__(diag16::kThreads) void potrf_block_kernel(int n, double* __restrict__ A, i64 lda,
+__global__ __launch_bounds__(diag16::kThreads, 4) void potrf_block_kernel(int n, double* __restrict__ A, i64 lda,
                                                                        int* __restrict__ info, int col_offset) {
-    __shared__ diag16::Lds sh;
+    __shared__ diag16::Lds<false> sh;
     __builtin_amdgcn_s_setprio(2);  // chain kernel (see potrf_unb_kernel)
     if (info != nullptr && *info != 0 && *info <= col_offset) return;
     diag16::factor_block<double, false>(sh, n, A, lda, nullptr, info, col_offset);

@@ -46,10 +46,10 @@ __device__ inline void tile_ab_t(f4_t& acc, const float (*P)[LP], int pr, int pc
 // col_offset + column in *info.  b = 128: 25 us alone, 37 us beside the
 // trailing update at n = 16384; the form before it (the block as float in
 // LDS, 32-column pieces through LDS, 94 KB) took 56 and 70 us.
-__global__ __launch_bounds__(diag16::kThreads) void potrf_f32_kernel(int b, float* __restrict__ A, i64 lda,
+__global__ __launch_bounds__(diag16::kThreads, 4) void potrf_f32_kernel(int b, float* __restrict__ A, i64 lda,
                                                                      float* __restrict__ Xd, int* __restrict__ info,
                                                                      int col_offset) {
-    __shared__ diag16::Lds sh;
+    __shared__ diag16::Lds<true> sh;
     // the factorization's chain: its waves issue ahead of the trailing
     // update's waves sharing the SIMD (wave priority, not queue priority)
     __builtin_amdgcn_s_setprio(2);

@@ -9,16 +9,25 @@
 // src/core/imports/blas.cpp:1043-1050).  The strictly upper triangle of C is
 // never read or written.
 //
-// CDNA4 mapping: one 256-thread workgroup per 128x128 lower tile of C (for a
-// square C the grid enumerates only the T(T+1)/2 lower tiles; otherwise it is
-// Tm x Tn and tiles above the diagonal exit), four waves each owning a 64x64
-// quadrant as 4x4 MFMA blocks
-// of 16x16.  K is streamed through double-buffered LDS in chunks of 16.
+// FP64 and FP32: one 256-thread workgroup per 64 x 64 lower tile of C
+// (tile64_dev.hpp; for a square C the grid enumerates only the T(T+1)/2 lower
+// tiles; otherwise it is Tm x Tn and tiles above the diagonal exit).
+// Measured (m x m update of depth k, one launch; before: 128 x 128 tiles with
+// addresses formed per load):
+//   FP64  m = 1024, k = 256: 19 us (54);  m = 8192, k = 256: 322 us (412);
+//         m = 15872, k = 256: 54 TF/s (48), k = 512: 61 TF/s (54)
+//   FP32  m = 1024, k = 256: 14 us (38);  m = 8192, k = 512: 92 TF/s (83)
+// 128-row tiles with the same loop measured less at every size in FP64 (m =
+// 15872, k = 512: 128 x 64 55.7, 128 x 128 54.5 TF/s): fewer waves share a
+// CU's matrix pipes.  A super-tile order per XCD changed nothing at k = 512.
+//
+// Split-BF16: 128x128 tiles, four waves each owning a 64x64 quadrant as 4x4
+// MFMA blocks of 16x16, K streamed through LDS.
 // MFMA "rows" index C's columns and MFMA "columns" index C's rows, so each
 // lane's four accumulator values land in four columns at one row and the 16
 // lanes of a row-group write 128 contiguous bytes.
 //
-// Three arithmetic modes share the tiling:
+// Arithmetic modes:
 //   F64    : v_mfma_f64_16x16x4_f64 on double storage
 //   F32    : v_mfma_f32_16x16x4_f32 on float storage
 //   BF16X3 : split-bf16 (hi + lo) of the float panel, three products
@@ -29,6 +38,7 @@
 #include "kernels.hpp"
 #include "syrk_dev.hpp"
 #include "solve_dev.hpp"
+#include "tile64_dev.hpp"
 
 namespace elemamd {
 
@@ -45,9 +55,13 @@ __device__ inline int syrk_valid_k(const int* info, int k, int kcol0, int nbp) {
     return lim < 0 ? 0 : (lim < k ? lim : k);
 }
 
-__global__ __launch_bounds__(256, 2) void syrk_ln_f64_kernel(int m, int n, int k, double alpha,
-        const double* __restrict__ A, i64 lda, const double* __restrict__ B, i64 ldb, double beta,
-        double* __restrict__ C, i64 ldc, const int* __restrict__ info, int kcol0, int nbp, int chain) {
+// FP64 and FP32 (storage and MFMA of type T), 64 x 64 tiles.
+template <typename T, int KC>
+__global__ __launch_bounds__(256, 4) void syrk_ln_kernel(int m, int n, int k, T alpha, const T* __restrict__ A,
+                                                         i64 lda, const T* __restrict__ B, i64 ldb, T beta,
+                                                         T* __restrict__ C, i64 ldc, const int* __restrict__ info,
+                                                         int kcol0, int nbp, int chain) {
+    __shared__ tile64::Smem<T, KC> sm;
     // a launch the factorization's chain waits for issues ahead of the
     // concurrent bulk update's waves (wave priority, not queue priority)
     if (chain) __builtin_amdgcn_s_setprio(3);
@@ -55,17 +69,9 @@ __global__ __launch_bounds__(256, 2) void syrk_ln_f64_kernel(int m, int n, int k
     if (info != nullptr && ke == 0) return;
     int ti, tj;
     if (!syrk_tile(m, n, ti, tj)) return;
-    syrk_tile_f64(m, n, ke, alpha, A, lda, B, ldb, beta, C, ldc, ti, tj);
-}
-
-__global__ __launch_bounds__(256, 2) void syrk_ln_f32_kernel(int m, int n, int k, float alpha,
-        const float* __restrict__ A, i64 lda, const float* __restrict__ B, i64 ldb, float beta,
-        float* __restrict__ C, i64 ldc, const int* __restrict__ info, int kcol0, int nbp) {
-    const int ke = syrk_valid_k(info, k, kcol0, nbp);
-    if (info != nullptr && ke == 0) return;
-    int ti, tj;
-    if (!syrk_tile(m, n, ti, tj)) return;
-    syrk_tile_f32(m, n, ke, alpha, A, lda, B, ldb, beta, C, ldc, ti, tj);
+    const int i0 = ti * tile64::kTile, j0 = tj * tile64::kTile;
+    tile64::RowLoader<T, KC> li(A, lda, m, ke, i0), lj(B, ldb, n, ke, j0);
+    tile64::tile<T, KC>(sm, li, lj, i0, j0, m, n, ke, alpha, beta, C, ldc, 1);
 }
 
 __global__ __launch_bounds__(256, 2) void syrk_ln_bf16x3_kernel(int m, int n, int k, float alpha,
@@ -78,8 +84,8 @@ __global__ __launch_bounds__(256, 2) void syrk_ln_bf16x3_kernel(int m, int n, in
     syrk_tile_bf16x3(m, n, ke, alpha, A, lda, B, ldb, beta, C, ldc, ti, tj);
 }
 
-static dim3 syrk_grid(int m, int n) {
-    const i64 Tm = ceil_div(m, kSyrkTile), Tn = ceil_div(n, kSyrkTile);
+static dim3 syrk_grid(int m, int n, int tile) {
+    const i64 Tm = ceil_div(m, tile), Tn = ceil_div(n, tile);
     if (m == n) return dim3((unsigned)(Tm * (Tm + 1) / 2));
     return dim3((unsigned)Tm, (unsigned)Tn);
 }
@@ -88,24 +94,32 @@ hipError_t launch_syrk_ln_f64(int m, int n, int k, double alpha, const double* A
                               double beta, double* C, i64 ldc, const int* info, int kcol0, int nbp, hipStream_t s,
                               bool beside_chain) {
     if (m <= 0 || n <= 0) return hipSuccess;
-    // beside the chain: 56 KB of LDS per workgroup (36 KB used), so at most
-    // two share a CU and 48 KB stay free for the chain's kernels; every other
-    // launch of the factorization is on its chain
-    const unsigned pad = beside_chain ? 20u * 1024u : 0u;
-    hipLaunchKernelGGL(syrk_ln_f64_kernel, syrk_grid(m, n), dim3(256), pad, s, m, n, k, alpha, A, lda, B, ldb, beta, C,
-                       ldc, info, kcol0, nbp, (info != nullptr && !beside_chain) ? 1 : 0);
+    // beside the chain: 34 KB of LDS per workgroup (20 KB used), so four share
+    // a CU instead of six and registers (4 x 80 of 512) and LDS (24 KB and
+    // what one leaving workgroup frees) stay for the chain's kernels: without
+    // it the diagonal factor waits until the whole update has drained (900 us
+    // at m = 14000).  n = 16384 solve: 41.7 ms with no reserve, 40.2 with
+    // four a CU, 41.5 with three, 45.2 with two.
+    const unsigned pad = beside_chain ? 14u * 1024u : 0u;
+    // every other launch of the factorization is on its chain
+    const int chain = (info != nullptr && !beside_chain) ? 1 : 0;
+    hipLaunchKernelGGL((syrk_ln_kernel<double, 16>), syrk_grid(m, n, tile64::kTile), dim3(256), pad, s, m, n, k, alpha, A,
+                       lda, B, ldb, beta, C, ldc, info, kcol0, nbp, chain);
     return hipGetLastError();
 }
 
 hipError_t launch_syrk_ln_f32(bool bf16x3, int m, int n, int k, float alpha, const float* A, i64 lda, const float* B,
-                              i64 ldb, float beta, float* C, i64 ldc, const int* info, int kcol0, int nbp, hipStream_t s) {
+                              i64 ldb, float beta, float* C, i64 ldc, const int* info, int kcol0, int nbp, hipStream_t s,
+                              bool beside_chain) {
     if (m <= 0 || n <= 0) return hipSuccess;
+    // (the reserve beside the chain: as in launch_syrk_ln_f64)
     if (bf16x3)
-        hipLaunchKernelGGL(syrk_ln_bf16x3_kernel, syrk_grid(m, n), dim3(256), 0, s, m, n, k, alpha, A, lda, B, ldb, beta,
-                           C, ldc, info, kcol0, nbp);
+        hipLaunchKernelGGL(syrk_ln_bf16x3_kernel, syrk_grid(m, n, kSyrkTile), dim3(256), 0, s, m, n, k, alpha, A, lda, B,
+                           ldb, beta, C, ldc, info, kcol0, nbp);
     else
-        hipLaunchKernelGGL(syrk_ln_f32_kernel, syrk_grid(m, n), dim3(256), 0, s, m, n, k, alpha, A, lda, B, ldb, beta, C,
-                           ldc, info, kcol0, nbp);
+        hipLaunchKernelGGL((syrk_ln_kernel<float, 32>), syrk_grid(m, n, tile64::kTile), dim3(256),
+                           beside_chain ? 14u * 1024u : 0u, s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, info, kcol0,
+                           nbp, (info != nullptr && !beside_chain) ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -160,10 +174,10 @@ hipError_t launch_syrk_ln_bf16_planes(int np, int m, int n, int k, float alpha, 
                                       hipStream_t s, int chain) {
     if (m <= 0 || n <= 0) return hipSuccess;
     if (np == 2)
-        hipLaunchKernelGGL(syrk_ln_bf16p_kernel<2>, syrk_grid(m, n), dim3(256), 0, s, m, n, k, alpha, planes, ps, ldk,
+        hipLaunchKernelGGL(syrk_ln_bf16p_kernel<2>, syrk_grid(m, n, kSyrkTile), dim3(256), 0, s, m, n, k, alpha, planes, ps, ldk,
                            beta, C, ldc, info, kcol0, nbp, chain);
     else if (np == 3)
-        hipLaunchKernelGGL(syrk_ln_bf16p_kernel<3>, syrk_grid(m, n), dim3(256), 0, s, m, n, k, alpha, planes, ps, ldk,
+        hipLaunchKernelGGL(syrk_ln_bf16p_kernel<3>, syrk_grid(m, n, kSyrkTile), dim3(256), 0, s, m, n, k, alpha, planes, ps, ldk,
                            beta, C, ldc, info, kcol0, nbp, chain);
     else
         return hipErrorInvalidValue;
