@@ -37,10 +37,9 @@ int solve_left(bool upper, bool trans, bool unit, int n, int k, const double* L,
                void* work, hipStream_t s) {
     if (work == nullptr) work = stream_scratch(solve_work_bytes<double>(n, k), s);
     if (work == nullptr) return ELEMAMD_ERR_HIP;
-    int* ctrl = solve_ctrl<double>(n, work);
+    int* ctrl = (int*)work;
     const bool backward = upper != trans;
-    const int rc = solve_apply<double>(!backward, backward, n, k, L, ldl, B, ldb, nullptr, ctrl, nullptr, s, upper,
-                                       unit);
+    const int rc = solve_apply<double>(!backward, backward, n, k, L, ldl, B, ldb, ctrl, nullptr, s, upper, unit);
     return rc ? rc : solve_read_error(ctrl, s);
 }
 
@@ -223,7 +222,7 @@ int elemamd_solve_after_f64(char uplo, char orientation, int n, int k, const dou
     if (work == nullptr) return ELEMAMD_ERR_HIP;
     const int rc = solve_after_lower<double>(n, k, A, lda, B, ldb, nullptr, work, S(stream), uplo == 'U');
     if (rc || n == 0 || k == 0) return rc;
-    return solve_read_error(solve_ctrl<double>(n, work), S(stream));
+    return solve_read_error((const int*)work, S(stream));
 }
 
 int elemamd_hpd_solve_f64(char uplo, char orientation, int n, int k, double* A, int64_t lda, double* B, int64_t ldb,
@@ -240,10 +239,10 @@ int elemamd_hpd_solve_f64(char uplo, char orientation, int n, int k, double* A, 
     // transpose back
     if (upper && launch_transpose_inplace_f64(n, A, lda, s) != hipSuccess) return ELEMAMD_ERR_HIP;
     int rc = cholesky_lower<double>(n, A, lda, nb, kTrailingF64, dinfo, s);
-    if (rc == kOk) rc = solve_after_lower<double>(n, k, A, lda, B, ldb, dinfo, work, s, false, true);
+    if (rc == kOk) rc = solve_after_lower<double>(n, k, A, lda, B, ldb, dinfo, work, s);
     if (upper && launch_transpose_inplace_f64(n, A, lda, s) != hipSuccess) return ELEMAMD_ERR_HIP;
     if (rc || n == 0 || k == 0) return rc;
-    return solve_read_error(solve_ctrl<double>(n, work), s);
+    return solve_read_error((const int*)work, s);
 }
 
 // ------------------------------------------------- inverses and Gemm
@@ -349,7 +348,7 @@ int solve_after_f32_lower(int n, int k, const float* L, i64 ldl, float* B, i64 l
                           hipStream_t s) {
     const int rc = solve_after_lower<float>(n, k, L, ldl, B, ldb, dinfo, work, s);
     if (rc || n == 0 || k == 0) return rc;
-    return solve_read_error(solve_ctrl<float>(n, work), s);
+    return solve_read_error((const int*)work, s);
 }
 }  // namespace
 
@@ -393,7 +392,7 @@ int elemamd_hpd_solve_f32(char uplo, char orientation, int n, int k, float* A, i
     if (rc == kOk && n > 0 && k > 0) rc = solve_after_lower<float>(n, k, A, lda, B, ldb, dinfo, w, s);
     if (upper && launch_transpose_inplace<float>(n, A, lda, s) != hipSuccess) return ELEMAMD_ERR_HIP;
     if (rc || n == 0 || k == 0) return rc;
-    return solve_read_error(solve_ctrl<float>(n, w), s);
+    return solve_read_error((const int*)w, s);
 }
 
 static MixedOpts to_opts(const elemamd_ir_opts* o) {

@@ -115,35 +115,27 @@ hipError_t launch_trtri_fast_f64(int n, const double* L, i64 ldl, bool unit, dou
 // triangle of C := X^T X.
 hipError_t launch_trtrmm_unb_f64(int n, const double* X, i64 ldx, double* C, i64 ldc, const int* info, hipStream_t s);
 
-// solve.hip -- persistent triangular solves with precomputed inverses of the
-// 64x64 diagonal blocks.  Dinv holds solve_dinv_count(n) elements, ctrl
-// solve_ctrl_count(n, kc) ints (ctrl[1] != 0 after a solve means a bounded wait
-// expired).
+// solve_chain.hip -- triangular solves with a factor (forward: inv(L) B;
+// backward: inv(L^T) B; or both, in that order).  ctrl: chain_ctrl_count(n,
+// kc) ints (ctrl[1] != 0 after a solve means a bounded wait expired); part: n
+// kc elements; solve_ctrl_count is both together in ints.  upper: the factor
+// is stored in the upper triangle as U = L^T, so the forward solve is with
+// U^T and the backward one with U.  unit: unit diagonal (never read).
 size_t solve_ctrl_count(int n, int kc);
-// solve_chain.hip -- chain + helpers triangular solve (forward, or backward with L^T)
 size_t chain_ctrl_count(int n, int kc);
-// trans = false: the forward solve B := inv(L) B; trans = true: the backward
-// solve B := inv(L^T) B (blocks in reverse order).  upper: the factor is
-// stored in the upper triangle as U = L^T, so the forward solve is with U^T
-// and the backward one with U.  unit: unit diagonal (never read).
 template <typename T>
-hipError_t launch_trsm_chain(bool trans, int n, int kc, const T* L, i64 ldl, T* B, i64 ldb, const T* Dinv, int* ctrl,
+hipError_t launch_trsm_chain(bool forward, bool backward, int n, int kc, const T* L, i64 ldl, T* B, i64 ldb, int* ctrl,
                              T* part, const int* info, hipStream_t s, bool upper = false, bool unit = false);
+// solve.hip -- inverses of the 64 x 64 diagonal blocks I0 <= I < I1, into
+// Dinv (solve_dinv_count(n) elements)
 size_t solve_dinv_count(int n);
-template <typename T>
-hipError_t launch_trtri_diag64(int n, const T* L, i64 ldl, T* Dinv, hipStream_t s);
-// the 64-blocks I0 <= I < I1 only
-template <typename T>
-hipError_t launch_trtri_diag64_range(int n, int I0, int I1, const T* L, i64 ldl, T* Dinv, hipStream_t s);
-template <typename T>
-hipError_t launch_trsm_persist(bool trans, int n, int kc, const T* L, i64 ldl, T* B, i64 ldb, const T* Dinv,
-                               int* ctrl, const int* info, hipStream_t s);
+hipError_t launch_trtri_diag64_range(int n, int I0, int I1, const float* L, i64 ldl, float* Dinv, hipStream_t s);
 
 // solve_sweep.hip -- block-inverse sweeps for the float correction solves of
 // refinement.  Preparation (once per factor S, lower triangle = L): writes the
 // mirror of L into the strict upper triangle of S, the diagonal-block
 // inverses into Xp (sweep_xinv_count floats, scratch) and the sweep operands
-// into tiles (sweep_tiles_count floats).  Dinv: launch_trtri_diag64 output.
+// into tiles (sweep_tiles_count floats).  Dinv: launch_trtri_diag64_range output.
 size_t sweep_tiles_count(int n);
 size_t sweep_xinv_count(int n);
 size_t sweep_work_bytes(int n);

@@ -210,28 +210,22 @@ template int cholesky_lower<float>(int, float*, i64, int, int, int*, hipStream_t
 // pair in the reference; the persistent kernels handle k = 1 the same way.
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// `work` / `ctrl`: solve_ctrl_count(n, k) ints = tickets, error word and
+// flags, then the helpers' partial sums; ctrl[1] is the error word of the
+// whole solve (both directions).  The size also holds room for the inverses
+// of the 64 x 64 diagonal blocks, which the solves no longer use: a server's
+// memory budget and the workspace queries count it, and the requests that
+// they accept and refuse stay the same.
 template <typename T>
 size_t solve_work_bytes(int n, int k) {
     return align256(solve_dinv_count(n) * sizeof(T)) + align256(solve_ctrl_count(n, k) * sizeof(int));
 }
 
 template <typename T>
-int solve_prepare(int n, const T* L, i64 ldl, T* Dinv, hipStream_t s) {
-    ELEMAMD_HIP_TRY(launch_trtri_diag64<T>(n, L, ldl, Dinv, s));
-    return kOk;
-}
-
-template <typename T>
-int solve_apply(bool forward, bool backward, int n, int k, const T* L, i64 ldl, T* B, i64 ldb, const T* Dinv,
-                int* ctrl, const int* dinfo, hipStream_t s, bool upper, bool unit) {
-    // ctrl: solve_ctrl_count(n, k) ints = flags, then the helpers' partial sums;
-    // ctrl[1] is the error word of the whole solve (both directions)
+int solve_apply(bool forward, bool backward, int n, int k, const T* L, i64 ldl, T* B, i64 ldb, int* ctrl,
+                const int* dinfo, hipStream_t s, bool upper, bool unit) {
     T* part = (T*)((char*)ctrl + ((chain_ctrl_count(n, k) * sizeof(int) + 255) & ~(size_t)255));
-    if (n > 0 && k > 0) ELEMAMD_HIP_TRY(launch_fill_int(ctrl + 1, 0, 1, s));
-    if (forward)
-        ELEMAMD_HIP_TRY(launch_trsm_chain<T>(false, n, k, L, ldl, B, ldb, Dinv, ctrl, part, dinfo, s, upper, unit));
-    if (backward)
-        ELEMAMD_HIP_TRY(launch_trsm_chain<T>(true, n, k, L, ldl, B, ldb, Dinv, ctrl, part, dinfo, s, upper, unit));
+    ELEMAMD_HIP_TRY(launch_trsm_chain<T>(forward, backward, n, k, L, ldl, B, ldb, ctrl, part, dinfo, s, upper, unit));
     return kOk;
 }
 
@@ -243,40 +237,23 @@ int solve_read_error(const int* ctrl, hipStream_t s) {
 }
 
 template <typename T>
-int* solve_ctrl(int n, void* work) {
-    return (int*)((char*)work + align256(solve_dinv_count(n) * sizeof(T)));
-}
-
-template <typename T>
 int solve_after_lower(int n, int k, const T* L, i64 ldl, T* B, i64 ldb, const int* dinfo, void* work, hipStream_t s,
-                      bool upper, bool inverse_blocks) {
+                      bool upper) {
     if (n < 0 || k < 0 || ldl < std::max(1, n) || ldb < std::max(1, n)) return kErrArg;
     if (n == 0 || k == 0) return kOk;
     if (work == nullptr) return kErrWorkspace;
-    const bool inv = inverse_blocks && !upper;
-    T* Dinv = inv ? (T*)work : nullptr;
-    int* ctrl = solve_ctrl<T>(n, work);
-    if (inv) {
-        int rc = solve_prepare<T>(n, L, ldl, Dinv, s);
-        if (rc) return rc;
-    }
-    return solve_apply<T>(true, true, n, k, L, ldl, B, ldb, Dinv, ctrl, dinfo, s, upper, false);
+    return solve_apply<T>(true, true, n, k, L, ldl, B, ldb, (int*)work, dinfo, s, upper, false);
 }
 
 template size_t solve_work_bytes<double>(int, int);
 template size_t solve_work_bytes<float>(int, int);
-template int solve_prepare<double>(int, const double*, i64, double*, hipStream_t);
-template int solve_prepare<float>(int, const float*, i64, float*, hipStream_t);
-template int solve_apply<double>(bool, bool, int, int, const double*, i64, double*, i64, const double*, int*,
-                                 const int*, hipStream_t, bool, bool);
-template int solve_apply<float>(bool, bool, int, int, const float*, i64, float*, i64, const float*, int*, const int*,
-                                hipStream_t, bool, bool);
-template int* solve_ctrl<double>(int, void*);
-template int* solve_ctrl<float>(int, void*);
+template int solve_apply<double>(bool, bool, int, int, const double*, i64, double*, i64, int*, const int*, hipStream_t,
+                                 bool, bool);
+template int solve_apply<float>(bool, bool, int, int, const float*, i64, float*, i64, int*, const int*, hipStream_t,
+                                bool, bool);
 template int solve_after_lower<double>(int, int, const double*, i64, double*, i64, const int*, void*, hipStream_t,
-                                       bool, bool);
-template int solve_after_lower<float>(int, int, const float*, i64, float*, i64, const int*, void*, hipStream_t, bool,
-                                      bool);
+                                       bool);
+template int solve_after_lower<float>(int, int, const float*, i64, float*, i64, const int*, void*, hipStream_t, bool);
 
 // ------------------------------------------------------ mixed precision
 namespace {
@@ -774,7 +751,7 @@ int mixed_factor(int n, const double* A, i64 lda, const MixedOpts& o, MixedFacto
         if (c1 < n && 4 * (i64)c1 < 3 * (i64)n) return kOk;
         ELEMAMD_HIP_TRY(hipEventRecord(sp->ev_g, s));
         ELEMAMD_HIP_TRY(hipStreamWaitEvent(sp->aux3, sp->ev_g, 0));
-        ELEMAMD_HIP_TRY(launch_trtri_diag64_range<float>(n, prepared * (SB / 64), ready_blocks * (SB / 64), f.S, n,
+        ELEMAMD_HIP_TRY(launch_trtri_diag64_range(n, prepared * (SB / 64), ready_blocks * (SB / 64), f.S, n,
                                                          f.Dinv, sp->aux3));
         ELEMAMD_HIP_TRY(
             launch_sweep_prepare_blocks(n, prepared, ready_blocks, f.S, n, f.Dinv, f.Xp, f.tiles, sp->aux3));
@@ -859,9 +836,9 @@ static int fallback_fp64(int n, int k, const double* A, i64 lda, double* B, i64 
     r.info = info;
     if (info != 0) return kErrNotConverged;
     ELEMAMD_HIP_TRY(launch_copy_f64(n, k, fw.B0, n, B, ldb, s));
-    rc = solve_after_lower<double>(n, k, fw.Af, n, B, ldb, nullptr, fw.solve, s, false, true);
+    rc = solve_after_lower<double>(n, k, fw.Af, n, B, ldb, nullptr, fw.solve, s);
     if (rc) return rc;
-    rc = solve_read_error(solve_ctrl<double>(n, fw.solve), s);
+    rc = solve_read_error((const int*)fw.solve, s);
     if (rc) return rc;
     // eta = max_c ||b - A x||_inf / (||A||_inf ||x||_inf + ||b||_inf)
     ELEMAMD_HIP_TRY(launch_symm_lower_residual(n, k, A, lda, B, ldb, fw.B0, n, fw.R, n, fw.part, s));

@@ -66,27 +66,17 @@ template <typename T>
 size_t solve_work_bytes(int n, int k);
 // upper: the factor is stored in the upper triangle as U = L^T
 // (cholesky::SolveAfter(UPPER, ...): the forward solve with U^T, the backward
-// one with U).  inverse_blocks: the 64 x 64 diagonal blocks are applied as
-// products with their inverses (computed first) instead of by substitution
-// (always for float; for double the faster form that HPDSolve uses, while
-// the SolveAfter entry point keeps the substitution, exact on integer
-// problems); lower-stored factors only.
+// one with U).
 template <typename T>
 int solve_after_lower(int n, int k, const T* L, i64 ldl, T* B, i64 ldb, const int* dinfo, void* work, hipStream_t s,
-                      bool upper = false, bool inverse_blocks = sizeof(T) == 4);
-// The control words of solve_after_lower inside its `work` buffer.
-template <typename T>
-int* solve_ctrl(int n, void* work);
+                      bool upper = false);
 // Synchronize `s` and report a persistent solve whose bounded wait gave up
-// (kErrHip; the solution is then wrong) since solve_apply cleared ctrl[1].
+// (kErrHip; the solution is then wrong); ctrl: its `work`.
 int solve_read_error(const int* ctrl, hipStream_t s);
-// The two halves of it for repeated solves with one factor: the diagonal
-// block inverses are computed once (solve_prepare) and reused (solve_apply).
+// The forward solve, the backward one or both.
 template <typename T>
-int solve_prepare(int n, const T* L, i64 ldl, T* Dinv, hipStream_t s);
-template <typename T>
-int solve_apply(bool forward, bool backward, int n, int k, const T* L, i64 ldl, T* B, i64 ldb, const T* Dinv,
-                int* ctrl, const int* dinfo, hipStream_t s, bool upper = false, bool unit = false);
+int solve_apply(bool forward, bool backward, int n, int k, const T* L, i64 ldl, T* B, i64 ldb, int* ctrl,
+                const int* dinfo, hipStream_t s, bool upper = false, bool unit = false);
 
 struct MixedOpts {
     int nb = 128;

@@ -56,16 +56,14 @@ int elemamd_solve_after_f64_noalloc(char uplo, char orientation, int n, int k, c
     if ((uplo != 'L' && uplo != 'U') || (o != 'N' && o != 'T' && o != 'C')) return ELEMAMD_ERR_ARG;
     if (n < 0 || k < 0 || lda < (n > 1 ? n : 1) || ldb < (n > 1 ? n : 1)) return ELEMAMD_ERR_ARG;
     if (n == 0 || k == 0) return ELEMAMD_OK;
-    // the same ints the allocating entry point carves after its (unused for
-    // FP64) diagonal-inverse region: flags, then the partial sums
+    // the same ints as the allocating entry point's: flags, then the partial sums
     if (solve_ctrl_count(n, k) * sizeof(int) > kScratchBytes) return ELEMAMD_ERR_WORKSPACE;
     int* ctrl = (int*)scratch_ptr();
     if (ctrl == nullptr) return ELEMAMD_ERR_HIP;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // solve_apply clears the error word and every launch its tickets and
-    // flags (fill kernels, no memset); the partial sums are written before
-    // they are read
-    const int rc = solve_apply<double>(true, true, n, k, A, lda, B, ldb, nullptr, ctrl, nullptr, s, uplo == 'U', false);
+    // solve_apply clears the error word, the tickets and the flags (a fill
+    // kernel, no memset); the partial sums are written before they are read
+    const int rc = solve_apply<double>(true, true, n, k, A, lda, B, ldb, ctrl, nullptr, s, uplo == 'U', false);
     return rc ? rc : solve_read_error(ctrl, s);
 }
 
