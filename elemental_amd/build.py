@@ -30,6 +30,7 @@ SOURCES = [
     "blas1.hip",
     "lapack.cpp",
     "batch.hip",
+    "batch_solve.hip",
     "batch_plan.cpp",
     "runtime.cpp",
     "server.cpp",

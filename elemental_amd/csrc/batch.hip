@@ -4,8 +4,8 @@
 // Each matrix is the same computation as the single-matrix path: LVar3 with
 // block size nb (the same potrf / panel-solve / trailing-update device code,
 // so a matrix gives the same result alone and inside a batch), then the
-// forward and backward solves.  Matrices are processed in order of decreasing
-// size; step j of the factorization of every matrix that has a step j runs in
+// forward and backward solves (batch_solve.hip).  Matrices are processed in
+// order of decreasing size; step j of the factorization of every matrix that has a step j runs in
 // one launch per kernel type, and a workgroup finds its (matrix, tile) from a
 // per-step prefix sum of work counts, so small and large matrices share
 // launches without idle workgroups.  The whole sequence is captured in a
@@ -91,170 +91,21 @@ __global__ __launch_bounds__(256, 2) void batch_syrk_kernel(BatchArgs a, T* A, i
         syrk_tile_bf16x3(m, m, nb, -1.0f, (const float*)P, n, (const float*)P, n, 1.0f, (float*)C, n, ti, tj);
 }
 
-// ------------------------------------------------------------------ solve
-// One workgroup per matrix: forward then backward solve in 64-row blocks,
-// 16 right-hand sides at a time.  Contributions of solved blocks are staged
-// through LDS and applied with fused multiply-adds; the 64x64 diagonal block
-// is solved by substitution (one wave per four right-hand sides, lanes =
-// rows), the backward sweep as the forward sweep on reversed indices.
-constexpr int kBS = 64;
-constexpr int kBC = 16;
-
-template <typename T>
-__device__ inline T bcast_lane(T v, int lane);
-template <>
-__device__ inline double bcast_lane<double>(double v, int lane) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-    return __hiloint2double(hi, lo);
-}
-template <>
-__device__ inline float bcast_lane<float>(float v, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
-// LDS from the caller: sL (contraction tile / diagonal block), sX (solved
-// block / right-hand sides), sR (block being solved), sRinv.
-template <typename T>
-__device__ __forceinline__ void batch_solve_one(const BatchArgs& a, const T* L_all, T* B_all, int p,
-                                                T (*sL)[kBS + 1], T (*sX)[kBC + 1], T (*sR)[kBC + 1], T* sRinv) {
-    if (a.info[p] != 0) return;
-    if (a.skip != nullptr && a.skip[p]) return;
-    const int n = a.n[p], k = a.k[p];
-    const T* L = L_all + a.a_off[p];
-    T* B = B_all + a.b_off[p];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int nT = (n + kBS - 1) / kBS;
-    for (int cs = 0; cs < k; cs += kBC) {
-        const int kc = min(kBC, k - cs);
-        for (int dir = 0; dir < 2; ++dir) {
-            const bool back = dir == 1;
-            for (int ii = 0; ii < nT; ++ii) {
-                const int I = back ? (nT - 1 - ii) : ii;
-                const int r0 = I * kBS;
-                const int bs = min(kBS, n - r0);
-                // thread (row pl = t % 64, column group cg = t / 64: columns cg, cg+4, cg+8, cg+12)
-                const int pl = t & 63, cg = t >> 6;
-                T acc[4] = {T(0), T(0), T(0), T(0)};
-                for (int jj = 0; jj < ii; ++jj) {
-                    const int J = back ? (nT - 1 - jj) : jj;
-                    const int q0 = J * kBS;
-                    const int qs = min(kBS, n - q0);
-                    __syncthreads();
-                    // tile M[q][p]: forward L(r0+p, q0+q); backward L(q0+q, r0+p).
-                    // All loads of a thread first (clamped addresses), then LDS.
-                    {
-                        const int x = t & 63, y0 = t >> 6;
-                        T g[16], gx[4];
-#pragma unroll
-                        for (int s2 = 0; s2 < 16; ++s2) {
-                            const int y = y0 + 4 * s2;
-                            const bool ok = !back ? (x < bs && y < qs) : (x < qs && y < bs);
-                            const i64 off = !back ? (r0 + x) + (i64)(q0 + y) * n : (q0 + x) + (i64)(r0 + y) * n;
-                            const T v = L[ok ? off : 0];
-                            g[s2] = ok ? v : T(0);
-                        }
-#pragma unroll
-                        for (int s2 = 0; s2 < 4; ++s2) {
-                            const int c = y0 + 4 * s2;
-                            const bool ok = x < qs && c < kc;
-                            const T v = B[ok ? (q0 + x) + (i64)(cs + c) * n : 0];
-                            gx[s2] = ok ? v : T(0);
-                        }
-#pragma unroll
-                        for (int s2 = 0; s2 < 16; ++s2) {
-                            const int y = y0 + 4 * s2;
-                            if (!back) sL[y][x] = g[s2];
-                            else sL[x][y] = g[s2];
-                        }
-#pragma unroll
-                        for (int s2 = 0; s2 < 4; ++s2) sX[x][y0 + 4 * s2] = gx[s2];
-                    }
-                    __syncthreads();
-                    for (int q = 0; q < qs; ++q) {
-                        const T mv = sL[q][pl];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) acc[u] += mv * sX[q][cg + 4 * u];
-                    }
-                }
-                __syncthreads();
-                // R = B_I - acc
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int c = cg + 4 * u;
-                    sR[pl][c] = (pl < bs && c < kc) ? B[(r0 + pl) + (i64)(cs + c) * n] - acc[u] : T(0);
-                }
-                // diagonal block in lower-triangular form on (possibly reversed) indices
-                {
-                    const int x = t & 63, y0 = t >> 6;  // M(x, y) into sL[y][x]
-                    T g[16];
-#pragma unroll
-                    for (int s2 = 0; s2 < 16; ++s2) {
-                        const int y = y0 + 4 * s2;
-                        const int gi = back ? (kBS - 1 - y) : x;
-                        const int gk = back ? (kBS - 1 - x) : y;
-                        const bool ok = gi < bs && gk < bs && x >= y;
-                        const T v = L[ok ? (r0 + gi) + (i64)(r0 + gk) * n : 0];
-                        g[s2] = ok ? v : ((x == y) ? T(1) : T(0));
-                    }
-#pragma unroll
-                    for (int s2 = 0; s2 < 16; ++s2) sL[y0 + 4 * s2][x] = g[s2];
-                }
-                __syncthreads();
-                if (t < kBS) sRinv[t] = T(1) / sL[t][t];
-                __syncthreads();
-                const int myrow = back ? (kBS - 1 - lane) : lane;
-                T v[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = sR[myrow][4 * w + u];
-                for (int kk = 0; kk < kBS; ++kk) {
-                    const T rk = sRinv[kk];
-                    const T lik = sL[kk][lane];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const T y = bcast_lane<T>(v[u], kk) * rk;
-                        if (lane == kk) v[u] = y;
-                        else if (lane > kk) v[u] -= lik * y;
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int c = 4 * w + u;
-                    if (myrow < bs && c < kc) B[(r0 + myrow) + (i64)(cs + c) * n] = v[u];
-                }
-                __threadfence_block();
-                __syncthreads();
-            }
-        }
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void batch_solve_kernel(BatchArgs a, const T* L_all, T* B_all) {
-    __shared__ T sL[kBS][kBS + 1];
-    __shared__ T sX[kBS][kBC + 1];
-    __shared__ T sR[kBS][kBC + 1];
-    __shared__ T sRinv[kBS];
-    batch_solve_one<T>(a, L_all, B_all, blockIdx.x, sL, sX, sR, sRinv);
-}
-
 // ------------------------------------------------------ persistent launch
 // One launch per size bucket: every workgroup takes the bucket's matrices in
 // processing order (largest first) from a counter and factors each one whole
 // with the device code of the stepwise launches above -- LVar3Unb on the
 // diagonal block (256 threads, the same operation order), the register
 // panel solve, the trailing tiles in the same K order -- so a matrix's
-// factor is the same bit for bit in either form; for FP64 it then solves the
-// matrix's right-hand sides.  Workgroups never wait on each other.  The
-// phases share one LDS arena (the panel, trailing and solve phases never
-// overlap), so two workgroups fit on a CU.
+// factor is the same bit for bit in either form.  Workgroups never wait on
+// each other.  The phases share one LDS arena (they never overlap), so two
+// workgroups fit on a CU.
 constexpr int kArenaPanel = (2 * 32 * 32 + 128 + 4 * 16 * 34) * 8;
 constexpr int kArenaSyrk64 = 2 * 2 * kSyrkKC64 * kSyrkLdp * 8;
 constexpr int kArenaSyrk32 = 2 * 2 * kSyrkKC * kSyrkLdpF * 4;
 constexpr int kArenaBf16 = 4 * kSyrkTile * kBfLd * 2;
-constexpr int kArenaSolve = (kBS * (kBS + 1) + 2 * kBS * (kBC + 1) + kBS) * 8;
 constexpr int cmax(int x, int y) { return x > y ? x : y; }
-constexpr int kArenaBytes = cmax(cmax(kArenaPanel, kArenaSyrk64), cmax(cmax(kArenaSyrk32, kArenaBf16), kArenaSolve));
+constexpr int kArenaBytes = cmax(cmax(kArenaPanel, kArenaSyrk64), cmax(kArenaSyrk32, kArenaBf16));
 
 // The phases are separate (not inlined) functions: each gets the registers
 // it needs on its own (inlined together they spilled).
@@ -303,16 +154,8 @@ __device__ __noinline__ void persist_trailing(int m, int b, const T* P, T* C, in
     }
 }
 
-__device__ __noinline__ void persist_solve(const BatchArgs& a, const double* A, double* B, int p, char* arena) {
-    auto sL = reinterpret_cast<double(*)[kBS + 1]>(arena);
-    auto sX = reinterpret_cast<double(*)[kBC + 1]>(arena + kBS * (kBS + 1) * 8);
-    auto sR = reinterpret_cast<double(*)[kBC + 1]>(arena + (kBS * (kBS + 1) + kBS * (kBC + 1)) * 8);
-    double* sRinv = reinterpret_cast<double*>(arena + (kBS * (kBS + 1) + 2 * kBS * (kBC + 1)) * 8);
-    batch_solve_one<double>(a, A, B, p, sL, sX, sR, sRinv);
-}
-
-template <typename T, int MODE, bool SOLVE>
-__global__ __launch_bounds__(256, 2) void batch_persistent_kernel(BatchArgs a, T* A, double* B, int nb, int* counter) {
+template <typename T, int MODE>
+__global__ __launch_bounds__(256, 2) void batch_persistent_kernel(BatchArgs a, T* A, int nb, int* counter) {
     __shared__ __align__(16) char arena[kArenaBytes];
     __shared__ int s_p;
     for (;;) {
@@ -335,17 +178,13 @@ __global__ __launch_bounds__(256, 2) void batch_persistent_kernel(BatchArgs a, T
             persist_panel<T>(m, b, L, n, arena);
             persist_trailing<T, MODE>(m, b, L + b, M + (c0 + b) + (i64)(c0 + b) * n, n, arena);
         }
-        if constexpr (SOLVE) {
-            __syncthreads();
-            persist_solve(a, (const double*)A, B, p, arena);
-        }
     }
 }
 
 // -------------------------------------------------- refinement helpers
 // S_i := float(A_i) (lower triangle), one workgroup row per (matrix, column block)
-__global__ void batch_to_float_kernel(BatchArgs a, const double* A, float* S) {
-    const int p = blockIdx.y;
+__global__ void batch_to_float_kernel(BatchArgs a, const double* A, float* S, int first) {
+    const int p = first + blockIdx.y;
     const int n = a.n[p];
     const i64 total = (i64)n * n;
     const double* src = A + a.a_off[p];
@@ -581,36 +420,24 @@ hipError_t batch_syrk(const BatchArgs& a, void* A, int mode, int step, int nb, c
     return hipGetLastError();
 }
 
-hipError_t batch_persistent(const BatchArgs& a, void* F, double* B, int mode, int nb, int* counter, int grid,
-                            hipStream_t s) {
+hipError_t batch_persistent(const BatchArgs& a, void* F, int mode, int nb, int* counter, int grid, hipStream_t s) {
     if (a.count <= 0) return hipSuccess;
     if (nb < 1 || nb > kPersistMaxNb || grid < 1) return hipErrorInvalidValue;
     const dim3 g((unsigned)std::min(grid, a.count));
     if (mode == 0)
-        hipLaunchKernelGGL((batch_persistent_kernel<double, 0, true>), g, dim3(256), 0, s, a, (double*)F, B, nb,
-                           counter);
+        hipLaunchKernelGGL((batch_persistent_kernel<double, 0>), g, dim3(256), 0, s, a, (double*)F, nb, counter);
     else if (mode == 1)
-        hipLaunchKernelGGL((batch_persistent_kernel<float, 1, false>), g, dim3(256), 0, s, a, (float*)F, B, nb,
-                           counter);
+        hipLaunchKernelGGL((batch_persistent_kernel<float, 1>), g, dim3(256), 0, s, a, (float*)F, nb, counter);
     else
-        hipLaunchKernelGGL((batch_persistent_kernel<float, 2, false>), g, dim3(256), 0, s, a, (float*)F, B, nb,
-                           counter);
-    return hipGetLastError();
-}
-
-hipError_t batch_solve(const BatchArgs& a, const void* L, void* B, bool f32, hipStream_t s) {
-    if (a.count <= 0) return hipSuccess;
-    if (f32)
-        hipLaunchKernelGGL(batch_solve_kernel<float>, dim3(a.count), dim3(256), 0, s, a, (const float*)L, (float*)B);
-    else
-        hipLaunchKernelGGL(batch_solve_kernel<double>, dim3(a.count), dim3(256), 0, s, a, (const double*)L,
-                           (double*)B);
+        hipLaunchKernelGGL((batch_persistent_kernel<float, 2>), g, dim3(256), 0, s, a, (float*)F, nb, counter);
     return hipGetLastError();
 }
 
 hipError_t batch_to_float(const BatchArgs& a, const double* A, float* S, hipStream_t s) {
     if (a.count <= 0) return hipSuccess;
-    hipLaunchKernelGGL(batch_to_float_kernel, dim3(16, a.count), dim3(256), 0, s, a, A, S);
+    for (int first = 0; first < a.count; first += 32768)  // (a grid's y stays below 65536)
+        hipLaunchKernelGGL(batch_to_float_kernel, dim3(16, std::min(a.count - first, 32768)), dim3(256), 0, s, a, A, S,
+                           first);
     return hipGetLastError();
 }
 

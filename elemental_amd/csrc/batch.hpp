@@ -28,13 +28,13 @@ hipError_t batch_trsm(const BatchArgs& a, void* A, bool f32, int step, int nb, c
                       hipStream_t s);
 hipError_t batch_syrk(const BatchArgs& a, void* A, int mode, int step, int nb, const int* prefix, int cnt, int wgs,
                       hipStream_t s);
-hipError_t batch_solve(const BatchArgs& a, const void* L, void* B, bool f32, hipStream_t s);
+// batch_solve.hip -- forward and backward solves of every matrix (k <= kmax
+// columns each).  A bounded wait that gave up leaves info = -1.
+hipError_t batch_solve(const BatchArgs& a, const void* L, void* B, bool f32, int kmax, hipStream_t s);
 // The bucket's whole factorization (mode 0 FP64, 1 FP32, 2 BF16x3 trailing;
-// F = A, or the float copy) and, for FP64, its solves into B, as one launch
-// of `grid` workgroups that take the matrices from *counter (zeroed before).
-// nb <= kPersistMaxNb.
-hipError_t batch_persistent(const BatchArgs& a, void* F, double* B, int mode, int nb, int* counter, int grid,
-                            hipStream_t s);
+// F = A, or the float copy) as one launch of `grid` workgroups that take the
+// matrices from *counter (zeroed before).  nb <= kPersistMaxNb.
+hipError_t batch_persistent(const BatchArgs& a, void* F, int mode, int nb, int* counter, int grid, hipStream_t s);
 hipError_t batch_to_float(const BatchArgs& a, const double* A, float* S, hipStream_t s);
 // R := B - A X per matrix; eta (and rscale = ||r_c||_inf when non-null) per
 // matrix; prefix/wgs: 64-row blocks of the matrices; red: count*(1+3*kmax)
@@ -54,8 +54,14 @@ struct BatchBucket {
     int nb = 128;
     int grid = 0;   // 0: one launch per step and kernel; > 0: one persistent launch of grid workgroups
     int first = 0, count = 0;  // processing positions [first, first + count)
-    int steps = 0;
-    int res_prefix_off = 0, res_wgs = 0;  // 64-row blocks of the residual
+};
+
+// Consecutive buckets factored together: a persistent launch, or the steps of
+// all buckets with one block size (a matrix's result does not depend on what
+// shares its launches).
+struct BatchRun {
+    int nb = 128, grid = 0;
+    int first = 0, count = 0;
     struct Step {
         int active, trsm_wgs, syrk_wgs, trsm_prefix_off, syrk_prefix_off;
     };
@@ -72,12 +78,14 @@ struct BatchPlan {
     std::vector<i64> a_off, b_off;  // caller order, packed (ld = n_i)
     i64 a_total = 0, b_total = 0;
     std::vector<int> order;         // processing position -> caller index
-    std::vector<BatchBucket> buckets;
+    std::vector<BatchBucket> buckets;  // largest matrices first
+    std::vector<BatchRun> runs;
+    int res_prefix_off = 0, res_wgs = 0;  // 64-row blocks of the residual
     // device descriptors (processing order)
     int *d_n = nullptr, *d_k = nullptr, *d_prefix = nullptr;
     i64 *d_aoff = nullptr, *d_boff = nullptr;
     int *d_info = nullptr, *d_skip = nullptr, *d_iters = nullptr;
-    int* d_counters = nullptr;  // one per bucket: the persistent launches' matrix counters
+    int* d_counters = nullptr;  // one per run: the persistent launches' matrix counters
     double *d_eta = nullptr, *d_rscale = nullptr, *d_red = nullptr;
     std::vector<void*> dev_allocs;
     // captured graph and the arguments it was captured with

@@ -24,15 +24,70 @@ hipError_t upload(T** dst, const std::vector<T>& v) {
 
 inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// descriptors of one bucket (positions [first, first + count))
-BatchArgs bucket_args(const BatchPlan* P, const BatchBucket& b, bool with_skip) {
-    return BatchArgs{b.count,
-                     P->d_n + b.first,
-                     P->d_k + b.first,
-                     P->d_aoff + b.first,
-                     P->d_boff + b.first,
-                     P->d_info + b.first,
-                     with_skip ? P->d_skip + b.first : nullptr};
+// descriptors of the positions [first, first + count)
+BatchArgs plan_args(const BatchPlan* P, int first, int count, bool with_skip) {
+    return BatchArgs{count,
+                     P->d_n + first,
+                     P->d_k + first,
+                     P->d_aoff + first,
+                     P->d_boff + first,
+                     P->d_info + first,
+                     with_skip ? P->d_skip + first : nullptr};
+}
+BatchArgs plan_args(const BatchPlan* P, bool with_skip) { return plan_args(P, 0, P->count, with_skip); }
+
+// The runs and their steps' work prefix sums, from the buckets and their
+// launch forms.  Buckets with the same block size share their steps' launches
+// (each of which lasts as long as its largest matrix's chain): 1024 matrices
+// of n = 16 ... 1024 in six buckets take 10 block steps instead of 17.
+int plan_runs(BatchPlan* P) {
+    P->runs.clear();
+    for (const BatchBucket& bk : P->buckets) {
+        BatchRun* last = P->runs.empty() ? nullptr : &P->runs.back();
+        if (last != nullptr && bk.grid == 0 && last->grid == 0 && last->nb == bk.nb) {
+            last->count += bk.count;
+            continue;
+        }
+        BatchRun r;
+        r.nb = bk.nb;
+        r.grid = bk.grid;
+        r.first = bk.first;
+        r.count = bk.count;
+        P->runs.push_back(r);
+    }
+    std::vector<int> prefix;
+    auto size = [&](int p) { return P->n[P->order[p]]; };
+    for (BatchRun& r : P->runs) {
+        if (r.grid > 0) continue;
+        const int nb = r.nb, steps = (size(r.first) + nb - 1) / nb;
+        for (int j = 0; j < steps; ++j) {
+            BatchRun::Step st;
+            st.active = 0;
+            while (st.active < r.count && size(r.first + st.active) > j * nb) ++st.active;
+            std::vector<int> pt(st.active + 1, 0), ps(st.active + 1, 0);
+            for (int q = 0; q < st.active; ++q) {
+                const int m = size(r.first + q) - (j + 1) * nb;
+                const i64 T = m > 0 ? (m + 127) / 128 : 0;
+                pt[q + 1] = pt[q] + (m > 0 ? (m + 63) / 64 : 0);  // panel: 64 rows per workgroup
+                ps[q + 1] = ps[q] + (int)(T * (T + 1) / 2);       // trailing: lower 128x128 tiles
+            }
+            st.trsm_wgs = pt[st.active];
+            st.syrk_wgs = ps[st.active];
+            st.trsm_prefix_off = (int)prefix.size();
+            prefix.insert(prefix.end(), pt.begin(), pt.end());
+            st.syrk_prefix_off = (int)prefix.size();
+            prefix.insert(prefix.end(), ps.begin(), ps.end());
+            r.step.push_back(st);
+        }
+    }
+    std::vector<int> pr(P->count + 1, 0);
+    for (int q = 0; q < P->count; ++q) pr[q + 1] = pr[q] + (size(q) + 63) / 64;
+    P->res_wgs = pr[P->count];
+    P->res_prefix_off = (int)prefix.size();
+    prefix.insert(prefix.end(), pr.begin(), pr.end());
+    if (P->d_prefix != nullptr) (void)hipFree(P->d_prefix);
+    P->d_prefix = nullptr;
+    return upload(&P->d_prefix, prefix) == hipSuccess ? kOk : kErrHip;
 }
 
 }  // namespace
@@ -40,6 +95,7 @@ BatchArgs bucket_args(const BatchPlan* P, const BatchBucket& b, bool with_skip) 
 BatchPlan::~BatchPlan() {
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     if (capture_stream) (void)hipStreamDestroy(capture_stream);
+    if (d_prefix) (void)hipFree(d_prefix);
     for (void* p : dev_allocs) (void)hipFree(p);
 }
 
@@ -74,8 +130,9 @@ int batch_plan_create(int count, const int* n, const int* k, int precision, int 
     }
     P->a_total = ao;
     P->b_total = bo;
-    // bucket of each matrix; processing order = by bucket, then by decreasing
-    // size, so that the matrices still active at step j form a prefix
+    // bucket of each matrix; processing order = by decreasing size, so that
+    // the matrices still active at step j form a prefix and each bucket is a
+    // range
     std::vector<int> bk(count);
     for (int i = 0; i < count; ++i) {
         int b = 0;
@@ -85,7 +142,7 @@ int batch_plan_create(int count, const int* n, const int* k, int precision, int 
     P->order.resize(count);
     std::iota(P->order.begin(), P->order.end(), 0);
     std::stable_sort(P->order.begin(), P->order.end(),
-                     [&](int a, int b) { return bk[a] != bk[b] ? bk[a] < bk[b] : P->n[a] > P->n[b]; });
+                     [&](int a, int b) { return P->n[a] > P->n[b]; });
     std::vector<int> ns(count), ks(count);
     std::vector<i64> aos(count), bos(count);
     for (int p = 0; p < count; ++p) {
@@ -95,45 +152,17 @@ int batch_plan_create(int count, const int* n, const int* k, int precision, int 
         aos[p] = P->a_off[i];
         bos[p] = P->b_off[i];
     }
-    std::vector<int> prefix_all;
     int pos = 0;
-    for (int b = 0; b < nbuckets; ++b) {
+    for (int b = nbuckets - 1; b >= 0; --b) {
         BatchBucket B;
         B.index = b;
         B.nb = bucket_nb[b];
         B.first = pos;
         while (pos < count && bk[P->order[pos]] == b) ++pos;
         B.count = pos - B.first;
-        if (B.count == 0) continue;
-        const int nb = B.nb;
-        B.steps = (ns[B.first] + nb - 1) / nb;
-        for (int j = 0; j < B.steps; ++j) {
-            BatchBucket::Step st;
-            st.active = 0;
-            while (st.active < B.count && ns[B.first + st.active] > j * nb) ++st.active;
-            std::vector<int> pt(st.active + 1, 0), ps(st.active + 1, 0);
-            for (int q = 0; q < st.active; ++q) {
-                const int m = ns[B.first + q] - (j + 1) * nb;
-                const i64 T = m > 0 ? (m + 127) / 128 : 0;
-                pt[q + 1] = pt[q] + (m > 0 ? (m + 63) / 64 : 0);  // panel: 64 rows per workgroup
-                ps[q + 1] = ps[q] + (int)(T * (T + 1) / 2);       // trailing: lower 128x128 tiles
-            }
-            st.trsm_wgs = pt[st.active];
-            st.syrk_wgs = ps[st.active];
-            st.trsm_prefix_off = (int)prefix_all.size();
-            prefix_all.insert(prefix_all.end(), pt.begin(), pt.end());
-            st.syrk_prefix_off = (int)prefix_all.size();
-            prefix_all.insert(prefix_all.end(), ps.begin(), ps.end());
-            B.step.push_back(st);
-        }
-        std::vector<int> pr(B.count + 1, 0);
-        for (int q = 0; q < B.count; ++q) pr[q + 1] = pr[q] + (ns[B.first + q] + 63) / 64;
-        B.res_wgs = pr[B.count];
-        B.res_prefix_off = (int)prefix_all.size();
-        prefix_all.insert(prefix_all.end(), pr.begin(), pr.end());
-        P->buckets.push_back(B);
+        if (B.count > 0) P->buckets.push_back(B);
     }
-    int *d_n = nullptr, *d_k = nullptr, *d_pref = nullptr, *d_ints = nullptr;
+    int *d_n = nullptr, *d_k = nullptr, *d_ints = nullptr;
     i64 *d_ao = nullptr, *d_bo = nullptr;
     double* d_dbl = nullptr;
     bool ok = upload(&d_n, ns) == hipSuccess;
@@ -144,8 +173,7 @@ int batch_plan_create(int count, const int* n, const int* k, int precision, int 
     if (d_ao) P->dev_allocs.push_back(d_ao);
     ok = ok && upload(&d_bo, bos) == hipSuccess;
     if (d_bo) P->dev_allocs.push_back(d_bo);
-    ok = ok && upload(&d_pref, prefix_all) == hipSuccess;
-    if (d_pref) P->dev_allocs.push_back(d_pref);
+    ok = ok && plan_runs(P) == kOk;
     ok = ok && hipMalloc(&d_ints, sizeof(int) * (size_t)(3 * count + nbuckets)) == hipSuccess;
     if (d_ints) P->dev_allocs.push_back(d_ints);
     // eta, rscale (kmax per matrix), reduction scratch (1 + 3 kmax per matrix)
@@ -159,7 +187,6 @@ int batch_plan_create(int count, const int* n, const int* k, int precision, int 
     P->d_k = d_k;
     P->d_aoff = d_ao;
     P->d_boff = d_bo;
-    P->d_prefix = d_pref;
     P->d_info = d_ints;
     P->d_skip = d_ints + count;
     P->d_iters = d_ints + 2 * count;
@@ -175,12 +202,17 @@ int batch_set_launch(BatchPlan* P, const int* bucket_grid) {
     if (P == nullptr || bucket_grid == nullptr) return kErrArg;
     for (const BatchBucket& bk : P->buckets)
         if (bucket_grid[bk.index] < 0 || (bucket_grid[bk.index] > 0 && bk.nb > kPersistMaxNb)) return kErrArg;
-    for (BatchBucket& bk : P->buckets) bk.grid = bucket_grid[bk.index];
+    bool same = true;
+    for (BatchBucket& bk : P->buckets) {
+        same = same && bk.grid == bucket_grid[bk.index];
+        bk.grid = bucket_grid[bk.index];
+    }
+    if (same) return kOk;
     if (P->graph_exec) {  // captured with the previous launch forms
         (void)hipGraphExecDestroy(P->graph_exec);
         P->graph_exec = nullptr;
     }
-    return kOk;
+    return plan_runs(P);
 }
 
 size_t batch_workspace_bytes(const BatchPlan* P) {
@@ -194,7 +226,7 @@ size_t batch_workspace_bytes(const BatchPlan* P) {
 static int enqueue(BatchPlan* P, double* A, double* B, void* work, hipStream_t s) {
     if (P->count == 0) return kOk;
     // info, skip, iters, the persistent launches' counters
-    ELEMAMD_HIP_TRY(launch_fill_int(P->d_info, 0, 3 * P->count + (int)P->buckets.size(), s));
+    ELEMAMD_HIP_TRY(launch_fill_int(P->d_info, 0, 3 * P->count + (int)P->runs.size(), s));
     const bool f32 = P->precision != 0;
     const int mode = P->precision;  // trailing update: 0 FP64, 1 FP32, 2 BF16x3
     float* S = nullptr;
@@ -210,49 +242,42 @@ static int enqueue(BatchPlan* P, double* A, double* B, void* work, hipStream_t s
         w += al256(sizeof(double) * P->b_total);
         Rf = (float*)w;
     }
-    for (const BatchBucket& bk : P->buckets) {
-        const BatchArgs a = bucket_args(P, bk, false);
-        if (f32) ELEMAMD_HIP_TRY(batch_to_float(a, A, S, s));
-        void* F = f32 ? (void*)S : (void*)A;
-        if (bk.grid > 0) {  // the whole factorization (and FP64 solves) in one launch
-            ELEMAMD_HIP_TRY(batch_persistent(a, F, B, mode, bk.nb, P->d_counters + (&bk - P->buckets.data()),
-                                             bk.grid, s));
-            if (!f32) continue;
-        }
-        for (int j = 0; bk.grid == 0 && j < bk.steps; ++j) {
-            const BatchBucket::Step& st = bk.step[j];
-            ELEMAMD_HIP_TRY(batch_potrf(a, F, f32, j, bk.nb, st.active, s));
+    const BatchArgs a = plan_args(P, false);
+    if (f32) ELEMAMD_HIP_TRY(batch_to_float(a, A, S, s));
+    void* F = f32 ? (void*)S : (void*)A;
+    for (const BatchRun& r : P->runs) {
+        const BatchArgs ar = plan_args(P, r.first, r.count, false);
+        if (r.grid > 0)  // the whole factorization in one launch
+            ELEMAMD_HIP_TRY(batch_persistent(ar, F, mode, r.nb, P->d_counters + (&r - P->runs.data()), r.grid, s));
+        for (size_t j = 0; j < r.step.size(); ++j) {
+            const BatchRun::Step& st = r.step[j];
+            ELEMAMD_HIP_TRY(batch_potrf(ar, F, f32, (int)j, r.nb, st.active, s));
             ELEMAMD_HIP_TRY(
-                batch_trsm(a, F, f32, j, bk.nb, P->d_prefix + st.trsm_prefix_off, st.active, st.trsm_wgs, s));
+                batch_trsm(ar, F, f32, (int)j, r.nb, P->d_prefix + st.trsm_prefix_off, st.active, st.trsm_wgs, s));
             ELEMAMD_HIP_TRY(
-                batch_syrk(a, F, mode, j, bk.nb, P->d_prefix + st.syrk_prefix_off, st.active, st.syrk_wgs, s));
+                batch_syrk(ar, F, mode, (int)j, r.nb, P->d_prefix + st.syrk_prefix_off, st.active, st.syrk_wgs, s));
         }
-        if (!f32) {
-            ELEMAMD_HIP_TRY(batch_solve(a, A, B, false, s));
-            continue;
-        }
-        // (the refinement below follows either launch form)
-        // low-precision factor + FP64-residual refinement from X = 0: a fixed
-        // number of sweeps (the sequence is replayable); a converged matrix
-        // is skipped by every kernel of the remaining sweeps
-        const BatchArgs ai = bucket_args(P, bk, true);
-        double* eta = P->d_eta + bk.first;
-        double* rscale = P->d_rscale + (i64)bk.first * P->kmax;
-        int* iters = P->d_iters + bk.first;
-        double* red = P->d_red + (i64)bk.first * (1 + 3 * P->kmax);
-        ELEMAMD_HIP_TRY(batch_copy_rhs(a, nullptr, X, nullptr, s));  // X := 0
-        for (int it = 0; it < P->ir_sweeps; ++it) {
-            ELEMAMD_HIP_TRY(batch_residual(ai, A, X, B, R, P->d_prefix + bk.res_prefix_off, bk.res_wgs, red, eta,
-                                           rscale, P->kmax, s));
-            ELEMAMD_HIP_TRY(batch_ir_prepare(ai, eta, P->tol, R, rscale, Rf, P->kmax, iters, s));
-            ELEMAMD_HIP_TRY(batch_solve(ai, S, Rf, true, s));
-            ELEMAMD_HIP_TRY(batch_ir_update(ai, Rf, rscale, X, P->kmax, s));
-        }
-        // backward error of every matrix of the bucket, then X -> B
-        ELEMAMD_HIP_TRY(batch_residual(a, A, X, B, R, P->d_prefix + bk.res_prefix_off, bk.res_wgs, red, eta, nullptr,
-                                       P->kmax, s));
-        ELEMAMD_HIP_TRY(batch_copy_rhs(a, X, B, nullptr, s));
     }
+    if (!f32) {
+        ELEMAMD_HIP_TRY(batch_solve(a, A, B, false, P->kmax, s));
+        return kOk;
+    }
+    // low-precision factor + FP64-residual refinement from X = 0: a fixed
+    // number of sweeps (the sequence is replayable); a converged matrix is
+    // skipped by every kernel of the remaining sweeps
+    const BatchArgs ai = plan_args(P, true);
+    const int* res_prefix = P->d_prefix + P->res_prefix_off;
+    ELEMAMD_HIP_TRY(batch_copy_rhs(a, nullptr, X, nullptr, s));  // X := 0
+    for (int it = 0; it < P->ir_sweeps; ++it) {
+        ELEMAMD_HIP_TRY(batch_residual(ai, A, X, B, R, res_prefix, P->res_wgs, P->d_red, P->d_eta, P->d_rscale,
+                                       P->kmax, s));
+        ELEMAMD_HIP_TRY(batch_ir_prepare(ai, P->d_eta, P->tol, R, P->d_rscale, Rf, P->kmax, P->d_iters, s));
+        ELEMAMD_HIP_TRY(batch_solve(ai, S, Rf, true, P->kmax, s));
+        ELEMAMD_HIP_TRY(batch_ir_update(ai, Rf, P->d_rscale, X, P->kmax, s));
+    }
+    // backward error of every matrix, then X -> B
+    ELEMAMD_HIP_TRY(batch_residual(a, A, X, B, R, res_prefix, P->res_wgs, P->d_red, P->d_eta, nullptr, P->kmax, s));
+    ELEMAMD_HIP_TRY(batch_copy_rhs(a, X, B, nullptr, s));
     return kOk;
 }
 
@@ -315,12 +340,8 @@ int batch_backward_error(const BatchPlan* P, const double* A, const double* X, c
                          double* eta, hipStream_t s) {
     if (P == nullptr || eta == nullptr) return kErrArg;
     if (P->count == 0) return kOk;
-    for (const BatchBucket& bk : P->buckets) {
-        const BatchArgs a = bucket_args(P, bk, false);
-        ELEMAMD_HIP_TRY(batch_residual(a, A, X, B, R, P->d_prefix + bk.res_prefix_off, bk.res_wgs,
-                                       P->d_red + (i64)bk.first * (1 + 3 * P->kmax), P->d_eta + bk.first, nullptr,
-                                       P->kmax, s));
-    }
+    ELEMAMD_HIP_TRY(batch_residual(plan_args(P, false), A, X, B, R, P->d_prefix + P->res_prefix_off, P->res_wgs,
+                                   P->d_red, P->d_eta, nullptr, P->kmax, s));
     std::vector<double> he(P->count);
     ELEMAMD_HIP_TRY(hipMemcpyAsync(he.data(), P->d_eta, sizeof(double) * he.size(), hipMemcpyDeviceToHost, s));
     ELEMAMD_HIP_TRY(hipStreamSynchronize(s));
