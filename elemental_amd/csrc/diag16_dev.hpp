@@ -250,44 +250,51 @@ __device__ __forceinline__ int piece_careful(Lds<INV>& sh, int p, int nrows) {
 }
 
 // The b x b (b <= 128) block at A, lower triangle, by the calling workgroup
-// of kThreads threads; storage T, arithmetic FP64.  A failing pivot records
+// of 64 NW threads; storage T, arithmetic FP64.  NW = 4: wave w owns the tile
+// rows w and w + 4, with the same operations (and bits) as NW = 8.  A failing pivot records
 // col_offset + column (1-based) in *info.  INV: the inverses of the block's
 // 32 x 32 diagonal pieces also go to Xd (4 x 32 x 32, row-major).
-template <typename T, bool INV>
+template <typename T, bool INV, int NW = kWaves>
 __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict__ A, i64 lda, float* __restrict__ Xd,
                                              int* __restrict__ info, int col_offset) {
+    static_assert(NW == kWaves || (2 * NW == kWaves && !INV), "tile rows per wave");
+    constexpr int NR = kWaves / NW;  // tile rows of a wave: w0, w0 + NW
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int w0 = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int np = (b + 15) / 16;
     // tile row w, tiles 0 .. w (zero past b, the padded diagonal one; the
     // diagonal tile whole, mirrored).  Clamped addresses, no branch per load;
     // the masks only where the block is padded, so that a full block's later
     // tiles are still on their way while the first pieces are factored.
-    d4_t t[kWaves];
+    d4_t t[NR][kWaves];  // (row r has no tiles from NW (r + 1) on)
 #pragma unroll
-    for (int J = 0; J < kWaves; ++J)
+    for (int r = 0; r < NR; ++r)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int i = 16 * w + g + 4 * v, j = 16 * min(J, w) + c;
-            const int row = min(max(i, j), b - 1), col = min(min(i, j), b - 1);
-            t[J][v] = (double)A[row + (i64)col * lda];
-        }
-    if (b < 16 * kWaves)
-#pragma unroll
-        for (int J = 0; J < kWaves; ++J)
+        for (int J = 0; J < NW * (r + 1); ++J)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int i = 16 * w + g + 4 * v, j = 16 * J + c;
-                if (i >= b || j >= b) t[J][v] = i == j ? 1.0 : 0.0;
+                const int w = w0 + NW * r, i = 16 * w + g + 4 * v, j = 16 * min(J, w) + c;
+                const int row = min(max(i, j), b - 1), col = min(min(i, j), b - 1);
+                t[r][J][v] = (double)A[row + (i64)col * lda];
             }
-    if (tid == 0) sh.bad = 0;
-    if (w == 0) {
+    if (b < 16 * kWaves)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sh.D[g + 4 * v][c] = t[0][v];
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+            for (int J = 0; J < NW * (r + 1); ++J)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int i = 16 * (w0 + NW * r) + g + 4 * v, j = 16 * J + c;
+                    if (i >= b || j >= b) t[r][J][v] = i == j ? 1.0 : 0.0;
+                }
+    if (tid == 0) sh.bad = 0;
+    if (w0 == 0) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sh.D[g + 4 * v][c] = t[0][0][v];
         __builtin_amdgcn_wave_barrier();
     }
     // tile (w, q) of the factor, from its rows of sh.X
-    auto store_tile = [&](int q) __attribute__((always_inline)) {
+    auto store_tile = [&](int w, int q) __attribute__((always_inline)) {
         // (opaque lane: the addresses are made here, not kept in registers
         // across the loop)
         int lv = lane;
@@ -301,7 +308,8 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
     };
     int failed = 0;  // 1-based failing column of the block
     for (int p = 0; p < np; ++p) {
-        if (w == p) {
+        const bool mine = w0 == p % NW;  // piece p's diagonal tile is this wave's
+        if (mine) {
             __builtin_amdgcn_s_setprio(3);
             int lv = lane;  // (opaque, as in store_tile)
             asm volatile("" : "+v"(lv));
@@ -311,46 +319,53 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
             for (int q = 0; q < 16; ++q) d[q] = sh.D[c][q];
             const double piv = bcast<0>(d[0]);
             bool good = __builtin_amdgcn_class(piv, 0x180);
-            Column<0>::run(d, rsqrt_full(piv), c, good, sh.M, sh.V[w % Lds<INV>::kV]);
+            Column<0>::run(d, rsqrt_full(piv), c, good, sh.M, sh.V[p % Lds<INV>::kV]);
             if (!good && lane == 0) sh.bad = 1;
             __builtin_amdgcn_s_setprio(2);
         }
-        if (p > 0)  // t[0]: this piece's tile
+        if (p > 0)  // t[r][0]: this piece's tile
 #pragma unroll
-            for (int J = 0; J + 1 < kWaves; ++J) t[J] = t[J + 1];
+            for (int r = 0; r < NR; ++r)
+#pragma unroll
+                for (int J = 0; J + 1 < NW * (r + 1); ++J) t[r][J] = t[r][J + 1];
         __syncthreads();
         int kend = 16;  // columns of the piece that were factored
         const bool careful = sh.bad != 0;
         if (!careful) {
-            if (w > p && w < np) {
-                double m[16], a[4] = {t[0][0], t[0][1], t[0][2], t[0][3]};
 #pragma unroll
-                for (int k = 0; k < 16; ++k) m[k] = sh.M[c][k];  // (the last one is not used)
-                const double rv = rsqrt_full(sh.V[p % Lds<INV>::kV][c][c]);
-                // (the copies above end two wait states before the first DPP read)
-                asm volatile("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
-                TileColumn<0>::run(a, m);
+            for (int r = 0; r < NR; ++r) {
+                const int w = w0 + NW * r;
+                if (w > p && w < np) {
+                    double m[16], a[4] = {t[r][0][0], t[r][0][1], t[r][0][2], t[r][0][3]};
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    sh.X[c][16 * w + g + 4 * v] = a[v] * rv;
+                    for (int k = 0; k < 16; ++k) m[k] = sh.M[c][k];  // (the last one is not used)
+                    const double rv = rsqrt_full(sh.V[p % Lds<INV>::kV][c][c]);
+                    // (the copies above end two wait states before the first DPP read)
+                    asm volatile("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
+                    TileColumn<0>::run(a, m);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sh.X[c][16 * w + g + 4 * v] = a[v] * rv;
                 }
             }
             __syncthreads();
         } else {
-            if (w > p)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) sh.X[c][16 * w + g + 4 * v] = t[0][v];
-            if (w == p && p > 0) store_tile(p - 1);
+            for (int r = 0; r < NR; ++r)
+                if (w0 + NW * r > p)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sh.X[c][16 * (w0 + NW * r) + g + 4 * v] = t[r][0][v];
+            if (mine && p > 0) store_tile(p, p - 1);
             __syncthreads();
             if (tid == 0) sh.bad = 0;
             kend = piece_careful(sh, p, 16 * np);
             if (kend < 16) failed = 16 * p + kend + 1;
-            if (w == p) {
+            if (mine) {
 #pragma unroll 1
-                for (int q = 0; q < 16; ++q) sh.V[w % Lds<INV>::kV][q][c] = sh.X[q][16 * w + c];
+                for (int q = 0; q < 16; ++q) sh.V[p % Lds<INV>::kV][q][c] = sh.X[q][16 * p + c];
             }
             if (failed) {
-                if (w > p && w < np) store_tile(p);
+                for (int w = w0; w < np; w += NW)
+                    if (w > p) store_tile(w, p);
                 __syncthreads();
                 // columns from the failing one on update nothing
                 if (tid < 128)
@@ -359,30 +374,35 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
             }
             __syncthreads();
         }
-        if (w > p && w < np) {
-            double fa[4];
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) fa[ks] = -sh.X[4 * ks + g][16 * w + c];
+        for (int r = 0; r < NR; ++r) {
+            const int w = w0 + NW * r;
+            if (w > p && w < np) {
+                double fa[4];
 #pragma unroll
-            for (int j = 1; j < kWaves; ++j)
-                if (p + j <= w) {
-                    double fb[4];
+                for (int ks = 0; ks < 4; ++ks) fa[ks] = -sh.X[4 * ks + g][16 * w + c];
 #pragma unroll
-                    for (int ks = 0; ks < 4; ++ks) fb[ks] = sh.X[4 * ks + g][16 * (p + j) + c];
-                    mfma_tile(t[j], fa, fb);
-                }
-            // the solved tile (unsolved columns as they stand); wave p + 1 has
-            // the next piece to factor first and stores its tile afterwards
-            if (w != p + 1 && !failed) store_tile(p);
+                for (int j = 1; j < NW * (r + 1); ++j)
+                    if (p + j <= w) {
+                        double fb[4];
+#pragma unroll
+                        for (int ks = 0; ks < 4; ++ks) fb[ks] = sh.X[4 * ks + g][16 * (p + j) + c];
+                        mfma_tile(t[r][j], fa, fb);
+                    }
+                // the solved tile (unsolved columns as they stand); the wave of
+                // p + 1 has the next piece to factor first and stores its tile
+                // afterwards
+                if (w != p + 1 && !failed) store_tile(w, p);
+            }
         }
-        if (w == p) {
-            if (p > 0 && !careful) store_tile(p - 1);
+        if (mine) {
+            if (p > 0 && !careful) store_tile(p, p - 1);
             // the diagonal tile's columns, scaled by the reciprocal roots; l_kk
             // is the root itself, pivot * r with one correction
             int lv = lane;  // (opaque, as in store_tile)
             asm volatile("" : "+v"(lv));
             const int c = lv & 15, g = lv >> 4;
-            double pv = sh.V[w % Lds<INV>::kV][c][c], rv = 1.0;
+            double pv = sh.V[p % Lds<INV>::kV][c][c], rv = 1.0;
             if (kend == 16 && !careful) {
                 rv = rsqrt_full(pv);
                 const double s = pv * rv;
@@ -392,14 +412,14 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int r = g + 4 * v;
-                l[v] = r == c ? pv : sh.V[w % Lds<INV>::kV][c][r] * rv;
+                l[v] = r == c ? pv : sh.V[p % Lds<INV>::kV][c][r] * rv;
                 const int row = 16 * p + r, col = 16 * p + c;
                 if (row < b && c <= r) A[row + (i64)col * lda] = (T)l[v];
             }
             if constexpr (INV) {
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int v = 0; v < 4; ++v) sh.V[w % Lds<INV>::kV][c][g + 4 * v] = l[v];
+                for (int v = 0; v < 4; ++v) sh.V[p % Lds<INV>::kV][c][g + 4 * v] = l[v];
             }
         }
         if (failed) {
@@ -407,24 +427,31 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
             int lv = lane;  // (opaque, as in store_tile)
             asm volatile("" : "+v"(lv));
             const int c = lv & 15, g = lv >> 4;
-            if (w > p && w < np)
 #pragma unroll
-                for (int J = 1; J < kWaves; ++J)
+            for (int r = 0; r < NR; ++r) {
+                const int w = w0 + NW * r;
+                if (w > p && w < np)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int row = 16 * w + g + 4 * v, col = 16 * (p + J) + c;
-                        if (p + J <= w && row < b && col <= row) A[row + (i64)col * lda] = (T)t[J][v];
-                    }
+                    for (int J = 1; J < NW * (r + 1); ++J)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            const int row = 16 * w + g + 4 * v, col = 16 * (p + J) + c;
+                            if (p + J <= w && row < b && col <= row) A[row + (i64)col * lda] = (T)t[r][J][v];
+                        }
+            }
             if (tid == 0 && info != nullptr) *info = col_offset + failed;
             return;
         }
-        if (w == p + 1) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sh.D[g + 4 * v][c] = t[1][v];
-            __builtin_amdgcn_wave_barrier();
-        }
+        for (int r = 0; r < NR; ++r)
+            if (w0 + NW * r == p + 1) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) sh.D[g + 4 * v][c] = t[r][1][v];
+                __builtin_amdgcn_wave_barrier();
+            }
     }
     if constexpr (INV) {
+        const int w = w0;
         __syncthreads();
         // wave w: the inverse of its diagonal tile (the identity past b), then
         // X21 = -X22 (L21 X11) of each 32 x 32 piece by the odd waves
