@@ -16,11 +16,10 @@
 #include <algorithm>
 
 #include "batch.hpp"
-#include "chain64_dev.hpp"
 #include "common.hpp"
 #include "diag16_dev.hpp"
 #include "kernels.hpp"
-#include "panel_dev.hpp"
+#include "panel16_dev.hpp"
 #include "syrk_dev.hpp"
 
 namespace elemamd {
@@ -54,9 +53,7 @@ __global__ __launch_bounds__(diag16::kThreads, 4) void batch_potrf_kernel(BatchA
 template <typename T>
 __global__ __launch_bounds__(256) void batch_trsm_kernel(BatchArgs a, T* A, int step, int nb, const int* prefix,
                                                          int cnt) {
-    __shared__ double sDg[2][32][32];
-    __shared__ double sRinv[128];
-    __shared__ double sXq[4][16][34];
+    __shared__ panel16::Lds sh;
     const int p = find_item(prefix, cnt, blockIdx.x);
     const int rb = blockIdx.x - prefix[p];
     const int n = a.n[p];
@@ -67,7 +64,7 @@ __global__ __launch_bounds__(256) void batch_trsm_kernel(BatchArgs a, T* A, int 
     const int* info = a.info + p;
     if (*info != 0 && *info <= c0 + nb) return;
     T* L = A + a.a_off[p] + c0 + (i64)c0 * n;
-    chain64::panel64_slab<T>(m, nb, L, n, L + nb, n, rb, sDg, sRinv, sXq);
+    panel16::slab<T>(sh, m, nb, L, n, L + nb, n, rb);
 }
 
 template <typename T, int MODE>
@@ -103,7 +100,7 @@ __global__ __launch_bounds__(256, 2) void batch_syrk_kernel(BatchArgs a, T* A, i
 // factor is the same bit for bit in either form.  Workgroups never wait on
 // each other.  The phases share one LDS arena (they never overlap), so two
 // workgroups fit on a CU.
-constexpr int kArenaPanel = (2 * 32 * 32 + 128 + 4 * 16 * 34) * 8;
+constexpr int kArenaPanel = sizeof(panel16::Lds);
 constexpr int kArenaSyrk64 = 2 * 2 * kSyrkKC64 * kSyrkLdp * 8;
 constexpr int kArenaSyrk32 = 2 * 2 * kSyrkKC * kSyrkLdpF * 4;
 constexpr int kArenaBf16 = 4 * kSyrkTile * kBfLd * 2;
@@ -120,11 +117,8 @@ __device__ __noinline__ void persist_factor_block(int b, T* L, int n, int* info,
 
 template <typename T>
 __device__ __noinline__ void persist_panel(int m, int b, T* L, int n, char* arena) {
-    double(*sDg)[32][32] = reinterpret_cast<double(*)[32][32]>(arena);
-    double* sRinv = reinterpret_cast<double*>(arena + 2 * 32 * 32 * 8);
-    double(*sXq)[16][34] = reinterpret_cast<double(*)[16][34]>(arena + (2 * 32 * 32 + 128) * 8);
     for (int rb = 0; rb < (m + 63) / 64; ++rb) {
-        chain64::panel64_slab<T>(m, b, L, n, L + b, n, rb, sDg, sRinv, sXq);
+        panel16::slab<T>(*reinterpret_cast<panel16::Lds*>(arena), m, b, L, n, L + b, n, rb);
         __syncthreads();
     }
 }
