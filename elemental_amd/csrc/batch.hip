@@ -21,6 +21,7 @@
 #include "kernels.hpp"
 #include "panel16_dev.hpp"
 #include "syrk_dev.hpp"
+#include "tile64_dev.hpp"
 
 namespace elemamd {
 
@@ -67,9 +68,16 @@ __global__ __launch_bounds__(256) void batch_trsm_kernel(BatchArgs a, T* A, int 
     panel16::slab<T>(sh, m, nb, L, n, L + nb, n, rb);
 }
 
+// MODE 0, 1 (FP64, FP32): 64 x 64 tiles, as in the single matrix's update (in
+// the persistent launch, where one workgroup has all of a matrix's tiles, 128
+// x 128; each entry's operations are the same).  Most tiles of a batch belong
+// to updates of a few hundred rows, where 128 x 128 ones leave half of the
+// diagonal tiles' work and most CUs unused: 1024 matrices (n = 16 ... 1024),
+// seven steps of 128: FP64 1.15 ms with 128 x 128 tiles, 0.88 now, FP32 0.79
+// and 0.54.
 template <typename T, int MODE>
-__global__ __launch_bounds__(256, 2) void batch_syrk_kernel(BatchArgs a, T* A, int step, int nb, const int* prefix,
-                                                            int cnt) {
+__global__ __launch_bounds__(256, MODE == 2 ? 2 : 4) void batch_syrk_kernel(BatchArgs a, T* A, int step, int nb,
+                                                                            const int* prefix, int cnt) {
     const int p = find_item(prefix, cnt, blockIdx.x);
     const int t = blockIdx.x - prefix[p];
     const int n = a.n[p];
@@ -83,12 +91,15 @@ __global__ __launch_bounds__(256, 2) void batch_syrk_kernel(BatchArgs a, T* A, i
     tri_tile(t, ti, tj);
     const T* P = A + a.a_off[p] + (c0 + nb) + (i64)c0 * n;
     T* C = A + a.a_off[p] + (c0 + nb) + (i64)(c0 + nb) * n;
-    if constexpr (MODE == 0)
-        syrk_tile_f64(m, m, nb, -1.0, (const double*)P, n, (const double*)P, n, 1.0, (double*)C, n, ti, tj);
-    else if constexpr (MODE == 1)
-        syrk_tile_f32(m, m, nb, -1.0f, (const float*)P, n, (const float*)P, n, 1.0f, (float*)C, n, ti, tj);
-    else
+    if constexpr (MODE == 2) {
         syrk_tile_bf16x3(m, m, nb, -1.0f, (const float*)P, n, (const float*)P, n, 1.0f, (float*)C, n, ti, tj);
+    } else {
+        constexpr int KC = MODE == 0 ? 16 : 32;
+        __shared__ tile64::Smem<T, KC> sm;
+        const int i0 = ti * tile64::kTile, j0 = tj * tile64::kTile;
+        tile64::RowLoader<T, KC> li(P, n, m, nb, i0), lj(P, n, m, nb, j0);
+        tile64::tile<T, KC>(sm, li, lj, i0, j0, m, m, nb, T(-1), T(1), C, n, 1);
+    }
 }
 
 // ------------------------------------------------------ persistent launch

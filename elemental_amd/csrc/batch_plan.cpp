@@ -55,6 +55,7 @@ int plan_runs(BatchPlan* P) {
         r.count = bk.count;
         P->runs.push_back(r);
     }
+    const int tile = P->precision == 2 ? 128 : 64;  // of the trailing update
     std::vector<int> prefix;
     auto size = [&](int p) { return P->n[P->order[p]]; };
     for (BatchRun& r : P->runs) {
@@ -67,9 +68,9 @@ int plan_runs(BatchPlan* P) {
             std::vector<int> pt(st.active + 1, 0), ps(st.active + 1, 0);
             for (int q = 0; q < st.active; ++q) {
                 const int m = size(r.first + q) - (j + 1) * nb;
-                const i64 T = m > 0 ? (m + 127) / 128 : 0;
+                const i64 T = m > 0 ? (m + tile - 1) / tile : 0;
                 pt[q + 1] = pt[q] + (m > 0 ? (m + 63) / 64 : 0);  // panel: 64 rows per workgroup
-                ps[q + 1] = ps[q] + (int)(T * (T + 1) / 2);       // trailing: lower 128x128 tiles
+                ps[q + 1] = ps[q] + (int)(T * (T + 1) / 2);       // trailing: lower tiles
             }
             st.trsm_wgs = pt[st.active];
             st.syrk_wgs = ps[st.active];

@@ -33,7 +33,7 @@ __device__ inline bool syrk_tile(int m, int n, int& ti, int& tj) {
 }
 
 // ---------------------------------------------------------------- FP64
-// (batched launches; the single-matrix update is tile64_dev.hpp)
+// (the persistent batched launch; all others: tile64_dev.hpp)
 // K chunks of 8, double-buffered: 36 KB of LDS per workgroup.  With beta == 1 (the factorization) the accumulators start from
 // C, read at the start under the first chunk's loads, and the tile is only
 // stored at the end.
@@ -151,15 +151,6 @@ __device__ __forceinline__ void syrk_tile_f64_lds(int m, int n, int k, double al
     }
 }
 
-
-__device__ __forceinline__ void syrk_tile_f64(int m, int n, int k, double alpha,
-        const double* __restrict__ A, i64 lda, const double* __restrict__ B, i64 ldb, double beta,
-        double* __restrict__ C, i64 ldc, int ti, int tj) {
-    __shared__ double sI[2][kSyrkKC64][kSyrkLdp];
-    __shared__ double sJ[2][kSyrkKC64][kSyrkLdp];
-    syrk_tile_f64_lds(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ti, tj, sI, sJ);
-}
-
 // ---------------------------------------------------------------- FP32
 constexpr int kSyrkLdpF = kSyrkTile + 16;  // 144 floats: k-rows 16 banks apart
 
@@ -249,13 +240,6 @@ __device__ __forceinline__ void syrk_tile_f32_lds(int m, int n, int k, float alp
 // dropped), each a v_mfma_f32_16x16x32_bf16 with fp32 accumulation.
 // LDS holds row-major [row][k] planes so one lane fetches its 8 consecutive
 // k values (16 bytes) per operand.
-__device__ __forceinline__ void syrk_tile_f32(int m, int n, int k, float alpha,
-        const float* __restrict__ A, i64 lda, const float* __restrict__ B, i64 ldb, float beta,
-        float* __restrict__ C, i64 ldc, int ti, int tj) {
-    __shared__ float sI[2][kSyrkKC][kSyrkLdpF];
-    __shared__ float sJ[2][kSyrkKC][kSyrkLdpF];
-    syrk_tile_f32_lds(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ti, tj, sI, sJ);
-}
 
 constexpr int kBfKC = 32;
 constexpr int kBfLd = kBfKC + 8;  // 40 bf16 = 80 B per row: 8 lanes of 16 B hit disjoint banks
