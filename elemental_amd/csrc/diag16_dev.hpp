@@ -262,21 +262,59 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int w0 = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int np = (b + 15) / 16;
+    const bool full = b == 16 * kWaves;
     // tile row w, tiles 0 .. w (zero past b, the padded diagonal one; the
-    // diagonal tile whole, mirrored).  Clamped addresses, no branch per load;
-    // the masks only where the block is padded, so that a full block's later
-    // tiles are still on their way while the first pieces are factored.
+    // diagonal tile whole, mirrored).  16 rows by 4 columns per load, whole
+    // lines (with lanes along columns every lane is an access of its own, 64
+    // cycles a load, 7 us in all), then turned through the wave's part of sh.X.
     d4_t t[NR][kWaves];  // (row r has no tiles from NW (r + 1) on)
+    {
+        T raw[NR][kWaves][4];
 #pragma unroll
-    for (int r = 0; r < NR; ++r)
-#pragma unroll
-        for (int J = 0; J < NW * (r + 1); ++J)
+        for (int r = 0; r < NR; ++r) {
+            const int w = w0 + NW * r;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int w = w0 + NW * r, i = 16 * w + g + 4 * v, j = 16 * min(J, w) + c;
+                const int i = 16 * w + g + 4 * v, j = 16 * w + c;
                 const int row = min(max(i, j), b - 1), col = min(min(i, j), b - 1);
-                t[r][J][v] = (double)A[row + (i64)col * lda];
+                raw[r][kWaves - 1][v] = A[row + (i64)col * lda];
             }
+            if (full) {  // addresses by steps
+                const T* q = A + 16 * w + c + (i64)g * lda;
+#pragma unroll
+                for (int J = 0; J < NW * (r + 1) - 1; ++J)
+                    if (J < w)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v, q += 4 * lda) raw[r][J][v] = *q;
+            } else {
+#pragma unroll
+                for (int J = 0; J < NW * (r + 1) - 1; ++J)
+                    if (J < w)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            raw[r][J][v] = A[min(16 * w + c, b - 1) + (i64)min(16 * J + g + 4 * v, b - 1) * lda];
+            }
+        }
+        double(*sx)[16] = reinterpret_cast<double(*)[16]>(&sh.X[0][0] + 256 * w0);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int w = w0 + NW * r;
+#pragma unroll
+            for (int J = 0; J < NW * (r + 1); ++J) {
+                if (J < w && J < NW * (r + 1) - 1) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sx[c][(g + 4 * v) ^ c] = (double)raw[r][J][v];
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) t[r][J][v] = sx[g + 4 * v][c ^ (g + 4 * v)];
+                    __builtin_amdgcn_wave_barrier();
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) t[r][J][v] = (double)raw[r][kWaves - 1][v];
+                }
+            }
+        }
+    }
     if (b < 16 * kWaves)
 #pragma unroll
         for (int r = 0; r < NR; ++r)
@@ -299,11 +337,17 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
         // across the loop)
         int lv = lane;
         asm volatile("" : "+v"(lv));
-        const int cs = lv & 15, gs = lv >> 4, col = 16 * q + cs;
+        const int cs = lv & 15, gs = lv >> 4, row = 16 * w + cs;
+        if (full) {
+            T* to = A + row + (i64)(16 * q + gs) * lda;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int row = 16 * w + gs + 4 * v;
-            if (row < b && col < b) A[row + (i64)col * lda] = (T)sh.X[cs][row];
+            for (int v = 0; v < 4; ++v, to += 4 * lda) *to = (T)sh.X[gs + 4 * v][row];
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int col = 16 * q + gs + 4 * v;
+                if (row < b && col < b) A[row + (i64)col * lda] = (T)sh.X[gs + 4 * v][row];
+            }
         }
     };
     int failed = 0;  // 1-based failing column of the block
