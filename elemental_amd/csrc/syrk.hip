@@ -56,8 +56,8 @@ __device__ inline int syrk_valid_k(const int* info, int k, int kcol0, int nbp) {
 }
 
 // FP64 and FP32 (storage and MFMA of type T), 64 x 64 tiles.
-template <typename T, int KC>
-__global__ __launch_bounds__(256, 4) void syrk_ln_kernel(int m, int n, int k, T alpha, const T* __restrict__ A,
+template <typename T, int KC, int DEPTH, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void syrk_ln_kernel(int m, int n, int k, T alpha, const T* __restrict__ A,
                                                          i64 lda, const T* __restrict__ B, i64 ldb, T beta,
                                                          T* __restrict__ C, i64 ldc, const int* __restrict__ info,
                                                          int kcol0, int nbp, int chain) {
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256, 4) void syrk_ln_kernel(int m, int n, int k, T 
     int ti, tj;
     if (!syrk_tile(m, n, ti, tj)) return;
     const int i0 = ti * tile64::kTile, j0 = tj * tile64::kTile;
-    tile64::RowLoader<T, KC> li(A, lda, m, ke, i0), lj(B, ldb, n, ke, j0);
+    tile64::RowLoader<T, KC, DEPTH, NW> li(A, lda, m, ke, i0), lj(B, ldb, n, ke, j0);
     tile64::tile<T, KC>(sm, li, lj, i0, j0, m, n, ke, alpha, beta, C, ldc, 1);
 }
 
@@ -103,8 +103,9 @@ hipError_t launch_syrk_ln_f64(int m, int n, int k, double alpha, const double* A
     const unsigned pad = beside_chain ? 14u * 1024u : 0u;
     // every other launch of the factorization is on its chain
     const int chain = (info != nullptr && !beside_chain) ? 1 : 0;
-    hipLaunchKernelGGL((syrk_ln_kernel<double, 16>), syrk_grid(m, n, tile64::kTile), dim3(256), pad, s, m, n, k, alpha, A,
-                       lda, B, ldb, beta, C, ldc, info, kcol0, nbp, chain);
+    auto kernel = chain ? syrk_ln_kernel<double, 16, 2, 8> : syrk_ln_kernel<double, 16, 1, 4>;
+    hipLaunchKernelGGL(kernel, syrk_grid(m, n, tile64::kTile), dim3(chain ? 512 : 256), pad, s, m, n, k, alpha, A, lda, B, ldb, beta, C,
+                       ldc, info, kcol0, nbp, chain);
     return hipGetLastError();
 }
 
@@ -116,10 +117,12 @@ hipError_t launch_syrk_ln_f32(bool bf16x3, int m, int n, int k, float alpha, con
     if (bf16x3)
         hipLaunchKernelGGL(syrk_ln_bf16x3_kernel, syrk_grid(m, n, kSyrkTile), dim3(256), 0, s, m, n, k, alpha, A, lda, B,
                            ldb, beta, C, ldc, info, kcol0, nbp);
-    else
-        hipLaunchKernelGGL((syrk_ln_kernel<float, 32>), syrk_grid(m, n, tile64::kTile), dim3(256),
-                           beside_chain ? 14u * 1024u : 0u, s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, info, kcol0,
-                           nbp, (info != nullptr && !beside_chain) ? 1 : 0);
+    else {
+        const int chain = (info != nullptr && !beside_chain) ? 1 : 0;
+        auto kernel = chain ? syrk_ln_kernel<float, 32, 2, 8> : syrk_ln_kernel<float, 32, 1, 4>;
+        hipLaunchKernelGGL(kernel, syrk_grid(m, n, tile64::kTile), dim3(chain ? 512 : 256), beside_chain ? 14u * 1024u : 0u, s, m, n, k,
+                           alpha, A, lda, B, ldb, beta, C, ldc, info, kcol0, nbp, chain);
+    }
     return hipGetLastError();
 }
 

@@ -25,36 +25,43 @@ struct Smem {
     T I[KC][kLd], J[KC][kLd];
 };
 
+// What an operand without columns reads in their place.
+static __device__ double kNoColumn[1] = {};
+
 // One operand, rows x0 .. x0 + 63 of an ext x k matrix with element (x, l) at
-// M[x + l ld], KC columns per chunk.
-template <typename T, int KC>
+// M[x + l ld], KC columns per chunk, DEPTH chunks on their way.  Each load()
+// issues the same number of loads on every path (columns past k repeat the
+// last one), so the compiler waits for the chunk it needs and not for the
+// ones behind it.
+template <typename T, int KC, int DEPTH = 1, int NW = 4>
 struct RowLoader {
-    const T* p;  // this thread's row (clamped), first column
-    i64 ld;
-    int k, l0;
-    T g[KC / 4];
-    __device__ __forceinline__ RowLoader(const T* M, i64 ld_, int ext, int k_, int x0)
-        : ld(ld_), k(k_), l0(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
+    static constexpr int kDepth = DEPTH, kW = NW;
+    const T* p;  // this thread's row (clamped), the column to load next
+    i64 step;
+    int k, l0, next;
+    T g[DEPTH][KC / NW];
+    __device__ __forceinline__ RowLoader(const T* M, i64 ld, int ext, int k_, int x0)
+        : step(NW * ld), k(k_), l0(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), next(l0) {
         const int x = x0 + (int)(threadIdx.x & 63);
-        p = M + (x < ext ? x : ext - 1);
+        p = k > 0 ? M + (x < ext ? x : ext - 1) + (i64)min(l0, k - 1) * ld : (const T*)kNoColumn;
     }
-    __device__ __forceinline__ void load(int k0) {
-        if (k0 >= k) return;  // (k = 0: nothing may be read)
-        if (k0 + KC <= k) {
+    __device__ __forceinline__ void load(int d = 0) {  // the next chunk, into slot d
 #pragma unroll
-            for (int q = 0; q < KC / 4; ++q) g[q] = p[(i64)(k0 + l0 + 4 * q) * ld];
-        } else {
-#pragma unroll
-            for (int q = 0; q < KC / 4; ++q) {
-                const int l = k0 + l0 + 4 * q;
-                const T v = p[(i64)(l < k ? l : 0) * ld];
-                g[q] = l < k ? v : T(0);
-            }
+        for (int q = 0; q < KC / NW; ++q) {
+            g[d][q] = *p;
+            next += NW;
+            p += next < k ? step : 0;
         }
     }
-    __device__ __forceinline__ void store(T (*s)[kLd], T scale) const {
+    __device__ __forceinline__ void store(T (*s)[kLd], T scale, int k0, int d = 0) const {
+        if (k0 + KC <= k) {
 #pragma unroll
-        for (int q = 0; q < KC / 4; ++q) s[l0 + 4 * q][threadIdx.x & 63] = scale * g[q];
+            for (int q = 0; q < KC / NW; ++q) s[l0 + NW * q][threadIdx.x & 63] = scale * g[d][q];
+        } else {
+#pragma unroll
+            for (int q = 0; q < KC / NW; ++q)
+                s[l0 + NW * q][threadIdx.x & 63] = k0 + l0 + NW * q < k ? scale * g[d][q] : T(0);
+        }
     }
 };
 
@@ -69,68 +76,124 @@ __device__ __forceinline__ void tile(Smem<T, KC>& sm, LI& li, LJ& lj, int i0, in
                                      T beta, T* __restrict__ C, i64 ldc, int tri) {
     typedef typename Acc4<T>::type acc_t;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c16 = lane & 15, g = lane >> 4;
-    const int wj = (w >> 1) * 32, wi = (w & 1) * 32;
-    const bool skip = i0 == j0 && ((tri == 1 && wj > wi) || (tri == 2 && wi > wj));
+    constexpr int NW = LI::kW, NA = 8 / NW;  // waves, 16-column tiles of a wave
+    const int wj = (w >> 1) * 16 * NA, wi = (w & 1) * 32;
+    const bool skip = i0 == j0 && ((tri == 1 && wj >= wi + 32) || (tri == 2 && wi >= wj + 16 * NA));
     constexpr bool kFromC = sizeof(T) == 8;
     const bool acc_c = beta == T(1);
-    auto in = [&](int i, int j) { return i < m && j < n && (tri == 0 || (tri == 1 ? j <= i : i <= j)); };
-    li.load(0);
-    lj.load(0);
-    acc_t acc[2][2], pre[2][2];
+    // the thread's entries: rows i + 16 b, columns j + 16 a + jv v; a whole tile
+    // off the diagonal needs no masks
+    const int i = i0 + wi + c16, j = j0 + wj + mfma_row<T>(lane, 0), jv = mfma_row<T>(0, 1);
+    T* const Ct = C + i + (i64)j * ldc;
+    const bool whole = i0 + kTile <= m && j0 + kTile <= n && (tri == 0 || i0 != j0);
+    auto in = [&](int a, int b, int v) __attribute__((always_inline)) {
+        const int r = i + 16 * b, c = j + 16 * a + jv * v;
+        return r < m && c < n && (tri == 0 || (tri == 1 ? c <= r : r <= c));
+    };
+    constexpr int DEPTH = LI::kDepth;
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int d = 0; d < DEPTH; ++d) {
+        li.load(d);
+        lj.load(d);
+    }
+    acc_t acc[NA][2], pre[NA][2] = {};
+    if (acc_c && whole) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const T* c = Ct + (i64)(16 * a + jv * v) * ldc;
+#pragma unroll
+                for (int b = 0; b < 2; ++b) pre[a][b][v] = c[16 * b];
+            }
+    } else if (acc_c && !skip) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    if (in(a, b, v)) pre[a][b][v] = Ct[16 * b + (i64)(16 * a + jv * v) * ldc];
+    }
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = i0 + wi + 16 * b + c16, j = j0 + wj + 16 * a + mfma_row<T>(lane, v);
-                pre[a][b][v] = (acc_c && !skip && in(i, j)) ? C[i + (i64)j * ldc] : T(0);
-                acc[a][b][v] = kFromC ? pre[a][b][v] : T(0);
-            }
+            for (int v = 0; v < 4; ++v) acc[a][b][v] = kFromC ? pre[a][b][v] : T(0);
     const T scale = (kFromC && acc_c) ? alpha : T(1);
-    for (int k0 = 0; k0 < k; k0 += KC) {
-        li.store(sm.I, T(1));
-        lj.store(sm.J, scale);
-        __syncthreads();
-        if (k0 + KC < k) {
-            li.load(k0 + KC);
-            lj.load(k0 + KC);
-        }
-        if (!skip) {
+    for (int k1 = 0; k1 < k; k1 += DEPTH * KC) {
 #pragma unroll
-            for (int ks = 0; ks < KC / 4; ++ks) {
-                const int kr = 4 * ks + g;
-                T fa[2], fb[2];
+        for (int d = 0; d < DEPTH; ++d) {
+            const int k0 = k1 + d * KC;
+            if (k0 >= k) break;
+            li.store(sm.I, T(1), k0, d);
+            lj.store(sm.J, scale, k0, d);
+            __syncthreads();
+            li.load(d);
+            lj.load(d);
+            if (!skip) {
 #pragma unroll
-                for (int a = 0; a < 2; ++a) fa[a] = sm.J[kr][wj + 16 * a + c16];
+                for (int ks = 0; ks < KC / 4; ++ks) {
+                    const int kr = 4 * ks + g;
+                    T fa[NA], fb[2];
 #pragma unroll
-                for (int b = 0; b < 2; ++b) fb[b] = sm.I[kr][wi + 16 * b + c16];
+                    for (int a = 0; a < NA; ++a) fa[a] = sm.J[kr][wj + 16 * a + c16];
 #pragma unroll
-                for (int a = 0; a < 2; ++a)
+                    for (int b = 0; b < 2; ++b) fb[b] = sm.I[kr][wi + 16 * b + c16];
 #pragma unroll
-                    for (int b = 0; b < 2; ++b) acc[a][b] = mfma16(fa[a], fb[b], acc[a][b]);
+                    for (int a = 0; a < NA; ++a)
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) acc[a][b] = mfma16(fa[a], fb[b], acc[a][b]);
+                }
             }
+            __syncthreads();
         }
-        __syncthreads();
     }
     if (skip) return;
     // dependent zero-operand MFMAs before the accumulators are read (the
     // compiler's wait states after a loop back edge are short for FP64 MFMA)
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = mfma16(T(0), T(0), acc[a][b]);
+    if (acc_c) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+            for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = i0 + wi + 16 * b + c16, j = j0 + wj + 16 * a + mfma_row<T>(lane, v);
-                if (!in(i, j)) continue;
-                T* p = C + i + (i64)j * ldc;
-                if (acc_c) *p = kFromC ? acc[a][b][v] : pre[a][b][v] + alpha * acc[a][b][v];
-                else *p = beta == T(0) ? alpha * acc[a][b][v] : beta * *p + alpha * acc[a][b][v];
+                for (int v = 0; v < 4; ++v)
+                    if constexpr (!kFromC) acc[a][b][v] = pre[a][b][v] + alpha * acc[a][b][v];
+        if (whole) {
+#pragma unroll
+            for (int a = 0; a < NA; ++a)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    T* c = Ct + (i64)(16 * a + jv * v) * ldc;
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) c[16 * b] = acc[a][b][v];
+                }
+        } else {
+#pragma unroll
+            for (int a = 0; a < NA; ++a)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+                        if (in(a, b, v)) Ct[16 * b + (i64)(16 * a + jv * v) * ldc] = acc[a][b][v];
+        }
+        return;
+    }
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                if (!in(a, b, v)) continue;
+                T* c = Ct + 16 * b + (i64)(16 * a + jv * v) * ldc;
+                *c = beta == T(0) ? alpha * acc[a][b][v] : beta * *c + alpha * acc[a][b][v];
             }
 }
 
