@@ -35,6 +35,8 @@ namespace elemamd {
 //    auxiliary stream applies the group to the rest of the trailing matrix.
 //    The next group's update waits for the previous rest-update (they write
 //    the same elements); everything joins the caller's stream at the end.
+//    With few rows left the whole trailing pass goes to the caller's stream:
+//    it then takes less than the events that fork and join the streams.
 //  * Float storage (the low-precision factor): the panel solve multiplies by
 //    the inverses of the diagonal block's 32 x 32 pieces (potrf_f32.hip)
 //    instead of the substitution the FP64 path keeps.
@@ -173,7 +175,9 @@ int cholesky_lower(int n, T* A, i64 lda, int nb, int trailing, int* dinfo, hipSt
         if (rest_pending) ELEMAMD_HIP_TRY(hipStreamWaitEvent(s, sp->ev_b, 0));
         if (group == 0 && trailing_ready != nullptr) ELEMAMD_HIP_TRY(hipStreamWaitEvent(s, trailing_ready, 0));
         if (planes) Pl += (i64)(c1 - c0) * ldk;  // rows from c1 on
-        const bool rest = m2 > bn;
+        // few rows left: the whole trailing matrix on the caller's stream
+        const bool whole = !planes && m2 <= kForkRem;
+        const bool rest = !whole && m2 > bn;
         if (rest) {  // fork: the rest of the trailing matrix on aux
             ELEMAMD_HIP_TRY(hipEventRecord(sp->ev_a, s));
             ELEMAMD_HIP_TRY(hipStreamWaitEvent(sp->aux, sp->ev_a, 0));
@@ -193,7 +197,7 @@ int cholesky_lower(int n, T* A, i64 lda, int nb, int trailing, int* dinfo, hipSt
             ELEMAMD_HIP_TRY(launch_syrk_ln_bf16_planes(np, m2, bn, kg, -1.0f, Pl, (i64)plane_elems, ldk, 1.0f,
                                                        (float*)C, lda, dinfo, c0, nb, s, 1));
         else
-            ELEMAMD_HIP_TRY(syrk_launch<T>(trailing, m2, bn, kg, P, lda, C, lda, dinfo, c0, nb, s));
+            ELEMAMD_HIP_TRY(syrk_launch<T>(trailing, m2, whole ? m2 : bn, kg, P, lda, C, lda, dinfo, c0, nb, s));
     }
     if (rest_pending) ELEMAMD_HIP_TRY(hipStreamWaitEvent(s, sp->ev_b, 0));
     return kOk;
