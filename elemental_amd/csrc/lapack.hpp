@@ -22,6 +22,13 @@ enum : int { kRefineIR = 0, kRefineCG = 1 };
 // 40.2 ms, 512 throughout 39.2, the change at 4096, 6144 or 8192 columns 38.4,
 // at 10240 38.6; n = 2048: 256 1.78 ms, 512 1.85.
 constexpr int kUpdateDepthF64 = 256, kUpdateDepthF64Large = 512, kUpdateDepthF64Rem = 8192;
+// Rows left up to which a trailing pass is one launch on the caller's stream
+// (planes of BF16 apart).  An event pair costs the chain 10 to 20 us there and
+// the next group's columns alone another launch of 12 to 22; with 2048 rows
+// the rest is about 500 tiles, two a CU.  n = 2048: 1157 us with every pass
+// forked, 1119 / 1102 / 1084 / 1098 with 1024 / 1536 / 2048 / 2816; n = 3001:
+// 1803, 1762 / 1749 / 1719 / 1741; float n = 4000: 2242, 2222 / 2211 / 2186 / 2183.
+constexpr int kForkRem = 2048;
 constexpr int kUpdateDepthF32 = 512;
 constexpr int kUpdateDepthBf16x3 = 512;
 

@@ -1,5 +1,5 @@
-// Products and updates in 64 x 64 tiles of C, four waves of 32 x 32, K in
-// chunks of KC staged through LDS.
+// Products and updates in 64 x 64 tiles of C, four waves of 32 x 32 or eight
+// of 32 x 16, K in chunks of KC staged through LDS.
 //
 // What bounds them: with few tiles every chunk waits out a memory latency
 // (about 1 us), so small tiles spread the work over the CUs and a chunk's
@@ -8,7 +8,7 @@
 // share a CU (20 KB of LDS and about 100 registers each) and fill each
 // other's load, store and barrier phases.  Addresses cost no vector work
 // inside the loop: rows past the edge are clamped once (their products fall
-// on entries of C that are not stored), the k tail alone is masked.
+// on entries of C that are not stored), and loads step from column to column.
 #pragma once
 
 #include "common.hpp"
@@ -29,7 +29,8 @@ struct Smem {
 static __device__ double kNoColumn[1] = {};
 
 // One operand, rows x0 .. x0 + 63 of an ext x k matrix with element (x, l) at
-// M[x + l ld], KC columns per chunk, DEPTH chunks on their way.  Each load()
+// M[x + l ld], KC columns per chunk, DEPTH chunks on their way, loaded by NW
+// waves.  Each load()
 // issues the same number of loads on every path (columns past k repeat the
 // last one), so the compiler waits for the chunk it needs and not for the
 // ones behind it.
@@ -65,8 +66,8 @@ struct RowLoader {
     }
 };
 
-// Tile (i0, j0) of C := beta C + alpha I J^T by the calling 256-thread
-// workgroup (C m x n).  tri: 0 the whole tile, 1 entries j <= i, 2 entries
+// Tile (i0, j0) of C := beta C + alpha I J^T by the calling workgroup of the
+// loaders' NW waves (C m x n).  tri: 0 the whole tile, 1 entries j <= i, 2 entries
 // i <= j.  beta == 1 (the factorizations): C is read under the first chunk's
 // loads, and in FP64 the accumulators start from it (in FP32 they start from
 // zero and C is added at the end: fewer roundings at C's size); beta == 0: C
