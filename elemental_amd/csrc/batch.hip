@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void batch_trsm_kernel(BatchArgs a, T* A, int 
     const int* info = a.info + p;
     if (*info != 0 && *info <= c0 + nb) return;
     T* L = A + a.a_off[p] + c0 + (i64)c0 * n;
-    panel16::slab<T>(sh, m, nb, L, n, L + nb, n, rb);
+    panel16::slab<T>(sh, m, nb, L, n, L + nb, n, L + nb, n, rb);
 }
 
 // MODE 0, 1 (FP64, FP32): 64 x 64 tiles, as in the single matrix's update (in
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256, MODE == 2 ? 2 : 4) void batch_syrk_kernel(Batc
         __shared__ tile64::Smem<T, KC> sm;
         const int i0 = ti * tile64::kTile, j0 = tj * tile64::kTile;
         tile64::RowLoader<T, KC> li(P, n, m, nb, i0), lj(P, n, m, nb, j0);
-        tile64::tile<T, KC>(sm, li, lj, i0, j0, m, m, nb, T(-1), T(1), C, n, 1);
+        tile64::tile<sizeof(T) == 8>(sm, li, lj, i0, j0, m, m, nb, T(-1), T(1), C, n, 1);
     }
 }
 
@@ -129,7 +129,7 @@ __device__ __noinline__ void persist_factor_block(int b, T* L, int n, int* info,
 template <typename T>
 __device__ __noinline__ void persist_panel(int m, int b, T* L, int n, char* arena) {
     for (int rb = 0; rb < (m + 63) / 64; ++rb) {
-        panel16::slab<T>(*reinterpret_cast<panel16::Lds*>(arena), m, b, L, n, L + b, n, rb);
+        panel16::slab<T>(*reinterpret_cast<panel16::Lds*>(arena), m, b, L, n, L + b, n, L + b, n, rb);
         __syncthreads();
     }
 }

@@ -252,6 +252,24 @@ int elemamd_gemm_f64(char ta, char tb, int m, int n, int k, double alpha, const 
     const bool TA = is_trans(ta), TB = is_trans(tb);
     if (lda < std::max(1, TA ? k : m) || ldb < std::max(1, TB ? n : k) || ldc < std::max(1, m))
         return ELEMAMD_ERR_ARG;
+    // an operand that C overlaps (up to 128 x 128, read before it is written)
+    if (m > 0 && n > 0 && k > 0 && m <= 128 && n <= 128) {
+        const int ra = TA ? k : m, ca = TA ? m : k, rb = TB ? n : k, cb = TB ? k : n;
+        auto overlaps = [&](const double* X, int64_t ldx, int r, int c) {
+            return X < C + (n - 1) * ldc + m && C < X + (c - 1) * ldx + r;
+        };
+        const bool oa = overlaps(A, lda, ra, ca), ob = overlaps(B, ldb, rb, cb);
+        if (oa || ob) {
+            const size_t sa = al256(sizeof(double) * (size_t)ra * ca), sb = sizeof(double) * (size_t)rb * cb;
+            char* w = (char*)stream_scratch(sa + sb, S(stream));
+            if (w == nullptr) return ELEMAMD_ERR_HIP;
+            if (oa && launch_copy_f64(ra, ca, A, lda, (double*)w, ra, S(stream)) != hipSuccess) return ELEMAMD_ERR_HIP;
+            if (ob && launch_copy_f64(rb, cb, B, ldb, (double*)(w + sa), rb, S(stream)) != hipSuccess)
+                return ELEMAMD_ERR_HIP;
+            if (oa) A = (const double*)w, lda = ra;
+            if (ob) B = (const double*)(w + sa), ldb = rb;
+        }
+    }
     return launch_gemm_f64(TA, TB, m, n, k, alpha, A, lda, kGemmShapeFull, B, ldb, kGemmShapeFull, beta, C, ldc, 0,
                            nullptr, S(stream)) == hipSuccess
                ? ELEMAMD_OK

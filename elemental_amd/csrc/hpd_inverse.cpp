@@ -1,11 +1,11 @@
 // Host drivers of the direct callers of the Cholesky factor that invert:
 // the HPD inverse (hpd_inverse::CholeskyLVar2) and the triangular inverse
 // (triangular_inverse::LVar3).  Everything is enqueued on the caller's
-// stream.  The diagonal blocks' Cholesky factor is the bit-exact LVar3Unb
-// kernel (potrf.hip); their inverse and Trtrmm are the reference's unblocked
-// loops bit for bit when the whole matrix is one block, and the
-// recursive-doubling inverse and an MFMA product otherwise (inverse.hip,
-// gemm.hip); every other product runs on the FP64 MFMA GEMM.
+// stream.  When the whole matrix is one block, its factor, its inverse and
+// Trtrmm are the reference's unblocked loops bit for bit (potrf.hip,
+// inverse.hip); otherwise the diagonal blocks go through the blocked
+// factorization's kernels (16-column pieces, panel_f64.hip) and everything
+// else is FP64 MFMA products (gemm.hip).
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -15,8 +15,8 @@ namespace elemamd {
 
 static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// scratch: the diagonal block's inverse X11 (128 x 128, ld 128), then W
-// (nb x n) and P (n x nb)
+// scratch: the diagonal block's inverse (128 x 128, ld 128), then W (nb x n)
+// and P (n x nb)
 constexpr i64 kLdX = 128;
 size_t inverse_scratch_bytes(int n, int nb) {
     const size_t b = (size_t)std::max(1, std::min(nb, 128));
@@ -41,11 +41,16 @@ static hipError_t block_inverse(bool single, int b, const double* L11, i64 ld, b
 //     A00 += A10^T A10;  A20 -= A21 A10;  A22 -= A21 A21^T;
 //     A10 := inv(L11)^T A10;  A21 := -A21 inv(L11);
 //     A11 := inv(L11)^T inv(L11)        (TriangularInverse, then Trtrmm)
-// The four triangular solves with L11 become products with X11 = inv(L11)
-// (computed once per block), so the
-// whole step is one potrf, one small inverse and GEMMs:
-//     W = X11 A10,  P = A21 X11^T,  A00 += W^T W,  A20 -= P W,
-//     A22 -= P P^T,  A10 := X11^T W,  A21 := -P X11,  A11 := X11^T X11.
+// The triangular solves with L11 become one solve from the right, with the
+// rows of A21 and of the identity together, and products with what it gives:
+//     P = A21 inv(L11)^T,  R = inv(L11)^T;
+//     W = R^T A10,  A22 -= P P^T;
+//     A00 += W^T W,  A20 -= P W,  A10 := R W,  A21 := -P R^T,  A11 := R R^T.
+// Each line is one launch of products that do not depend on each other (four
+// launches a step with the diagonal factor): a step is bound by its launches'
+// latency, the products themselves being 1 to 2 GF.  n = 3000: 11.2 ms with a
+// separate inverse of the diagonal block (112 us) and seven products one after
+// the other (43 us each), 2.16 now.
 // A failed pivot stops everything after it (every launch checks *dinfo), so
 // A is left as the reference leaves it when Cholesky(A11) throws.
 int hpd_inverse_lower(int n, double* A, i64 lda, int nb, int* dinfo, void* scratch, hipStream_t s) {
@@ -56,8 +61,14 @@ int hpd_inverse_lower(int n, double* A, i64 lda, int nb, int* dinfo, void* scrat
     double* Xs = (double*)scratch;
     double* Ws = (double*)((char*)scratch + al256(kLdX * kLdX * sizeof(double)));
     double* Ps = (double*)((char*)Ws + al256((size_t)nb * n * sizeof(double)));
+    if (n <= nb) {
+        ELEMAMD_HIP_TRY(launch_potrf_unb<double>(n, A, lda, dinfo, 0, s));
+        ELEMAMD_HIP_TRY(launch_trtri_unb_f64(n, A, lda, false, Xs, kLdX, nullptr, lda, dinfo, s));
+        ELEMAMD_HIP_TRY(launch_trtrmm_unb_f64(n, Xs, kLdX, A, lda, dinfo, s));
+        return kOk;
+    }
     const i64 ldw = nb, ldp = n;
-    constexpr int F = kGemmShapeFull, Lo = kGemmShapeLower;
+    constexpr int F = kGemmShapeFull;
     for (int k0 = 0; k0 < n; k0 += nb) {
         const int b = std::min(nb, n - k0), j = k0, m = n - k0 - b;
         double* A11 = A + k0 + (i64)k0 * lda;
@@ -65,37 +76,18 @@ int hpd_inverse_lower(int n, double* A, i64 lda, int nb, int* dinfo, void* scrat
         double* A21 = A11 + b;
         double* A20 = A + k0 + b;
         double* A22 = A11 + b + (i64)b * lda;
-        ELEMAMD_HIP_TRY(n <= nb ? launch_potrf_unb<double>(b, A11, lda, dinfo, k0, s)
-                                : launch_potrf_block_f64(b, A11, lda, dinfo, k0, s));
-        ELEMAMD_HIP_TRY(block_inverse(n <= nb, b, A11, lda, false, Xs, nullptr, dinfo, s));
-        if (j > 0)  // W = X11 A10
-            ELEMAMD_HIP_TRY(launch_gemm_f64(false, false, b, j, b, 1.0, Xs, kLdX, Lo, A10, lda, F, 0.0, Ws, ldw, 0,
-                                            dinfo, s));
-        if (m > 0)  // P = A21 X11^T
-            ELEMAMD_HIP_TRY(launch_gemm_f64(false, true, m, b, b, 1.0, A21, lda, F, Xs, kLdX, Lo, 0.0, Ps, ldp, 0,
-                                            dinfo, s));
-        if (j > 0)  // A00 += W^T W (lower)
-            ELEMAMD_HIP_TRY(
-                launch_gemm_f64(true, false, j, j, b, 1.0, Ws, ldw, F, Ws, ldw, F, 1.0, A, lda, 1, dinfo, s));
-        if (j > 0 && m > 0)  // A20 -= P W
-            ELEMAMD_HIP_TRY(
-                launch_gemm_f64(false, false, m, j, b, -1.0, Ps, ldp, F, Ws, ldw, F, 1.0, A20, lda, 0, dinfo, s));
-        if (m > 0)  // A22 -= P P^T (lower)
-            ELEMAMD_HIP_TRY(
-                launch_gemm_f64(false, true, m, m, b, -1.0, Ps, ldp, F, Ps, ldp, F, 1.0, A22, lda, 1, dinfo, s));
-        if (j > 0)  // A10 := X11^T W
-            ELEMAMD_HIP_TRY(launch_gemm_f64(true, false, b, j, b, 1.0, Xs, kLdX, Lo, Ws, ldw, F, 0.0, A10, lda, 0,
-                                            dinfo, s));
-        if (m > 0)  // A21 := -P X11
-            ELEMAMD_HIP_TRY(launch_gemm_f64(false, false, m, b, b, -1.0, Ps, ldp, F, Xs, kLdX, Lo, 0.0, A21, lda, 0,
-                                            dinfo, s));
-        // A11 := X11^T X11 (lower): the reference's TrtrmmLUnblocked bit for
-        // bit for a single block, else the MFMA product
-        if (n <= nb)
-            ELEMAMD_HIP_TRY(launch_trtrmm_unb_f64(b, Xs, kLdX, A11, lda, dinfo, s));
-        else
-            ELEMAMD_HIP_TRY(
-                launch_gemm_f64(true, false, b, b, b, 1.0, Xs, kLdX, Lo, Xs, kLdX, Lo, 0.0, A11, lda, 1, dinfo, s));
+        ELEMAMD_HIP_TRY(launch_potrf_block_f64(b, A11, lda, dinfo, k0, s));
+        ELEMAMD_HIP_TRY(launch_panel_inverse_f64(m, b, A11, lda, A21, lda, Ps, ldp, Xs, kLdX, dinfo, s));
+        GemmJobs first, second;
+        first.add(true, false, b, j, b, 1.0, Xs, kLdX, F, A10, lda, F, 0.0, Ws, ldw, 0);   // W = R^T A10
+        first.add(false, true, m, m, b, -1.0, Ps, ldp, F, Ps, ldp, F, 1.0, A22, lda, 1);   // A22 -= P P^T (lower)
+        ELEMAMD_HIP_TRY(launch_gemm_jobs_f64(first, dinfo, s));
+        second.add(true, false, j, j, b, 1.0, Ws, ldw, F, Ws, ldw, F, 1.0, A, lda, 1);     // A00 += W^T W (lower)
+        second.add(false, false, m, j, b, -1.0, Ps, ldp, F, Ws, ldw, F, 1.0, A20, lda, 0);  // A20 -= P W
+        second.add(false, false, b, j, b, 1.0, Xs, kLdX, F, Ws, ldw, F, 0.0, A10, lda, 0);  // A10 := R W
+        second.add(false, true, m, b, b, -1.0, Ps, ldp, F, Xs, kLdX, F, 0.0, A21, lda, 0);  // A21 := -P R^T
+        second.add(false, true, b, b, b, 1.0, Xs, kLdX, F, Xs, kLdX, F, 0.0, A11, lda, 1);  // A11 := R R^T (lower)
+        ELEMAMD_HIP_TRY(launch_gemm_jobs_f64(second, dinfo, s));
     }
     return kOk;
 }

@@ -25,10 +25,13 @@ hipError_t launch_trsm_rlt(int m, int nb, const T* L, i64 ldl, T* B, i64 ldb, co
 
 
 // panel_f64.hip -- the FP64 factorization's panel solve B := B L^{-T}
-// (b <= 128): substitution inside 32-column pieces, FP64 MFMA products
+// (b <= 128): substitution inside 16-column tiles, FP64 MFMA products
 // between them, rows in registers (not bit-identical to launch_trsm_rlt).
 hipError_t launch_panel_f64(int m, int b, const double* L, i64 ldl, double* B, i64 ldb, const int* info, int limit,
                             hipStream_t s);
+// X := B L^{-T} (m x b, not in place) and R := L^{-T} (b x b) in one launch.
+hipError_t launch_panel_inverse_f64(int m, int b, const double* L, i64 ldl, const double* B, i64 ldb, double* X, i64 ldx,
+                                    double* R, i64 ldr, const int* info, hipStream_t s);
 
 // potrf_f32.hip -- panel step of the float-storage factor: the b x b
 // (b <= 128) diagonal block factored in place (FP64 on 32 x 32 pieces, whose
@@ -90,6 +93,21 @@ enum : int {
     kGemmShapeUpper = 3,
     kGemmShapeUpperUnit = 4,
 };
+struct GemmJob {
+    const double *A, *B;
+    double* C;
+    i64 lda, ldb, ldc;
+    double alpha, beta;
+    int m, n, k, tiles, ashape, bshape, ta, tb, tri;
+};
+// Products that do not depend on each other, for one launch.
+struct GemmJobs {
+    GemmJob job[5];
+    int count = 0;
+    void add(bool ta, bool tb, int m, int n, int k, double alpha, const double* A, i64 lda, int ashape, const double* B,
+             i64 ldb, int bshape, double beta, double* C, i64 ldc, int tri);
+};
+hipError_t launch_gemm_jobs_f64(const GemmJobs& jobs, const int* info, hipStream_t s);
 hipError_t launch_gemm_f64(bool ta, bool tb, int m, int n, int k, double alpha, const double* A, i64 lda, int ashape,
                            const double* B, i64 ldb, int bshape, double beta, double* C, i64 ldc, int tri,
                            const int* info, hipStream_t s);

@@ -40,12 +40,13 @@ struct TileColumn {
     }
 };
 
-// Rows [64 slab, 64 slab + 64) of B (m x b, b <= 128) := B L^{-T} by the
-// calling 256-thread workgroup, storage T (double, or float computed in
-// double).  Off: what holds the offset of three columns in bytes.
-template <typename T, typename Off = unsigned>
-__device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict__ L, i64 ldl, T* __restrict__ B,
-                                     i64 ldb, int slab) {
+// Rows [64 slab, 64 slab + 64) of X := B L^{-T} (m x b, b <= 128; X may be B)
+// by the calling 256-thread workgroup, storage T (double, or float computed in
+// double).  Off: what holds the offset of three columns in bytes.  IDENT: B
+// is the identity.
+template <typename T, typename Off = unsigned, bool IDENT = false>
+__device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict__ L, i64 ldl, const T* B, i64 ldb, T* X,
+                                     i64 ldx, int slab) {
     const int t = threadIdx.x, lane = t & 63, c = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int np = (b + 15) / 16;
@@ -86,7 +87,12 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
     const T* Bw = B + min(rw, m - 1);
     const Off rowc = (Off)min(c, max(m - 1 - rw, 0));
     T raw[kTiles][4];
-    if (full) {
+    if constexpr (IDENT) {
+#pragma unroll
+        for (int q = 0; q < kTiles; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) raw[q][v] = rw + c == 16 * q + g + 4 * v ? T(1) : T(0);
+    } else if (full) {
         const T* p = Bw;
         const Off off = (Off)g * (Off)ldb + rowc;
 #pragma unroll
@@ -177,19 +183,19 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
     }
     // (all stores at the end: a load behind a store waits for both)
     if (full && rw + 16 <= m) {
-        T* p = B + rw;
-        const Off off = (Off)g * (Off)ldb + (Off)c;
+        T* p = X + rw;
+        const Off off = (Off)g * (Off)ldx + (Off)c;
 #pragma unroll
         for (int q = 0; q < kTiles; ++q)
 #pragma unroll
-            for (int v = 0; v < 4; ++v, p += 4 * ldb) *(T*)((char*)p + off * (Off)sizeof(T)) = raw[q][v];
+            for (int v = 0; v < 4; ++v, p += 4 * ldx) *(T*)((char*)p + off * (Off)sizeof(T)) = raw[q][v];
     } else {
 #pragma unroll
         for (int q = 0; q < kTiles; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int r = rw + c, col = 16 * q + g + 4 * v;
-                if (r < m && col < b) B[r + (i64)col * ldb] = raw[q][v];
+                if (r < m && col < b) X[r + (i64)col * ldx] = raw[q][v];
             }
     }
 }

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void panel_f64_kernel(int m, int b, const doub
     // update's waves sharing the SIMD (wave priority, not queue priority)
     __builtin_amdgcn_s_setprio(3);
     if (info != nullptr && *info != 0 && *info <= limit) return;
-    panel16::slab<double, Off>(sh, m, b, L, ldl, B, ldb, blockIdx.x);
+    panel16::slab<double, Off>(sh, m, b, L, ldl, B, ldb, B, ldb, blockIdx.x);
 }
 
 hipError_t launch_panel_f64(int m, int b, const double* L, i64 ldl, double* B, i64 ldb, const int* info, int limit,
@@ -55,6 +55,33 @@ hipError_t launch_panel_f64(int m, int b, const double* L, i64 ldl, double* B, i
     // three columns' bytes in 32 bits
     auto kernel = std::max(ldl, ldb) < (i64)1 << 27 ? panel_f64_kernel<unsigned> : panel_f64_kernel<unsigned long long>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(m, 64)), dim3(256), 0, s, m, b, L, ldl, B, ldb, info, limit);
+    return hipGetLastError();
+}
+
+// X := B L^{-T} (m x b) and R := L^{-T} (b x b, zero below the diagonal) in one
+// launch: the panel of the HPD inverse and its diagonal block's inverse,
+// transposed.
+template <typename Off>
+__global__ __launch_bounds__(256) void panel_inverse_kernel(int m, int b, const double* __restrict__ L, i64 ldl,
+                                                            const double* B, i64 ldb, double* X, i64 ldx, double* R,
+                                                            i64 ldr, const int* __restrict__ info) {
+    __shared__ panel16::Lds sh;
+    if (info != nullptr && *info != 0) return;
+    const int ns = (b + 63) / 64;
+    if ((int)blockIdx.x < ns)
+        panel16::slab<double, Off, true>(sh, b, b, L, ldl, nullptr, 0, R, ldr, blockIdx.x);
+    else
+        panel16::slab<double, Off>(sh, m, b, L, ldl, B, ldb, X, ldx, blockIdx.x - ns);
+}
+
+hipError_t launch_panel_inverse_f64(int m, int b, const double* L, i64 ldl, const double* B, i64 ldb, double* X, i64 ldx,
+                                    double* R, i64 ldr, const int* info, hipStream_t s) {
+    if (b <= 0) return hipSuccess;
+    if (b > 128) return hipErrorInvalidValue;
+    const i64 ld = std::max(std::max(ldl, ldb), std::max(ldx, ldr));
+    auto kernel = ld < (i64)1 << 27 ? panel_inverse_kernel<unsigned> : panel_inverse_kernel<unsigned long long>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(ceil_div(b, 64) + (m > 0 ? ceil_div(m, 64) : 0))), dim3(256), 0, s, m, b, L,
+                       ldl, B, ldb, X, ldx, R, ldr, info);
     return hipGetLastError();
 }
 

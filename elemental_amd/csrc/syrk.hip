@@ -71,7 +71,7 @@ __global__ __launch_bounds__(64 * NW, 4) void syrk_ln_kernel(int m, int n, int k
     if (!syrk_tile(m, n, ti, tj)) return;
     const int i0 = ti * tile64::kTile, j0 = tj * tile64::kTile;
     tile64::RowLoader<T, KC, DEPTH, NW> li(A, lda, m, ke, i0), lj(B, ldb, n, ke, j0);
-    tile64::tile<T, KC>(sm, li, lj, i0, j0, m, n, ke, alpha, beta, C, ldc, 1);
+    tile64::tile<sizeof(T) == 8>(sm, li, lj, i0, j0, m, n, ke, alpha, beta, C, ldc, 1);
 }
 
 __global__ __launch_bounds__(256, 2) void syrk_ln_bf16x3_kernel(int m, int n, int k, float alpha,

@@ -20,9 +20,9 @@ namespace tile64 {
 constexpr int kTile = 64;
 constexpr int kLd = kTile + 16;  // LDS row stride of a chunk [k][row]: an MFMA operand's k rows start on other banks
 
-template <typename T, int KC>
+template <typename T, int KC, int LD = kLd>
 struct Smem {
-    T I[KC][kLd], J[KC][kLd];
+    T I[KC][LD], J[KC][LD];
 };
 
 // What an operand without columns reads in their place.
@@ -30,10 +30,8 @@ static __device__ double kNoColumn[1] = {};
 
 // One operand, rows x0 .. x0 + 63 of an ext x k matrix with element (x, l) at
 // M[x + l ld], KC columns per chunk, DEPTH chunks on their way, loaded by NW
-// waves.  Each load()
-// issues the same number of loads on every path (columns past k repeat the
-// last one), so the compiler waits for the chunk it needs and not for the
-// ones behind it.
+// waves.  load() has no branches (columns past k repeat an earlier one), so the
+// compiler waits for the chunk it needs and not for the ones behind it.
 template <typename T, int KC, int DEPTH = 1, int NW = 4>
 struct RowLoader {
     static constexpr int kDepth = DEPTH, kW = NW;
@@ -54,7 +52,8 @@ struct RowLoader {
             p += next < k ? step : 0;
         }
     }
-    __device__ __forceinline__ void store(T (*s)[kLd], T scale, int k0, int d = 0) const {
+    template <typename Row>
+    __device__ __forceinline__ void store(Row* s, T scale, int k0, int d = 0) const {
         if (k0 + KC <= k) {
 #pragma unroll
             for (int q = 0; q < KC / NW; ++q) s[l0 + NW * q][threadIdx.x & 63] = scale * g[d][q];
@@ -67,20 +66,20 @@ struct RowLoader {
 };
 
 // Tile (i0, j0) of C := beta C + alpha I J^T by the calling workgroup of the
-// loaders' NW waves (C m x n).  tri: 0 the whole tile, 1 entries j <= i, 2 entries
-// i <= j.  beta == 1 (the factorizations): C is read under the first chunk's
-// loads, and in FP64 the accumulators start from it (in FP32 they start from
-// zero and C is added at the end: fewer roundings at C's size); beta == 0: C
-// is not read.
-template <typename T, int KC, typename LI, typename LJ>
-__device__ __forceinline__ void tile(Smem<T, KC>& sm, LI& li, LJ& lj, int i0, int j0, int m, int n, int k, T alpha,
+// loaders' NW waves (C m x n).  tri: 0 the whole tile, 1 entries j <= i, 2
+// entries i <= j.  beta == 1: C is read under the first chunk's loads, and with
+// FROM_C (the FP64 factorizations) the accumulators start from it; otherwise
+// they start from zero and C is added at the end (fewer roundings at C's size:
+// the n = 3000 inverse's error against 64 bits is 4.4 times larger with it).
+// beta == 0: C is not read.
+template <bool FROM_C, typename T, int KC, int LD, typename LI, typename LJ>
+__device__ __forceinline__ void tile(Smem<T, KC, LD>& sm, LI& li, LJ& lj, int i0, int j0, int m, int n, int k, T alpha,
                                      T beta, T* __restrict__ C, i64 ldc, int tri) {
     typedef typename Acc4<T>::type acc_t;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c16 = lane & 15, g = lane >> 4;
     constexpr int NW = LI::kW, NA = 8 / NW;  // waves, 16-column tiles of a wave
     const int wj = (w >> 1) * 16 * NA, wi = (w & 1) * 32;
     const bool skip = i0 == j0 && ((tri == 1 && wj >= wi + 32) || (tri == 2 && wi >= wj + 16 * NA));
-    constexpr bool kFromC = sizeof(T) == 8;
     const bool acc_c = beta == T(1);
     // the thread's entries: rows i + 16 b, columns j + 16 a + jv v; a whole tile
     // off the diagonal needs no masks
@@ -121,8 +120,8 @@ __device__ __forceinline__ void tile(Smem<T, KC>& sm, LI& li, LJ& lj, int i0, in
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[a][b][v] = kFromC ? pre[a][b][v] : T(0);
-    const T scale = (kFromC && acc_c) ? alpha : T(1);
+            for (int v = 0; v < 4; ++v) acc[a][b][v] = FROM_C ? pre[a][b][v] : T(0);
+    const T scale = (FROM_C && acc_c) ? alpha : T(1);
     for (int k1 = 0; k1 < k; k1 += DEPTH * KC) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
@@ -165,7 +164,7 @@ __device__ __forceinline__ void tile(Smem<T, KC>& sm, LI& li, LJ& lj, int i0, in
             for (int b = 0; b < 2; ++b)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    if constexpr (!kFromC) acc[a][b][v] = pre[a][b][v] + alpha * acc[a][b][v];
+                    if constexpr (!FROM_C) acc[a][b][v] = pre[a][b][v] + alpha * acc[a][b][v];
         if (whole) {
 #pragma unroll
             for (int a = 0; a < NA; ++a)
