@@ -191,25 +191,11 @@ __global__ __launch_bounds__(256, 2) void batch_persistent_kernel(BatchArgs a, T
 }
 
 // -------------------------------------------------- refinement helpers
-// S_i := float(A_i) (lower triangle), one workgroup row per (matrix, column block)
-__global__ void batch_to_float_kernel(BatchArgs a, const double* A, float* S, int first) {
-    const int p = first + blockIdx.y;
-    const int n = a.n[p];
-    const i64 total = (i64)n * n;
-    const double* src = A + a.a_off[p];
-    float* dst = S + a.a_off[p];
-    for (i64 e = (i64)blockIdx.x * 256 + threadIdx.x; e < total; e += (i64)gridDim.x * 256) {
-        const int i = (int)(e % n), j = (int)(e / n);
-        if (i >= j) dst[e] = (float)src[e];
-    }
-}
-
 // R_i := B_i - A_i X_i (A_i symmetric, lower triangle read), FP64.  Work
 // items are 64-row blocks of every matrix (prefix sums over the bucket); a
 // workgroup streams the 64x64 tiles of its block row of the symmetric matrix
 // (tiles above the diagonal are read transposed from the stored lower
-// triangle) through LDS, with the right-hand sides in chunks of 8 columns.
-// Thread (row r, wave w) accumulates columns w and w + 4 of row r.  Per-matrix
+// triangle), with the right-hand sides in chunks of 8 columns.  Per-matrix
 // maxima -- ||A||_inf (row sums of |A|), ||r_c||_inf, ||x_c||_inf,
 // ||b_c||_inf -- are reduced per wave and merged with integer atomic max on
 // the bit patterns of the non-negative doubles, which is order independent.
@@ -227,11 +213,20 @@ __device__ inline void atomic_max_nonneg(double* p, double v) {
     atomicMax(reinterpret_cast<unsigned long long*>(p), (unsigned long long)__double_as_longlong(v));
 }
 
+// FIRST: X is zero and not read (R = B, the norms as above), and the tiles on
+// and below the diagonal also go to S as float.
+// What bounds it: reading A, each tile once in either orientation by the
+// workgroups of its two block rows.  A thread keeps its 16 entries of a tile in
+// registers and multiplies them by all columns (X by LDS broadcasts); only the
+// tiles above the diagonal are turned through LDS.  1024 matrices, n = 16 ...
+// 1024, up to 8 columns (1.03 GB read): 198 us (5.2 TB/s), with S 267; with all
+// tiles and X read from LDS for two columns a thread 304, and 201 more for S.
+template <bool FIRST>
 __global__ __launch_bounds__(256) void batch_symv_residual_kernel(BatchArgs a, const double* A, const double* X,
                                                                   const double* Bin, double* R, const int* prefix,
-                                                                  int cnt, double* red, int kmax) {
-    __shared__ double sM[64][65];  // sM[q][p] = Asym(r0 + p, q0 + q)
-    __shared__ double sX[64][9];
+                                                                  int cnt, double* red, int kmax, float* S) {
+    __shared__ double sM[64][65];  // a tile to be turned; at the end the waves' sums
+    __shared__ __align__(16) double sX[64][8];
     const int p = find_item(prefix, cnt, blockIdx.x);
     const int I = blockIdx.x - prefix[p];
     if (a.skip != nullptr && a.skip[p]) return;
@@ -248,64 +243,78 @@ __global__ __launch_bounds__(256) void batch_symv_residual_kernel(BatchArgs a, c
     const bool in = row < n;
     for (int c0 = 0; c0 < k; c0 += 8) {
         const int kc = min(8, k - c0);
-        double acc0 = 0.0, acc1 = 0.0, asum = 0.0;
+        double acc[8] = {}, asum = 0.0;
         for (int J = 0; J < nT; ++J) {
             const int q0 = J * 64;
-            __syncthreads();
-            {  // all 16 + 2 loads of a thread in flight (clamped addresses), then LDS
-                const int x = t & 63, y0 = t >> 6;
-                double g[16], gx[2];
+            // stored tile A(r0 + r, q0 + y) up to the diagonal (its lower part,
+            // mirrored below), else Asym(r0 + y, q0 + r) = A(q0 + r, r0 + y),
+            // y = w + 4 s; lanes along rows, clamped addresses
+            const int rb = J <= I ? r0 : q0, cb = J <= I ? q0 : r0;
+            double g[16];
+            if (rb + 64 <= n && J != I) {  // (cb < rb)
+                const double* e = Ap + (rb + r) + (i64)(cb + w) * n;
 #pragma unroll
-                for (int s2 = 0; s2 < 16; ++s2) {
-                    const int y = y0 + 4 * s2;
-                    bool ok;
-                    i64 off;
-                    if (J < I) {  // stored tile A(r0 + x, q0 + y): lanes along rows
-                        ok = r0 + x < n && q0 + y < n;
-                        off = (r0 + x) + (i64)(q0 + y) * n;
-                    } else if (J > I) {  // Asym(r0 + y, q0 + x) = A(q0 + x, r0 + y)
-                        ok = q0 + x < n && r0 + y < n;
-                        off = (q0 + x) + (i64)(r0 + y) * n;
-                    } else {  // diagonal tile, lower part (mirrored below)
-                        ok = r0 + x < n && x >= y;
-                        off = (r0 + x) + (i64)(r0 + y) * n;
-                    }
-                    const double v = Ap[ok ? off : 0];
-                    g[s2] = ok ? v : 0.0;
+                for (int s = 0; s < 16; ++s, e += 4 * (i64)n) g[s] = *e;
+            } else {
+#pragma unroll
+                for (int s = 0; s < 16; ++s) {
+                    const int y = w + 4 * s;
+                    const bool ok = rb + r < n && cb + y < n && (J != I || r >= y);
+                    const double v = Ap[ok ? (rb + r) + (i64)(cb + y) * n : 0];
+                    g[s] = ok ? v : 0.0;
                 }
-#pragma unroll
-                for (int s2 = 0; s2 < 2; ++s2) {
-                    const int c = y0 + 4 * s2;
-                    const bool ok = q0 + x < n && c < kc;
-                    const double v = Xp[ok ? (q0 + x) + (i64)(c0 + c) * n : 0];
-                    gx[s2] = ok ? v : 0.0;
-                }
-#pragma unroll
-                for (int s2 = 0; s2 < 16; ++s2) {
-                    const int y = y0 + 4 * s2;
-                    if (J < I) {
-                        sM[y][x] = g[s2];
-                    } else if (J > I) {
-                        sM[x][y] = g[s2];
-                    } else if (x >= y) {
-                        sM[y][x] = g[s2];
-                        sM[x][y] = g[s2];
-                    }
-                }
-#pragma unroll
-                for (int s2 = 0; s2 < 2; ++s2) sX[x][y0 + 4 * s2] = gx[s2];
             }
+            double x[2];
+            if constexpr (!FIRST)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int c = w + 4 * u;
+                    const bool ok = q0 + r < n && c < kc;
+                    const double v = Xp[ok ? (q0 + r) + (i64)(c0 + c) * n : 0];
+                    x[u] = ok ? v : 0.0;
+                }
+            if constexpr (FIRST)
+                if (c0 == 0 && J <= I && in) {
+                    float* Sp = S + a.a_off[p] + row + (i64)(q0 + w) * n;
+#pragma unroll
+                    for (int s = 0; s < 16; ++s, Sp += 4 * (i64)n)
+                        if (J < I || r >= w + 4 * s) *Sp = (float)g[s];
+                }
+            __syncthreads();  // the tile before is done with sM and sX
+            if (J > I) {
+#pragma unroll
+                for (int s = 0; s < 16; ++s) sM[r][w + 4 * s] = g[s];  // sM[q][row]
+            } else if (J == I) {
+#pragma unroll
+                for (int s = 0; s < 16; ++s) {
+                    const int y = w + 4 * s;
+                    if (r >= y) sM[y][r] = sM[r][y] = g[s];
+                }
+            }
+            if constexpr (!FIRST)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) sX[r][w + 4 * u] = x[u];
             __syncthreads();
-#pragma unroll 8
-            for (int q = 0; q < 64; ++q) {
-                const double m = sM[q][r];
-                acc0 += m * sX[q][w];
-                acc1 += m * sX[q][w + 4];
-                asum += fabs(m);
+            if (J >= I)
+#pragma unroll
+                for (int s = 0; s < 16; ++s) g[s] = sM[w + 4 * s][r];
+#pragma unroll
+            for (int s = 0; s < 16; ++s) {  // g[s] = Asym(r0 + r, q0 + w + 4 s)
+                asum += fabs(g[s]);
+                if constexpr (!FIRST)
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) acc[c] = fma(g[s], sX[w + 4 * s][c], acc[c]);
             }
         }
+        // the four waves' sums of row r, [wave][8] and [32 + wave]
+        __syncthreads();
+        if constexpr (!FIRST)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) sM[r][8 * w + c] = acc[c];
+        sM[r][32 + w] = asum;
+        __syncthreads();
         if (c0 == 0 && w == 0) {
-            const double am = wave_max(in ? asum : 0.0);
+            const double am = wave_max(in ? (sM[r][32] + sM[r][33]) + (sM[r][34] + sM[r][35]) : 0.0);
             if (r == 0) atomic_max_nonneg(&rd[0], am);
         }
 #pragma unroll
@@ -315,8 +324,11 @@ __global__ __launch_bounds__(256) void batch_symv_residual_kernel(BatchArgs a, c
             if (in && c < kc) {
                 const i64 e = row + (i64)(c0 + c) * n;
                 bv = Bp[e];
-                xv = Xp[e];
-                rv = bv - (u == 0 ? acc0 : acc1);
+                rv = bv;
+                if constexpr (!FIRST) {
+                    xv = Xp[e];
+                    rv -= (sM[r][c] + sM[r][8 + c]) + (sM[r][16 + c] + sM[r][24 + c]);
+                }
                 Rp[e] = rv;
             }
             const double rm = wave_max(fabs(rv)), xm = wave_max(fabs(xv)), bm = wave_max(fabs(bv));
@@ -442,23 +454,15 @@ hipError_t batch_persistent(const BatchArgs& a, void* F, int mode, int nb, int* 
     return hipGetLastError();
 }
 
-hipError_t batch_to_float(const BatchArgs& a, const double* A, float* S, hipStream_t s) {
-    if (a.count <= 0) return hipSuccess;
-    for (int first = 0; first < a.count; first += 32768)  // (a grid's y stays below 65536)
-        hipLaunchKernelGGL(batch_to_float_kernel, dim3(16, std::min(a.count - first, 32768)), dim3(256), 0, s, a, A, S,
-                           first);
-    return hipGetLastError();
-}
-
 hipError_t batch_residual(const BatchArgs& a, const double* A, const double* X, const double* B, double* R,
                           const int* prefix, int wgs, double* red, double* eta, double* rscale, int kmax,
-                          hipStream_t s) {
+                          hipStream_t s, float* S) {
     if (a.count <= 0 || wgs <= 0) return hipSuccess;
     const i64 nred = (i64)a.count * (1 + 3 * kmax);
     hipLaunchKernelGGL(batch_fill_kernel, dim3((unsigned)std::min<i64>(ceil_div(nred, 256), 1024)), dim3(256), 0, s,
                        red, 0.0, nred);
-    hipLaunchKernelGGL(batch_symv_residual_kernel, dim3((unsigned)wgs), dim3(256), 0, s, a, A, X, B, R, prefix,
-                       a.count, red, kmax);
+    auto kernel = S != nullptr ? batch_symv_residual_kernel<true> : batch_symv_residual_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, s, a, A, X, B, R, prefix, a.count, red, kmax, S);
     hipLaunchKernelGGL(batch_eta_kernel, dim3((unsigned)ceil_div(a.count, 256)), dim3(256), 0, s, a, red, eta, rscale,
                        kmax);
     return hipGetLastError();

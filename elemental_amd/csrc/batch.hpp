@@ -35,13 +35,13 @@ hipError_t batch_solve(const BatchArgs& a, const void* L, void* B, bool f32, int
 // F = A, or the float copy) as one launch of `grid` workgroups that take the
 // matrices from *counter (zeroed before).  nb <= kPersistMaxNb.
 hipError_t batch_persistent(const BatchArgs& a, void* F, int mode, int nb, int* counter, int grid, hipStream_t s);
-hipError_t batch_to_float(const BatchArgs& a, const double* A, float* S, hipStream_t s);
 // R := B - A X per matrix; eta (and rscale = ||r_c||_inf when non-null) per
 // matrix; prefix/wgs: 64-row blocks of the matrices; red: count*(1+3*kmax)
-// doubles of reduction scratch.
+// doubles of reduction scratch.  S (may be null): X is taken as zero, and S :=
+// float(A) (lower triangle) on the way.
 hipError_t batch_residual(const BatchArgs& a, const double* A, const double* X, const double* B, double* R,
                           const int* prefix, int wgs, double* red, double* eta, double* rscale, int kmax,
-                          hipStream_t s);
+                          hipStream_t s, float* S = nullptr);
 hipError_t batch_ir_prepare(const BatchArgs& a, const double* eta, double tol, const double* R, const double* rscale,
                             float* Rf, int kmax, int* iters, hipStream_t s);
 hipError_t batch_ir_update(const BatchArgs& a, const float* D, const double* rscale, double* X, int kmax,

@@ -244,7 +244,13 @@ static int enqueue(BatchPlan* P, double* A, double* B, void* work, hipStream_t s
         Rf = (float*)w;
     }
     const BatchArgs a = plan_args(P, false);
-    if (f32) ELEMAMD_HIP_TRY(batch_to_float(a, A, S, s));
+    const BatchArgs ai = plan_args(P, true);
+    const int* res_prefix = P->d_prefix + P->res_prefix_off;
+    // the refinement's first residual (X = 0) reads all of A: the float copy
+    // to factor is made on the way
+    if (f32)
+        ELEMAMD_HIP_TRY(batch_residual(ai, A, X, B, R, res_prefix, P->res_wgs, P->d_red, P->d_eta, P->d_rscale,
+                                       P->kmax, s, S));
     void* F = f32 ? (void*)S : (void*)A;
     for (const BatchRun& r : P->runs) {
         const BatchArgs ar = plan_args(P, r.first, r.count, false);
@@ -266,12 +272,11 @@ static int enqueue(BatchPlan* P, double* A, double* B, void* work, hipStream_t s
     // low-precision factor + FP64-residual refinement from X = 0: a fixed
     // number of sweeps (the sequence is replayable); a converged matrix is
     // skipped by every kernel of the remaining sweeps
-    const BatchArgs ai = plan_args(P, true);
-    const int* res_prefix = P->d_prefix + P->res_prefix_off;
     ELEMAMD_HIP_TRY(batch_copy_rhs(a, nullptr, X, nullptr, s));  // X := 0
     for (int it = 0; it < P->ir_sweeps; ++it) {
-        ELEMAMD_HIP_TRY(batch_residual(ai, A, X, B, R, res_prefix, P->res_wgs, P->d_red, P->d_eta, P->d_rscale,
-                                       P->kmax, s));
+        if (it > 0)
+            ELEMAMD_HIP_TRY(batch_residual(ai, A, X, B, R, res_prefix, P->res_wgs, P->d_red, P->d_eta, P->d_rscale,
+                                           P->kmax, s));
         ELEMAMD_HIP_TRY(batch_ir_prepare(ai, P->d_eta, P->tol, R, P->d_rscale, Rf, P->kmax, P->d_iters, s));
         ELEMAMD_HIP_TRY(batch_solve(ai, S, Rf, true, P->kmax, s));
         ELEMAMD_HIP_TRY(batch_ir_update(ai, Rf, P->d_rscale, X, P->kmax, s));
