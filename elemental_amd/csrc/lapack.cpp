@@ -462,6 +462,31 @@ bool cg_trace() {
     return on;
 }
 
+// One grow-only pinned buffer per host thread, kept until the thread ends.
+hipError_t pinned_doubles(size_t count, double** out) {
+    struct Pinned {
+        double* p = nullptr;
+        size_t cap = 0;
+        ~Pinned() {
+            if (p) (void)hipHostFree(p);
+        }
+    };
+    static thread_local Pinned b;
+    if (b.cap < count) {
+        if (b.p) {
+            const hipError_t e = hipHostFree(b.p);
+            if (e != hipSuccess) return e;
+        }
+        b.p = nullptr;
+        b.cap = 0;
+        const hipError_t e = hipHostMalloc((void**)&b.p, sizeof(double) * count, hipHostMallocDefault);
+        if (e != hipSuccess) return e;
+        b.cap = count;
+    }
+    *out = b.p;
+    return hipSuccess;
+}
+
 // Normwise backward error per column from the device column maxima of R
 // (dev[0..k)) and X (dev[k..2k)), copied to host; returns the maximum.
 int host_eta(Ctx& c, const std::vector<double>& bn, std::vector<double>& eta_c, double& eta) {
@@ -506,22 +531,8 @@ int cg_refine(Ctx& c, const MixedOpts& o, const std::vector<double>& bn, MixedRe
     if (sp == nullptr) return kErrHip;
     // column maxima of R and X land in pinned memory behind an event, so the
     // next step's preconditioner can be enqueued before the host reads them
-    // (one grow-only buffer per host thread, kept until the thread ends)
-    struct Pinned {
-        double* p = nullptr;
-        size_t cap = 0;
-        ~Pinned() {
-            if (p) (void)hipHostFree(p);
-        }
-    };
-    static thread_local Pinned nx;
-    if (nx.cap < 2 * (size_t)k) {
-        if (nx.p) ELEMAMD_HIP_TRY(hipHostFree(nx.p));
-        nx.p = nullptr;
-        nx.cap = 0;
-        ELEMAMD_HIP_TRY(hipHostMalloc((void**)&nx.p, sizeof(double) * 2 * k, hipHostMallocDefault));
-        nx.cap = 2 * (size_t)k;
-    }
+    double* nx = nullptr;
+    ELEMAMD_HIP_TRY(pinned_doubles(2 * (size_t)k, &nx));
     auto push_active = [&]() -> hipError_t {
         if (act == act_dev) return hipSuccess;
         act_dev = act;
@@ -530,7 +541,7 @@ int cg_refine(Ctx& c, const MixedOpts& o, const std::vector<double>& bn, MixedRe
     auto eta_enqueue = [&]() -> hipError_t {
         hipError_t e = launch_col_absmax(n, k, w.R, n, w.nrm + k, s);
         if (e == hipSuccess) e = launch_col_absmax(n, k, w.X, n, w.nrm + 2 * k, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(nx.p, w.nrm + k, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(nx, w.nrm + k, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipEventRecord(sp->ev_d, s);
         return e;
     };
@@ -540,7 +551,7 @@ int cg_refine(Ctx& c, const MixedOpts& o, const std::vector<double>& bn, MixedRe
         eta_c.resize(k);
         eta = 0.0;
         for (int col = 0; col < k; ++col) {
-            eta_c[col] = column_backward_error(nx.p[col], c.anorm, nx.p[k + col], bn[col]);
+            eta_c[col] = column_backward_error(nx[col], c.anorm, nx[k + col], bn[col]);
             eta = std::max(eta, eta_c[col]);
         }
         return hipSuccess;
@@ -919,7 +930,11 @@ int mixed_refine(int n, int k, const double* A, i64 lda, double* B, i64 ldb, con
     MixedWork w = carve_refine(work, work_bytes, n, k, m, o.refine == kRefineCG);
     if (work == nullptr || work_bytes < w.bytes) return kErrWorkspace;
     Ctx c{n, k, A, lda, B, ldb, w, &f, s, f.anorm};
-    std::vector<double> bn, xn, rn;
+    std::vector<double> bn;
+    StreamPair* sp = stream_pair(s);
+    if (sp == nullptr) return kErrHip;
+    double* nx = nullptr;
+    ELEMAMD_HIP_TRY(pinned_doubles(2 * (size_t)k, &nx));
     ELEMAMD_HIP_TRY(launch_col_absmax(n, k, B, ldb, w.nrm, s));
     bn.resize(k);
     ELEMAMD_HIP_TRY(hipMemcpyAsync(bn.data(), w.nrm, sizeof(double) * k, hipMemcpyDeviceToHost, s));
@@ -933,6 +948,7 @@ int mixed_refine(int n, int k, const double* A, i64 lda, double* B, i64 ldb, con
     int stall = 0;
     double eta = INFINITY;
     double gmres_prev = INFINITY;  // backward error before the last GMRES-IR cycle
+    double last = 1.0, rate = 1.0;  // the last step's backward error and its ratio to the one before
     int it0 = 0, cg_conv = 0;
     if (o.refine == kRefineCG && !gmres) {
         int rc = cg_refine(c, o, bn, r, eta, &cg_conv);
@@ -950,15 +966,26 @@ int mixed_refine(int n, int k, const double* A, i64 lda, double* B, i64 ldb, con
             ELEMAMD_HIP_TRY(launch_symm_lower_residual(n, k, A, lda, w.X, n, B, ldb, w.R, n, w.part, s));
             r.iterations = base + it;
         }
-        // norms
-        int rc = host_colmax(c, w.R, w.nrm + k, rn);
-        if (rc) return rc;
-        rc = host_colmax(c, w.X, w.nrm + 2 * k, xn);
-        if (rc) return rc;
+        // norms of R and X, into pinned memory behind an event
+        ELEMAMD_HIP_TRY(launch_col_absmax(n, k, w.R, n, w.nrm + k, s));
+        ELEMAMD_HIP_TRY(launch_col_absmax(n, k, w.X, n, w.nrm + 2 * k, s));
+        ELEMAMD_HIP_TRY(hipMemcpyAsync(nx, w.nrm + k, sizeof(double) * 2 * k, hipMemcpyDeviceToHost, s));
+        ELEMAMD_HIP_TRY(hipEventRecord(sp->ev_d, s));
+        // d = M^{-1} r in float touches neither X nor R: with the target out
+        // of reach of this step's expected contraction (the last one's) it is
+        // enqueued before the host has seen the norms
+        auto correction = [&]() -> hipError_t {
+            hipError_t e = launch_copy_f64_to_f32_scaled(n, k, w.R, n, w.nrm + k, w.Rf, n, s);
+            return e == hipSuccess ? launch_sweep_solve(n, k, f.S, n, f.tiles, w.Rf, n, w.sweep, s) : e;
+        };
+        const bool ahead = !gmres && it < o.max_iter && (it == 0 || (it > 1 && last * rate > 20.0 * o.tol));
+        if (ahead) ELEMAMD_HIP_TRY(correction());
+        ELEMAMD_HIP_TRY(hipEventSynchronize(sp->ev_d));
         eta = 0.0;
-        for (int col = 0; col < k; ++col) {
-            eta = std::max(eta, column_backward_error(rn[col], c.anorm, xn[col], bn[col]));
-        }
+        for (int col = 0; col < k; ++col)
+            eta = std::max(eta, column_backward_error(nx[col], c.anorm, nx[k + col], bn[col]));
+        if (it > 0) rate = std::min(1.0, eta / last);
+        last = eta;
         if (it > 0 && eta <= o.tol) break;
         if (it == o.max_iter) break;
         // with a fallback, a GMRES-IR cycle that does not halve the backward
@@ -973,14 +1000,13 @@ int mixed_refine(int n, int k, const double* A, i64 lda, double* B, i64 ldb, con
         prev = std::min(prev, eta);
         if (!gmres) {
             // d = M^{-1} r in float, x += d
-            ELEMAMD_HIP_TRY(launch_copy_f64_to_f32_scaled(n, k, w.R, n, w.nrm + k, w.Rf, n, s));
-            ELEMAMD_HIP_TRY(launch_sweep_solve(n, k, f.S, n, f.tiles, w.Rf, n, w.sweep, s));
+            if (!ahead) ELEMAMD_HIP_TRY(correction());
             ELEMAMD_HIP_TRY(launch_axpy_f32_to_f64_scaled(n, k, w.Rf, n, w.nrm + k, w.X, n, s));
         } else {
             r.used_gmres = 1;
             gmres_prev = eta;
             int gi = 0;
-            rc = gmres_cycle(c, m, 1e-8, &gi);
+            const int rc = gmres_cycle(c, m, 1e-8, &gi);
             if (rc) return rc;
             r.gmres_iterations += gi;
             // X += D
