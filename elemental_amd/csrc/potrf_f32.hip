@@ -24,20 +24,24 @@ namespace elemamd {
 
 constexpr int kPiLd = 132;  // LDS row stride (floats): MFMA operand reads are conflict-free
 
-// acc (16 x 16) += P (16 x 32) Q^T: rows pr.. of P from column pc, rows qr..
-// of Q from column qc, both row-major in LDS; all 16 operand loads are in
-// flight together, then the 8 MFMA steps.
+// acc[nt] (16 x 16 each) += P (16 x 32) Q^T, nt < 2: rows pr.. of P from column
+// pc, rows 16 nt .. of Q, both row-major in LDS; all 24 operand loads are in
+// flight together, then the 16 MFMA steps.
 template <int LP, int LQ>
-__device__ inline void tile_ab_t(f4_t& acc, const float (*P)[LP], int pr, int pc, const float (*Q)[LQ], int qr, int qc,
-                                 int m, int g) {
-    float pa[8], qb[8];
+__device__ inline void tile_ab_t(f4_t (&acc)[2], const float (*P)[LP], int pr, int pc, const float (*Q)[LQ], int m,
+                                 int g) {
+    float pa[8], qb[2][8];
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
         pa[ks] = P[pr + m][pc + 4 * ks + g];
-        qb[ks] = Q[qr + m][qc + 4 * ks + g];
+        qb[0][ks] = Q[m][4 * ks + g];
+        qb[1][ks] = Q[16 + m][4 * ks + g];
     }
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) mfma_acc(acc, pa[ks], qb[ks]);
+    for (int ks = 0; ks < 8; ++ks) {
+        mfma_acc(acc[0], pa[ks], qb[0][ks]);
+        mfma_acc(acc[1], pa[ks], qb[1][ks]);
+    }
 }
 
 // One b x b (b <= 128) diagonal block at A (float storage): L11 overwrites
@@ -207,7 +211,8 @@ __device__ __forceinline__ void panel_slab_update_lds(float (*sB)[kPiLd], unsign
 }
 
 // B (m x b, b <= 128) := B L11^{-T}, L11 the b x b float factor at L; one
-// 64-row slab per workgroup, the result staged through LDS so the
+// 64-row slab per workgroup (n = 4000, no pending update: 10.2 us a launch,
+// 15.1 with an address made anew for every load), the result staged through LDS so the
 // column-major stores are contiguous.  With NPU > 0 the slab first takes the
 // block column's pending update from the group's earlier panels (NPU planes
 // at upd, uk columns; panel_slab_update), so no separate kernel has to
@@ -233,19 +238,30 @@ __global__ __launch_bounds__(256) void panel_f32_kernel(int m, int b, const floa
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, m16 = lane & 15, g = lane >> 4;
     const i64 r0 = (i64)blockIdx.x * 64;
     const int rw = 16 * w;
+    // Addresses of whole slabs and blocks are steps from one load to the next
+    // (a wave alone on its SIMD pays 4 to 8 cycles for every instruction).
+    const bool whole = r0 + 64 <= m, full = b == 128;
     float v[32];
     {  // the slab: row t % 64, columns t / 64 + 4q
         const int rs = t & 63, c_lo = t >> 6;
-        const i64 rb = r0 + rs < m ? r0 + rs : m - 1;
+        if (whole && full) {
+            const float* src = B + r0 + rs + (i64)c_lo * ldb;
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int c = c_lo + 4 * q;
-            v[q] = B[rb + (i64)(c < b ? c : b - 1) * ldb];
-        }
+            for (int q = 0; q < 32; ++q, src += 4 * ldb) v[q] = *src;
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int c = c_lo + 4 * q;
-            sB[rs][c] = (r0 + rs < m && c < b) ? v[q] : 0.0f;
+            for (int q = 0; q < 32; ++q) sB[rs][c_lo + 4 * q] = v[q];
+        } else {
+            const i64 rb = r0 + rs < m ? r0 + rs : m - 1;
+#pragma unroll
+            for (int q = 0; q < 32; ++q) {
+                const int c = c_lo + 4 * q;
+                v[q] = B[rb + (i64)(c < b ? c : b - 1) * ldb];
+            }
+#pragma unroll
+            for (int q = 0; q < 32; ++q) {
+                const int c = c_lo + 4 * q;
+                sB[rs][c] = (r0 + rs < m && c < b) ? v[q] : 0.0f;
+            }
         }
     }
     // the slab's pending update: wave w on rows 16w .. 16w+15
@@ -257,27 +273,37 @@ __global__ __launch_bounds__(256) void panel_f32_kernel(int m, int b, const floa
             panel_slab_update<NPU>(sB, upd, ps, ldk, uk, b, m, r0, rw, m16, g);
         __syncthreads();  // the staging area becomes L11's blocks
     }
-    // block e / 1024: row e % 32 (lanes along the column), column (e / 32) % 32
+    // block q / 4: row t % 32 (lanes along the column), column t / 32 + 8 (q % 4)
     // (clamped loads, then select)
-    for (int e0 = 0; e0 < 6 * 1024; e0 += 32 * 256) {
+    {
+        const int rr = t & 31, c0 = t >> 5;
+        if (full) {
+            const float* src = L + rr + (i64)c0 * ldl;
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int e = e0 + t + 256 * q;
-            const int blk = e >> 10, rr = e & 31, cc = (e >> 5) & 31;
-            const int p = blk < 1 ? 1 : blk < 3 ? 2 : 3, qb = blk - p * (p - 1) / 2;
-            const int r = 32 * p + rr, c = 32 * qb + cc;
-            v[q] = (e < 6 * 1024) ? L[(r < b ? r : b - 1) + (i64)(c < b ? c : b - 1) * ldl] : 0.0f;
-        }
+            for (int q = 0; q < 24; ++q) {
+                const int blk = q >> 2, p = blk < 1 ? 1 : blk < 3 ? 2 : 3, qb = blk - p * (p - 1) / 2;
+                v[q] = src[32 * p + (i64)(32 * qb + 8 * (q & 3)) * ldl];
+            }
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int e = e0 + t + 256 * q;
-            const int blk = e >> 10, rr = e & 31, cc = (e >> 5) & 31;
-            const int p = blk < 1 ? 1 : blk < 3 ? 2 : 3, qb = blk - p * (p - 1) / 2;
-            const int r = 32 * p + rr, c = 32 * qb + cc;
-            if (e < 6 * 1024) sLb[blk][rr][cc] = (r < b && c < b) ? v[q] : 0.0f;
+            for (int q = 0; q < 24; ++q) sLb[q >> 2][rr][c0 + 8 * (q & 3)] = v[q];
+        } else {
+#pragma unroll
+            for (int q = 0; q < 24; ++q) {
+                const int blk = q >> 2, p = blk < 1 ? 1 : blk < 3 ? 2 : 3, qb = blk - p * (p - 1) / 2;
+                const int r = 32 * p + rr, c = 32 * qb + c0 + 8 * (q & 3);
+                v[q] = L[(r < b ? r : b - 1) + (i64)(c < b ? c : b - 1) * ldl];
+            }
+#pragma unroll
+            for (int q = 0; q < 24; ++q) {
+                const int blk = q >> 2, p = blk < 1 ? 1 : blk < 3 ? 2 : 3, qb = blk - p * (p - 1) / 2;
+                const int r = 32 * p + rr, c = 32 * qb + c0 + 8 * (q & 3);
+                sLb[blk][rr][c0 + 8 * (q & 3)] = (r < b && c < b) ? v[q] : 0.0f;
+            }
         }
     }
-    for (int e = t; e < 4 * 1024; e += 256) sXd[e >> 10][(e >> 5) & 31][e & 31] = Xd[e];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)  // (the rows of sXd are 16-byte aligned)
+        *reinterpret_cast<f4_t*>(&sXd[q][t >> 3][4 * (t & 7)]) = *reinterpret_cast<const f4_t*>(Xd + 1024 * q + 4 * t);
     __syncthreads();
     // wave w: rows 16w .. 16w+15 of the slab, pieces p = 0..3 in order (no
     // other wave touches these rows)
@@ -285,8 +311,7 @@ __global__ __launch_bounds__(256) void panel_f32_kernel(int m, int b, const floa
         f4_t acc[2] = {};
         for (int q = 0; q < p; ++q) {  // S = sum_q X_q L_pq^T
             const float(*Lpq)[36] = sLb[p * (p - 1) / 2 + q];
-            tile_ab_t(acc[0], sB, rw, 32 * q, Lpq, 0, 0, m16, g);
-            tile_ab_t(acc[1], sB, rw, 32 * q, Lpq, 16, 0, m16, g);
+            tile_ab_t(acc, sB, rw, 32 * q, Lpq, m16, g);
         }
         mfma_retire();
 #pragma unroll
@@ -295,8 +320,7 @@ __global__ __launch_bounds__(256) void panel_f32_kernel(int m, int b, const floa
             for (int v = 0; v < 4; ++v) sB[rw + 4 * g + v][32 * p + 16 * nt + m16] -= acc[nt][v];
         // X_p = T inv(L_pp)^T (T = the updated columns, this wave's rows only)
         f4_t x[2] = {};
-        tile_ab_t(x[0], sB, rw, 32 * p, sXd[p], 0, 0, m16, g);
-        tile_ab_t(x[1], sB, rw, 32 * p, sXd[p], 16, 0, m16, g);
+        tile_ab_t(x, sB, rw, 32 * p, sXd[p], m16, g);
         mfma_retire();
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt)
@@ -304,9 +328,15 @@ __global__ __launch_bounds__(256) void panel_f32_kernel(int m, int b, const floa
             for (int v = 0; v < 4; ++v) sB[rw + 4 * g + v][32 * p + 16 * nt + m16] = x[nt][v];
     }
     __syncthreads();
-    for (int idx = t; idx < 64 * 128; idx += 256) {
-        const int r = idx & 63, c = idx >> 6;
-        if (r0 + r < m && c < b) B[r0 + r + (i64)c * ldb] = sB[r][c];
+    if (whole && full) {
+        float* dst = B + r0 + (t & 63) + (i64)(t >> 6) * ldb;
+#pragma unroll
+        for (int q = 0; q < 32; ++q, dst += 4 * ldb) *dst = sB[t & 63][(t >> 6) + 4 * q];
+    } else {
+        for (int idx = t; idx < 64 * 128; idx += 256) {
+            const int r = idx & 63, c = idx >> 6;
+            if (r0 + r < m && c < b) B[r0 + r + (i64)c * ldb] = sB[r][c];
+        }
     }
     if (planes != nullptr) {  // bf16 planes of the result: thread = (row, 8 columns), 16-byte stores
         for (int e = t; e < 64 * 16; e += 256) {
