@@ -252,8 +252,9 @@ int elemamd_gemm_f64(char ta, char tb, int m, int n, int k, double alpha, const 
     const bool TA = is_trans(ta), TB = is_trans(tb);
     if (lda < std::max(1, TA ? k : m) || ldb < std::max(1, TB ? n : k) || ldc < std::max(1, m))
         return ELEMAMD_ERR_ARG;
-    // an operand that C overlaps (up to 128 x 128, read before it is written)
-    if (m > 0 && n > 0 && k > 0 && m <= 128 && n <= 128) {
+    // an operand that C overlaps is copied first (a product of up to 128 rows or
+    // columns may be in place)
+    if (m > 0 && n > 0 && k > 0 && (m <= 128 || n <= 128)) {
         const int ra = TA ? k : m, ca = TA ? m : k, rb = TB ? n : k, cb = TB ? k : n;
         auto overlaps = [&](const double* X, int64_t ldx, int r, int c) {
             return X < C + (n - 1) * ldc + m && C < X + (c - 1) * ldx + r;

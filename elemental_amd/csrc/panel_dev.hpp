@@ -1,5 +1,5 @@
-// Device code of the panel triangular solve B := B inv(L)^T, shared by the
-// single-matrix and batched launches.
+// Device code of the panel triangular solve B := B inv(L)^T in the reference
+// BLAS's column order.
 #pragma once
 
 #include "common.hpp"

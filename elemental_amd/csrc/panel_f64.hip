@@ -27,7 +27,8 @@
 // were four instructions, whose loads ran along columns (every lane an access
 // of its own) and whose addresses were made anew for each.  The
 // factorization and solve at n = 2048: 1.53 -> 1.27 ms.
-// 24 KB of LDS, so that a workgroup fits beside four of the trailing update.
+// 24 KB of LDS fit beside four workgroups of the trailing update; its 234
+// registers take the place of one that leaves.
 #include <algorithm>
 
 #include "common.hpp"

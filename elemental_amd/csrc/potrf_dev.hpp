@@ -1,5 +1,5 @@
-// Device code of the diagonal-block Cholesky (LVar3Unb), shared by the
-// single-matrix and batched launches.
+// Device code of the diagonal-block Cholesky in the reference's rounding order
+// (LVar3Unb).
 #pragma once
 
 #include "common.hpp"
@@ -146,14 +146,13 @@ struct PotrfGroups<128 / NTC, NTC> {
     }
 };
 
-// One n x n (n <= 128) diagonal block by the calling workgroup of THREADS
-// (512 or 256) threads.  The operation order per element is LVar3Unb's
-// whatever the thread count, so the result is the same bit for bit.
-template <typename T, int THREADS = kPotrfThreads>
+// One n x n (n <= 128) diagonal block by the calling workgroup of 512 threads;
+// the operation order per element is LVar3Unb's.
+template <typename T>
 __device__ __forceinline__ void potrf_unb_block(int n, T* __restrict__ A, i64 lda, int* __restrict__ info,
                                                 int col_offset) {
 #pragma clang fp contract(off)
-    constexpr int NTC = THREADS / 32, NBC = 128 / NTC;
+    constexpr int NTC = kPotrfThreads / 32, NBC = 128 / NTC;
     __shared__ double col[4][kPotrfMaxN];
     __shared__ int sfail;
     if (info != nullptr && *info != 0 && *info <= col_offset) return;  // an earlier block failed

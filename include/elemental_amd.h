@@ -203,7 +203,7 @@ int elemamd_hermitian_gen_definite_eig_f64(int type, char uplo, int n, double *A
  * factorization keeps each 128 x 128 diagonal block's factor in FP64 before
  * storing it as float, solves the panels by products with the inverses of
  * its 32 x 32 diagonal pieces and updates the trailing matrix with FP32
- * MFMA; the float solves use the inverses of the 64 x 64 diagonal blocks. */
+ * MFMA; the float solves substitute in 16-row tiles. */
 int elemamd_cholesky_f32(char uplo, int n, float *A, int64_t lda, int nb, int *dinfo, void *stream);
 int elemamd_solve_after_f32(char uplo, char orientation, int n, int k, const float *A, int64_t lda, float *B,
                             int64_t ldb, void *stream);

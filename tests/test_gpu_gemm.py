@@ -61,9 +61,10 @@ def test_triangles(uplo, n):
     assert np.array_equal(Cm.to_numpy(), np.where(mask, C + 2.0 * (A @ B), C))
 
 
-def test_operand_in_place():
+@pytest.mark.parametrize("m", [100, 300])
+def test_operand_in_place(m):
     rng = np.random.default_rng(5)
-    A, B = ints(rng, 100, 100), ints(rng, 100, 100)
+    A, B = ints(rng, m, 100), ints(rng, 100, 100)
     Am = E.Matrix.from_numpy(A)
     E.Gemm(E.NORMAL, E.NORMAL, 1.0, Am, E.Matrix.from_numpy(B), 0.0, Am)
     torch.cuda.synchronize()
