@@ -59,8 +59,10 @@ static hipError_t syrk_launch(int trailing, int m, int n, int k, const T* A, i64
 // columns left
 template <typename T>
 static int update_depth(int trailing, int rem) {
-    if (sizeof(T) == 8) return rem > kUpdateDepthF64Rem ? kUpdateDepthF64Large : kUpdateDepthF64;
-    return trailing == kTrailingF32 ? kUpdateDepthF32 : kUpdateDepthBf16x3;
+    if (sizeof(T) == 8)
+        return rem > kUpdateDepthF64Rem ? kUpdateDepthF64Large : rem > kForkRem ? kUpdateDepthF64 : kUpdateDepthSmall;
+    if (trailing != kTrailingF32) return kUpdateDepthBf16x3;
+    return rem > kUpdateDepthF32Rem ? kUpdateDepthF32 : kUpdateDepthSmall;
 }
 
 // bf16 planes of the float factor's panels (two alternating sets) and the

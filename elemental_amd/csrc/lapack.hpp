@@ -16,12 +16,16 @@ enum : int { kRefineIR = 0, kRefineCG = 1 };
 
 // Columns of panels applied per pass over the trailing matrix (a multiple of
 // the block size nb is used: max(1, depth / nb) panels).
-// FP64: 512 while more than 8192 columns are left (the trailing update sets
-// the pace and runs at 61 TF/s instead of 54), 256 below (the chain sets the
-// pace, and a deeper group has more of it).  n = 16384 solve: 256 throughout
-// 40.2 ms, 512 throughout 39.2, the change at 4096, 6144 or 8192 columns 38.4,
-// at 10240 38.6; n = 2048: 256 1.78 ms, 512 1.85.
-constexpr int kUpdateDepthF64 = 256, kUpdateDepthF64Large = 512, kUpdateDepthF64Rem = 8192;
+// FP64: 768 while more than 8192 columns are left (the trailing update sets
+// the pace), 256 below (the chain sets the pace, and a deeper group has more
+// of it); n = 16384 solve: 33.6 ms with 512, 33.1 with 768, 33.4 with 1024, 33.4
+// with 512 down to 4096 columns.  Where a pass is one launch on the caller's
+// stream a group's inner updates cost more than the passes they save: 128 for
+// FP64 (n = 2048: 1098 us with 256, 1081; n = 3001: 1734, 1720) and, from 1024
+// columns on, for float (n = 4000: 2039 us with 512, 2011; from 2048 on 2000,
+// but mixed n = 5003, whose preparation goes by groups, 3329 instead of 3251).
+constexpr int kUpdateDepthF64 = 256, kUpdateDepthF64Large = 768, kUpdateDepthF64Rem = 8192;
+constexpr int kUpdateDepthSmall = 128, kUpdateDepthF32Rem = 1024;
 // Rows left up to which a trailing pass is one launch on the caller's stream
 // (planes of BF16 apart).  An event pair costs the chain 10 to 20 us there and
 // the next group's columns alone another launch of 12 to 22; with 2048 rows
