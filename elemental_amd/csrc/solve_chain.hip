@@ -66,7 +66,12 @@ namespace chain {
 
 constexpr int D = 3;          // blocks before its own that the chain workgroup applies (a helper the older ones)
 constexpr int RH = 4;         // helper: blocks of solved rows in LDS
-constexpr int kMaxSlabs = 8;  // slabs per launch: more right-hand sides take several launches
+// Slabs per launch (more right-hand sides take several launches): as many as
+// leave every workgroup a CU of its own, at least 8.  More than that and the
+// helpers of one slab keep the chains of others waiting: n = 8192, 256 columns
+// 1.28 ms in two launches, 2.2 to 7.8 in one.  Fewer, and small factors pay for
+// launches: n = 512, 400 columns 155 us with 8, 60 with all 25.
+constexpr int kMinSlabs = 8, kCus = 256;
 
 // R = 5: the band, the current block, the one being published
 template <typename T, int NV>
@@ -274,12 +279,13 @@ hipError_t launch_trsm_chain(bool forward, bool backward, int n, int kc, const T
     if (e != hipSuccess) return e;
     const long spin = solve_spin_limit();
     const int nT = (int)ceil_div(n, kSB);
+    const int slabs = std::max(chain::kMinSlabs, chain::kCus / (1 + std::max(0, nT - chain::D - 1)));
     int base = 0, epoch = 0;
     for (int dir = 0; dir < 2; ++dir) {
         if (dir == 0 ? !forward : !backward) continue;
         ++epoch;
-        for (int c0 = 0; c0 < kc; c0 += chain::kMaxSlabs * kSC) {
-            const int k = std::min(kc - c0, chain::kMaxSlabs * kSC), CY = (int)ceil_div(k, kSC);
+        for (int c0 = 0; c0 < kc; c0 += slabs * kSC) {
+            const int k = std::min(kc - c0, slabs * kSC), CY = (int)ceil_div(k, kSC);
             const unsigned grid = (unsigned)(CY + CY * std::max(0, nT - chain::D - 1));
             int* flags = ctrl + 2 + 2 * nT * (c0 / kSC);
             T* Bc = B + (i64)c0 * ldb;

@@ -43,6 +43,21 @@ def test_trsm_shapes(n, k, uplo, trans, unit):
     assert (np.abs(host(Bd) - X) <= 4 * bound).all()
 
 
+@pytest.mark.parametrize("n,k", [(70, 300), (400, 1100), (1100, 150), (2100, 300)])
+def test_many_columns(n, k):
+    """Several slabs a launch and several launches: every column as alone."""
+    stored, T = triangle(n, False, False, seed=n)
+    B = inputs.normal_host(n, k, seed=3)
+    Ad, Bd = E.Matrix.from_numpy(stored, ldim=n + 1), E.Matrix.from_numpy(B)
+    E.Trsm(E.LEFT, E.LOWER, E.TRANSPOSE, E.NON_UNIT, 1.0, Ad, Bd)
+    X = host(Bd)
+    for c0 in range(0, k, 16):
+        one = E.Matrix.from_numpy(np.asfortranarray(B[:, c0:c0 + 16]))
+        E.Trsm(E.LEFT, E.LOWER, E.TRANSPOSE, E.NON_UNIT, 1.0, Ad, one)
+        assert np.array_equal(host(one), X[:, c0:c0 + 16])
+
+
+
 @pytest.mark.parametrize("n,k", [(2500, 130), (1000, 300)])
 def test_many_columns_integer_exact(n, k):
     A, L0 = inputs.integer_factor(n, seed=n)
