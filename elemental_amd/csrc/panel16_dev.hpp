@@ -17,15 +17,17 @@ struct Lds {
 };
 
 // acc += A B over 16 contraction steps, four FP64 MFMAs in one statement (an
-// instruction of the same wave between two of them would wait for the first);
-// acc may be read 18 wait states later.
+// instruction of the same wave between two of them would wait for the first).
+// The statement ends with the wait states after which acc may be read: the
+// compiler, which does not know that it holds MFMAs, may copy or spill acc
+// right behind it.
 __device__ __forceinline__ void mfma_tile(d4_t& acc, const double (&a)[4], const double (&b)[4]) {
     asm volatile(
         "s_nop 1\n\t"
         "v_mfma_f64_16x16x4_f64 %0, %1, %5, %0\n\t"
         "v_mfma_f64_16x16x4_f64 %0, %2, %6, %0\n\t"
         "v_mfma_f64_16x16x4_f64 %0, %3, %7, %0\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %4, %8, %0"
+        "v_mfma_f64_16x16x4_f64 %0, %4, %8, %0\n\ts_nop 15\n\ts_nop 1"
         : "+v"(acc)
         : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
 }
@@ -178,8 +180,6 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
             if (p < np) mfma_tile(a[p], fa, y[p - 1]);
             if (p > q + 1) load_y(p, q + 1);
         }
-        // wait states before the next tile is read
-        asm volatile("s_nop 15\n\ts_nop 7" : "+v"(a[q + 1 < kTiles ? q + 1 : q]));
     }
     // (all stores at the end: a load behind a store waits for both)
     if (full && rw + 16 <= m) {
