@@ -18,7 +18,9 @@
 //   sides as rows) in the MFMA accumulator layout, and substitutes in
 //   registers with DPP row broadcasts: a_c -= a_k (l_ck / l_kk), then a
 //   scaling by the reciprocal diagonal (exact on integer problems with
-//   power-of-two diagonals).  A solved tile is written to LDS with a sequence
+//   power-of-two diagonals; a tile that this does not serve, because a
+//   multiplier over- or underflows or a row is not finite, is solved again
+//   as the reference's loop does it, solve_tile_careful).  A solved tile is written to LDS with a sequence
 //   number behind it (the LDS unit serves a wave's accesses in order); the
 //   other waves poll that number, so no barrier holds the waves together.
 //   The products with the block before and with the own block's earlier tiles

@@ -28,7 +28,10 @@ struct Lds {
     T Y[R][kSB][KC + 1];    // solved blocks [row][column]
     T Bv[RB][kSB][KC + 1];  // right-hand sides less the sums made elsewhere
     T Sb[RB][kSB][KC + 1];  // the band's sums
-    T M[RB][kSB][17];       // multipliers [row][column in the tile], [15]: reciprocal diagonal
+    // multipliers [row][column in the tile], [15]: reciprocal diagonal; for a
+    // tile with one that is not an ordinary number the coefficients themselves
+    // and NaN in [15]; [16]: the reciprocal diagonal in either case
+    T M[RB][kSB][17];
     int seq;                // tiles solved
     int fetched[2];         // blocks in Bv and M (counting each fetching wave's own)
     int taken[2];           // blocks read out of Y (counting each publishing wave's own)
@@ -96,6 +99,11 @@ struct Substitute {
     }
 };
 
+// Classes of v_cmp_class: normal numbers, infinities, infinities and NaN.
+constexpr int kNormal = 0x108, kInfinite = 0x204, kNotFinite = 0x207;
+__device__ __forceinline__ bool is_class(double x, int c) { return __builtin_amdgcn_class(x, c); }
+__device__ __forceinline__ bool is_class(float x, int c) { return __builtin_amdgcn_classf(x, c); }
+
 // The tile's multipliers: m[k] := l_ck / l_kk for k < c, else 0 (lane c of
 // every 16-lane row holds row c's coefficients in m; r its reciprocal
 // diagonal).
@@ -121,6 +129,15 @@ struct Multipliers {
         const T rk = row_lane<K>(r);
         m[K] = K < c ? m[K] * rk : T(0);
         if constexpr (K < 14) Multipliers<T, K + 1>::run(m, r, c);
+    }
+    // the same from the coefficients l; true where a multiplier lost its value
+    // (with l_kk = 0 an infinite one has not)
+    static __device__ __forceinline__ bool checked(T (&m)[15], const T (&l)[15], T r, int c) {
+        const T rk = row_lane<K>(r);
+        m[K] = K < c ? l[K] * rk : T(0);
+        const bool lost = (K < c) & (l[K] != T(0)) & !is_class(m[K], kNormal) & !is_class(rk, kInfinite);
+        if constexpr (K < 14) return lost | Multipliers<T, K + 1>::checked(m, l, r, c);
+        return lost;
     }
 };
 
@@ -210,23 +227,30 @@ __device__ __forceinline__ void fetch_blocks(S& sh, const Rows<T, TRANS, CONTIG>
         const i64 i = (i64)pos * kSB + lane;
         const bool in = i < L.n;
         const i64 ic = in ? i : L.n - 1, t0 = ic - (ic & 15);  // (clamped) row, its tile's first row
-        T m[15], b[KC];
+        T m[15], l[15], b[KC];
 #pragma unroll
-        for (int k = 0; k < 15; ++k) m[k] = L.L[ic * L.rs + lesser(t0 + k, ic) * L.cs];
+        for (int k = 0; k < 15; ++k) l[k] = L.L[ic * L.rs + lesser(t0 + k, ic) * L.cs];
         const T dd = L.L[ic * L.rs + ic * L.cs];
         const i64 row = L.phys(ic);
 #pragma unroll
         for (int c = 0; c < KC; ++c) b[c] = B[row + (i64)min(c, kcl - 1) * ldb];
         // multipliers l_ck / l_kk of the tile's earlier columns
         const T r = in && !unit ? T(1) / dd : T(1);
-        Multipliers<T, 0>::run(m, r, in ? lane & 15 : 0);
+        const int c16 = in ? lane & 15 : 0;
+        const bool lost = Multipliers<T, 0>::checked(m, l, r, c16) | (r != r);
+        // the whole tile takes the coefficients then
+        const bool careful = (__ballot(lost) >> (lane & 48) & 0xffff) != 0;
+        if (careful)
+#pragma unroll
+            for (int k = 0; k < 15; ++k) m[k] = k < c16 ? l[k] : T(0);
         less(pos, ic, b);
         await(&sh.seq, 4 * (pos - RB + 1), limit, &sh.err);  // the slot's last block is solved
 #pragma unroll
         for (int c = 0; c < KC; ++c) sh.Bv[pos % RB][lane][c] = b[c];
 #pragma unroll
         for (int k = 0; k < 15; ++k) sh.M[pos % RB][lane][k] = m[k];
-        sh.M[pos % RB][lane][15] = r;
+        sh.M[pos % RB][lane][15] = careful ? T(__builtin_nan("")) : r;
+        sh.M[pos % RB][lane][16] = r;
         post(&sh.fetched[u], pos / 2 + 1);
     }
 }
@@ -264,6 +288,47 @@ __device__ __forceinline__ void hand_over(S& sh, int pos, int w, int lane, const
 #pragma unroll
     for (int v = 0; v < (S::KC + 3) / 4; ++v) sh.Sb[pos % S::RB][16 * w + (lane & 15)][mfma_row<T>(lane, v)] = acc[v];
     post(&sh.band[w], pos + 1);
+}
+
+// A tile once more, row by row as the reference's loop: x_k = a_k r_k, then
+// a_c -= l_ck x_k for the later rows only.  The substitution in registers lets
+// a row that is not finite into the tile's earlier rows (zero times infinity),
+// and its multipliers l_ck / l_kk may overflow or vanish where x_k does not;
+// the chain comes here when a result is not finite, which the NaN of a tile
+// kept as coefficients sees to.  The rows pass through their places in sh.Y.
+// n = 4096, 16 columns, forward: 253 us, 1130 with every tile solved here; the
+// test alone costs 0.6 % (n = 8192, both solves: 1007 and 1013 us).
+template <int NV, typename S, typename A>
+__device__ __forceinline__ void solve_tile_careful(S& sh, int pos, int w, int lane, bool in, const A& acc) {
+    typedef typename S::value T;
+    const int c16 = lane & 15, row = 16 * w + c16;
+    const T(*Ms)[17] = sh.M[pos % S::RB];
+    T(*Y)[S::KC + 1] = sh.Y[pos % S::R];
+    const bool coefficients = Ms[row][15] != Ms[row][15];
+    T a[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const int c = mfma_row<T>(lane, v);
+        a[v] = in ? sh.Bv[pos % S::RB][row][c] - sh.Sb[pos % S::RB][row][c] - acc[v] : T(0);
+    }
+#pragma unroll 1
+    for (int k = 0; k < 15; ++k) {
+        const T m = Ms[row][k], rk = Ms[16 * w + k][16];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) Y[row][mfma_row<T>(lane, v)] = a[v];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            // (m has l_ck's zeros and, but for r_k's, its sign)
+            const T ak = Y[16 * w + k][mfma_row<T>(lane, v)], xk = ak * rk;
+            const bool far = !coefficients & is_class(xk, kNotFinite);
+            const T f = far & (rk < T(0)) ? -m : m, x = coefficients | far ? xk : ak;
+            if (in & (c16 > k)) a[v] = fma(-f, x, a[v]);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) Y[row][mfma_row<T>(lane, v)] = a[v] * Ms[row][16];
 }
 
 // Chain wave w: solves the tiles 4 pos + w.
@@ -337,8 +402,14 @@ __device__ __forceinline__ void solve_tiles(S& sh, const Rows<T, TRANS, CONTIG>&
         for (int v = 0; v < NV; ++v) asm volatile("s_nop 0" : "+v"(a[v]));  // all written, two states before the first DPP read
         if constexpr (NV == 1) asm volatile("s_nop 0");
         Substitute<T, NV, 0>::run(a, m);
+        bool lost = false;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) sh.Y[pos % R][16 * w + c16][mfma_row<T>(lane, v)] = a[v] * r;
+        for (int v = 0; v < NV; ++v) {
+            a[v] *= r;
+            sh.Y[pos % R][16 * w + c16][mfma_row<T>(lane, v)] = a[v];
+            lost = lost | is_class(a[v], kNotFinite);
+        }
+        if (__ballot(lost) != 0) solve_tile_careful<NV>(sh, pos, w, lane, in, acc);
         post(&sh.seq, 4 * pos + w + 1);
     }
 }
