@@ -29,7 +29,10 @@
 // piece_careful(), which follows LVar3Unb's columns in LDS with real square
 // roots and divisions: +infinity goes on as in the reference loop, and a
 // failing column leaves the reference's state (columns before it factored,
-// the trailing triangle updated by them).
+// the trailing triangle updated by them).  So does every piece of a
+// block that holds an infinity or NaN off its diagonal tiles: the tiles'
+// substitution would let it into the row's earlier columns (zero times
+// infinity).  The waves look for one while the first piece is factored.
 #pragma once
 
 #include "common.hpp"
@@ -48,7 +51,7 @@ struct Lds {
     double D[16][18];          // the diagonal tile before its factorization, by rows
     double M[16][18];          // [c][k]: l_ck / l_kk for c > k, else 0 (the piece's multipliers)
     double V[kV][16][17];      // wave w, [w % kV]: its diagonal tile's unscaled columns [column][row]; then its inverse (INV)
-    int bad;
+    int bad;                   // bit 0: this piece goes through piece_careful(), bit 1: every piece
 };
 
 // acc -= (lane N of the 16-lane row's x) * l.  The DPP operand needs two wait
@@ -263,6 +266,8 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
     const int w0 = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int np = (b + 15) / 16;
     const bool full = b == 16 * kWaves;
+    if (tid == 0) sh.bad = 0;
+    __syncthreads();
     // tile row w, tiles 0 .. w (zero past b, the padded diagonal one; the
     // diagonal tile whole, mirrored).  16 rows by 4 columns per load, whole
     // lines (with lanes along columns every lane is an access of its own, 64
@@ -325,7 +330,15 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
                     const int i = 16 * (w0 + NW * r) + g + 4 * v, j = 16 * J + c;
                     if (i >= b || j >= b) t[r][J][v] = i == j ? 1.0 : 0.0;
                 }
-    if (tid == 0) sh.bad = 0;
+    bool odd = false;
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int J = 0; J < NW * (r + 1) - 1; ++J)
+            if (J < w0 + NW * r)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) odd = odd | __builtin_amdgcn_class(t[r][J][v], 0x207);
+    if (__ballot(odd) != 0 && lane == 0) atomicOr(&sh.bad, 2);
     if (w0 == 0) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) sh.D[g + 4 * v][c] = t[0][0][v];
@@ -364,7 +377,7 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
             const double piv = bcast<0>(d[0]);
             bool good = __builtin_amdgcn_class(piv, 0x180);
             Column<0>::run(d, rsqrt_full(piv), c, good, sh.M, sh.V[p % Lds<INV>::kV]);
-            if (!good && lane == 0) sh.bad = 1;
+            if (!good && lane == 0) atomicOr(&sh.bad, 1);
             __builtin_amdgcn_s_setprio(2);
         }
         if (p > 0)  // t[r][0]: this piece's tile
@@ -400,7 +413,7 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
                     for (int v = 0; v < 4; ++v) sh.X[c][16 * (w0 + NW * r) + g + 4 * v] = t[r][0][v];
             if (mine && p > 0) store_tile(p, p - 1);
             __syncthreads();
-            if (tid == 0) sh.bad = 0;
+            if (tid == 0) atomicAnd(&sh.bad, 2);
             kend = piece_careful(sh, p, 16 * np);
             if (kend < 16) failed = 16 * p + kend + 1;
             if (mine) {
