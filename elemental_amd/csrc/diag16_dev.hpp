@@ -412,6 +412,13 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
 #pragma unroll
                     for (int v = 0; v < 4; ++v) sh.X[c][16 * (w0 + NW * r) + g + 4 * v] = t[r][0][v];
             if (mine && p > 0) store_tile(p, p - 1);
+            // (with INV, tile (p, p-1), whose rows piece_careful() takes, comes
+            // back afterwards, since the end needs it; sh.M is free here)
+            int lk = lane;  // (opaque, as in store_tile)
+            asm volatile("" : "+v"(lk));
+            if (INV && mine)
+#pragma unroll 1
+                for (int q = lk >> 4; q < 16; q += 4) sh.M[q][lk & 15] = sh.X[q][16 * p + (lk & 15)];
             __syncthreads();
             if (tid == 0) atomicAnd(&sh.bad, 2);
             kend = piece_careful(sh, p, 16 * np);
@@ -419,6 +426,10 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
             if (mine) {
 #pragma unroll 1
                 for (int q = 0; q < 16; ++q) sh.V[p % Lds<INV>::kV][q][c] = sh.X[q][16 * p + c];
+                __builtin_amdgcn_wave_barrier();
+                if (INV && !failed)  // (a failing piece's pivot may still be read; nothing needs the tile then)
+#pragma unroll 1
+                    for (int q = lk >> 4; q < 16; q += 4) sh.X[q][16 * p + (lk & 15)] = sh.M[q][lk & 15];
             }
             if (failed) {
                 for (int w = w0; w < np; w += NW)
@@ -533,8 +544,8 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
             Xp[(h + g + 4 * v) * 32 + h + c] = (float)sh.V[w][g + 4 * v][c];
         d4_t y = {0.0, 0.0, 0.0, 0.0};
         if ((w & 1) && w < np) {
-            // L21 = tile (w, w-1): its rows of sh.X still hold it (later pieces
-            // wrote only later rows)
+            // L21 = tile (w, w-1): its rows of sh.X still hold it (a later piece
+            // wrote only later rows, or put them back)
             d4_t z = {0.0, 0.0, 0.0, 0.0};
             double fa[4], fb[4];
 #pragma unroll

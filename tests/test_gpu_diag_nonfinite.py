@@ -57,3 +57,18 @@ def test_entry_below_the_diagonal(row, col, value, dtype, tol):
     fin = np.isfinite(want)
     assert np.array_equal(np.isfinite(got), fin)
     assert np.linalg.norm(got[fin] - want[fin]) <= tol * np.linalg.norm(want[fin])
+
+
+@pytest.mark.parametrize("col", [3, 20, 47, 112, 140])
+def test_infinite_pivot_float(oracle, col):
+    n = 300
+    A = matrix(n, "f32", 8)
+    A[col, col] = np.inf
+    ref = np.asfortranarray(A.astype(np.float64))
+    assert oracle.lvar3(ref, 128) == 0
+    M = E.Matrix.from_numpy(A)
+    E.Cholesky(E.LOWER, M)
+    got, want = np.tril(host(M).astype(np.float64)), np.tril(ref)
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and not np.isnan(got).any()
+    fin = np.isfinite(want)
+    assert np.linalg.norm(got[fin] - want[fin]) <= 2e-5 * np.linalg.norm(want[fin])
