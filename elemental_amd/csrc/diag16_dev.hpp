@@ -36,6 +36,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "solve_dev.hpp"
 
 namespace elemamd {
 namespace diag16 {
@@ -118,21 +119,6 @@ __device__ __forceinline__ double fma_here(double a, double b, double c) {
     double r;
     asm volatile("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
-}
-
-// acc += A B over 16 contraction steps (four FP64 MFMAs) and the wait states
-// before acc may be read, in one statement: nothing the compiler puts between
-// the products (copies of the accumulator at the ends of branches) can read
-// it too early.
-__device__ __forceinline__ void mfma_tile(d4_t& acc, const double (&a)[4], const double (&b)[4]) {
-    asm volatile(
-        "s_nop 1\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %1, %5, %0\n\ts_nop 1\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %2, %6, %0\n\ts_nop 1\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %3, %7, %0\n\ts_nop 1\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %4, %8, %0\n\ts_nop 15\n\ts_nop 7"
-        : "+v"(acc)
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
 }
 
 // d[C] -= l_C l of the diagonal tile, C = FROM .. TO - 1 (below 16).

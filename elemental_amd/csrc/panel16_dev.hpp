@@ -16,22 +16,6 @@ struct Lds {
     double X[4][16][16];       // wave w: a tile, [row][column ^ row]
 };
 
-// acc += A B over 16 contraction steps, four FP64 MFMAs in one statement (an
-// instruction of the same wave between two of them would wait for the first).
-// The statement ends with the wait states after which acc may be read: the
-// compiler, which does not know that it holds MFMAs, may copy or spill acc
-// right behind it.
-__device__ __forceinline__ void mfma_tile(d4_t& acc, const double (&a)[4], const double (&b)[4]) {
-    asm volatile(
-        "s_nop 1\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %1, %5, %0\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %2, %6, %0\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %3, %7, %0\n\t"
-        "v_mfma_f64_16x16x4_f64 %0, %4, %8, %0\n\ts_nop 15\n\ts_nop 1"
-        : "+v"(acc)
-        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
-}
-
 // a[v] -= (lane K of the 16-lane row's a[v]) m[K] for K = 0 .. 14
 template <int K>
 struct TileColumn {

@@ -66,6 +66,23 @@ __device__ inline void mfma_acc_bf16(f4_t& acc, s8_t a, s8_t b) {
     asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
 
+// acc += A B over 16 contraction steps, four FP64 16x16x4 MFMAs in one
+// statement (an instruction of the same wave between two of them would wait
+// for the first).  It ends with the wait states after which anything may read
+// acc, 19 for a vector instruction or an MFMA operand and 18 for a store: the
+// compiler, which does not know that it holds MFMAs, may copy or spill acc
+// right behind it.
+__device__ __forceinline__ void mfma_tile(d4_t& acc, const double (&a)[4], const double (&b)[4]) {
+    asm volatile(
+        "s_nop 1\n\t"
+        "v_mfma_f64_16x16x4_f64 %0, %1, %5, %0\n\t"
+        "v_mfma_f64_16x16x4_f64 %0, %2, %6, %0\n\t"
+        "v_mfma_f64_16x16x4_f64 %0, %3, %7, %0\n\t"
+        "v_mfma_f64_16x16x4_f64 %0, %4, %8, %0\n\ts_nop 15\n\ts_nop 2"
+        : "+v"(acc)
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
+}
+
 // Store of a value another workgroup will read (device-coherent, bypassing
 // the per-XCD caches that are not coherent across XCDs) and the matching load.
 template <typename T>
