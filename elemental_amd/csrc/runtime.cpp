@@ -1,5 +1,6 @@
 #include "runtime.hpp"
 
+#include <atomic>
 #include <cstdlib>
 #include <initializer_list>
 #include <map>
@@ -61,6 +62,16 @@ long solve_spin_limit() {
         if (l > 0) return l;
     }
     return 1L << 26;
+}
+
+int device_cus() {
+    static std::atomic<int> known[64];  // (zero until asked for)
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64 && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64) known[dev].store(cus, std::memory_order_relaxed);
+    return cus;
 }
 
 void* stream_scratch(size_t bytes, hipStream_t stream) {

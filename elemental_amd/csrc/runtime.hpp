@@ -30,4 +30,7 @@ StreamPair* stream_pair(hipStream_t stream);
 // every launch; tests set a tiny limit to exercise the error path).
 long solve_spin_limit();
 
+// Compute units of the current device (0 on failure).
+int device_cus();
+
 }  // namespace elemamd

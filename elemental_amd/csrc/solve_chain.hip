@@ -52,11 +52,14 @@
 // acknowledgement of its stores before it raises a flag (solve_dev.hpp).
 // Workgroups take tickets in launch order: the chains first, then helpers by
 // increasing position, so every wait is on a workgroup that is running or
-// done.  Every wait is bounded (spin_limit polls, then an error in ctrl[1],
-// which the caller clears once per solve, so a wait that gave up in the
-// forward solve is still reported after the backward one).
+// done, or (a chain's) on the next helper to be dispatched, for which
+// chain_slabs() leaves CUs as long as no more than four such launches run at a
+// time, one for each hardware queue.  Every wait is bounded (spin_limit polls,
+// then an error in ctrl[1], which the caller clears once per solve, so a wait
+// that gave up in the forward solve is still reported after the backward one).
 #include <algorithm>
 
+#include "chain_slabs.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 #include "runtime.hpp"
@@ -68,13 +71,6 @@ namespace chain {
 
 constexpr int D = 3;          // blocks before its own that the chain workgroup applies (a helper the older ones)
 constexpr int RH = 4;         // helper: blocks of solved rows in LDS
-// Slabs per launch (more right-hand sides take several launches): as many as
-// leave every workgroup a CU of its own, at least 8.  More than that and the
-// helpers of one slab keep the chains of others waiting: n = 8192, 256 columns
-// 1.28 ms in two launches, 2.2 to 7.8 in one.  Fewer, and small factors pay for
-// launches: n = 512, 400 columns 155 us with 8, 60 with all 25.
-constexpr int kMinSlabs = 8, kCus = 256;
-
 // R = 5: the band, the current block, the one being published
 template <typename T, int NV>
 struct Shared : Lds<T, columns<T>(NV), 5, 3> {
@@ -281,14 +277,16 @@ hipError_t launch_trsm_chain(bool forward, bool backward, int n, int kc, const T
     if (e != hipSuccess) return e;
     const long spin = solve_spin_limit();
     const int nT = (int)ceil_div(n, kSB);
-    const int slabs = std::max(chain::kMinSlabs, chain::kCus / (1 + std::max(0, nT - chain::D - 1)));
+    const int cus = device_cus();
+    if (cus <= 0) return hipErrorInvalidDevice;
+    const int helpers = std::max(0, nT - chain::D - 1), slabs = chain_slabs(helpers, cus);
     int base = 0, epoch = 0;
     for (int dir = 0; dir < 2; ++dir) {
         if (dir == 0 ? !forward : !backward) continue;
         ++epoch;
         for (int c0 = 0; c0 < kc; c0 += slabs * kSC) {
             const int k = std::min(kc - c0, slabs * kSC), CY = (int)ceil_div(k, kSC);
-            const unsigned grid = (unsigned)(CY + CY * std::max(0, nT - chain::D - 1));
+            const unsigned grid = (unsigned)(CY + CY * helpers);
             int* flags = ctrl + 2 + 2 * nT * (c0 / kSC);
             T* Bc = B + (i64)c0 * ldb;
             T* pc = part + (i64)c0 * n;
