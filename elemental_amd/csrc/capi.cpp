@@ -6,6 +6,7 @@
 #include "batch.hpp"
 #include "kernels.hpp"
 #include "lapack.hpp"
+#include "overlap.hpp"
 #include "runtime.hpp"
 #include "server.hpp"
 
@@ -104,7 +105,9 @@ int elemamd_herk_f64(char uplo, char trans, int n, int k, double alpha, const do
     if (n < 0 || k < 0 || lda < std::max(1, tr ? k : n) || ldc < std::max(1, n)) return ELEMAMD_ERR_ARG;
     if (n == 0) return ELEMAMD_OK;
     hipStream_t s = S(stream);
-    if (uplo == 'L' && !tr)  // the Cholesky trailing update's form
+    // up to 128 rows may be in place (elemamd_gemm_f64)
+    const bool in_place = n <= 128 && blocks_overlap(C, ldc, n, n, A, lda, tr ? k : n, tr ? n : k);
+    if (uplo == 'L' && !tr && !in_place)  // the Cholesky trailing update's form
         return launch_syrk_ln_f64(n, n, k, alpha, A, lda, A, lda, beta, C, ldc, nullptr, 0, 1, s) == hipSuccess
                    ? ELEMAMD_OK
                    : ELEMAMD_ERR_HIP;
@@ -119,7 +122,7 @@ int elemamd_herk_f64(char uplo, char trans, int n, int k, double alpha, const do
         At = w;
         ldat = std::max(1, k);
     }
-    return launch_gemm_tn_f64(n, n, k, alpha, At, ldat, At, ldat, beta, C, ldc, uplo == 'L' ? 1 : 2, s) ==
+    return launch_gemm_tn_f64(n, n, k, alpha, At, ldat, At, ldat, beta, C, ldc, uplo == 'L' ? 1 : 2, s, in_place) ==
                    hipSuccess
                ? ELEMAMD_OK
                : ELEMAMD_ERR_HIP;
@@ -144,6 +147,15 @@ int elemamd_herk_f32(int mode, int n, int k, float alpha, const float* A, int64_
                        hipSuccess
                    ? ELEMAMD_OK
                    : ELEMAMD_ERR_HIP;
+    }
+    if (n <= 128 && blocks_overlap(C, ldc, n, n, A, lda, n, k)) {  // in place: from a copy
+        float* w = (float*)stream_scratch(sizeof(float) * (size_t)n * k, s);
+        if (w == nullptr) return ELEMAMD_ERR_HIP;
+        if (hipMemcpy2DAsync(w, sizeof(float) * n, A, sizeof(float) * lda, sizeof(float) * n, k,
+                             hipMemcpyDeviceToDevice, s) != hipSuccess)
+            return ELEMAMD_ERR_HIP;
+        A = w;
+        lda = n;
     }
     return launch_syrk_ln_f32(false, n, n, k, alpha, A, lda, A, lda, beta, C, ldc, nullptr, 0, 1, s) == hipSuccess
                ? ELEMAMD_OK
@@ -181,7 +193,10 @@ int elemamd_trrk_f64(char uplo, char orientA, char orientB, int n, int k, double
         Bo = (const double*)(w + one);
         ldbo = ldk;
     }
-    return launch_gemm_tn_f64(n, n, k, alpha, Ao, ldao, Bo, ldbo, beta, C, ldc, uplo == 'L' ? 1 : 2, s) ==
+    // up to 128 rows may be in place (elemamd_gemm_f64)
+    const bool in_place = n <= 128 && (blocks_overlap(C, ldc, n, n, Ao, ldao, k, n) ||
+                                       blocks_overlap(C, ldc, n, n, Bo, ldbo, k, n));
+    return launch_gemm_tn_f64(n, n, k, alpha, Ao, ldao, Bo, ldbo, beta, C, ldc, uplo == 'L' ? 1 : 2, s, in_place) ==
                    hipSuccess
                ? ELEMAMD_OK
                : ELEMAMD_ERR_HIP;
@@ -252,27 +267,33 @@ int elemamd_gemm_f64(char ta, char tb, int m, int n, int k, double alpha, const 
     const bool TA = is_trans(ta), TB = is_trans(tb);
     if (lda < std::max(1, TA ? k : m) || ldb < std::max(1, TB ? n : k) || ldc < std::max(1, m))
         return ELEMAMD_ERR_ARG;
-    // an operand that C overlaps is copied first (a product of up to 128 rows or
-    // columns may be in place)
-    if (m > 0 && n > 0 && k > 0 && (m <= 128 || n <= 128)) {
+    // A product of up to 128 rows or columns may be in place: with 128 x 128
+    // tiles a workgroup has read its operands whole before it writes, so a
+    // single tile is safe, and an operand in C's own place as long as each
+    // tile reads only its own rows (columns) of it.  Any other operand that C
+    // overlaps is copied first.
+    bool in_place = false;
+    if (m <= 128 || n <= 128) {
         const int ra = TA ? k : m, ca = TA ? m : k, rb = TB ? n : k, cb = TB ? k : n;
-        auto overlaps = [&](const double* X, int64_t ldx, int r, int c) {
-            return X < C + (n - 1) * ldc + m && C < X + (c - 1) * ldx + r;
-        };
-        const bool oa = overlaps(A, lda, ra, ca), ob = overlaps(B, ldb, rb, cb);
-        if (oa || ob) {
-            const size_t sa = al256(sizeof(double) * (size_t)ra * ca), sb = sizeof(double) * (size_t)rb * cb;
-            char* w = (char*)stream_scratch(sa + sb, S(stream));
+        const bool oa = blocks_overlap(C, ldc, m, n, A, lda, ra, ca), ob = blocks_overlap(C, ldc, m, n, B, ldb, rb, cb);
+        const bool one = m <= 128 && n <= 128;
+        const bool copy_a = oa && !one && !(n <= 128 && A == C && lda == ldc && !TA);
+        const bool copy_b = ob && !one && !(m <= 128 && B == C && ldb == ldc && !TB);
+        in_place = (oa && !copy_a) || (ob && !copy_b);
+        if (copy_a || copy_b) {
+            const size_t sa = copy_a ? al256(sizeof(double) * (size_t)ra * ca) : 0;
+            char* w = (char*)stream_scratch(sa + (copy_b ? sizeof(double) * (size_t)rb * cb : 0), S(stream));
             if (w == nullptr) return ELEMAMD_ERR_HIP;
-            if (oa && launch_copy_f64(ra, ca, A, lda, (double*)w, ra, S(stream)) != hipSuccess) return ELEMAMD_ERR_HIP;
-            if (ob && launch_copy_f64(rb, cb, B, ldb, (double*)(w + sa), rb, S(stream)) != hipSuccess)
+            if (copy_a && launch_copy_f64(ra, ca, A, lda, (double*)w, ra, S(stream)) != hipSuccess)
                 return ELEMAMD_ERR_HIP;
-            if (oa) A = (const double*)w, lda = ra;
-            if (ob) B = (const double*)(w + sa), ldb = rb;
+            if (copy_b && launch_copy_f64(rb, cb, B, ldb, (double*)(w + sa), rb, S(stream)) != hipSuccess)
+                return ELEMAMD_ERR_HIP;
+            if (copy_a) A = (const double*)w, lda = ra;
+            if (copy_b) B = (const double*)(w + sa), ldb = rb;
         }
     }
     return launch_gemm_f64(TA, TB, m, n, k, alpha, A, lda, kGemmShapeFull, B, ldb, kGemmShapeFull, beta, C, ldc, 0,
-                           nullptr, S(stream)) == hipSuccess
+                           nullptr, S(stream), in_place) == hipSuccess
                ? ELEMAMD_OK
                : ELEMAMD_ERR_HIP;
 }

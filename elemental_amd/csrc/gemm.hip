@@ -291,11 +291,11 @@ hipError_t launch_gemm_jobs_f64(const GemmJobs& jobs, const int* info, hipStream
 
 hipError_t launch_gemm_f64(bool ta, bool tb, int m, int n, int k, double alpha, const double* A, i64 lda, int ashape,
                            const double* B, i64 ldb, int bshape, double beta, double* C, i64 ldc, int tri,
-                           const int* info, hipStream_t s) {
+                           const int* info, hipStream_t s, bool in_place) {
     if (m <= 0 || n <= 0) return hipSuccess;
     if (tri != 0 && m != n) return hipErrorInvalidValue;
     const i64 Tm = ceil_div(m, kGemmTile), Tn = ceil_div(n, kGemmTile), tiles = tri != 0 ? Tm * (Tm + 1) / 2 : Tm * Tn;
-    if (tiles >= kGemmBigTiles) {
+    if (tiles >= kGemmBigTiles || in_place) {
         const dim3 grid = tri != 0 ? dim3((unsigned)tiles) : dim3((unsigned)Tm, (unsigned)Tn);
         auto kernel = ta ? (tb ? gemm_big_f64_kernel<true, true> : gemm_big_f64_kernel<true, false>)
                          : (tb ? gemm_big_f64_kernel<false, true> : gemm_big_f64_kernel<false, false>);
@@ -309,9 +309,9 @@ hipError_t launch_gemm_f64(bool ta, bool tb, int m, int n, int k, double alpha, 
 }
 
 hipError_t launch_gemm_tn_f64(int m, int n, int k, double alpha, const double* A, i64 lda, const double* B, i64 ldb,
-                              double beta, double* C, i64 ldc, int tri, hipStream_t s) {
+                              double beta, double* C, i64 ldc, int tri, hipStream_t s, bool in_place) {
     return launch_gemm_f64(true, false, m, n, k, alpha, A, lda, kGemmShapeFull, B, ldb, kGemmShapeFull, beta, C, ldc,
-                           tri, nullptr, s);
+                           tri, nullptr, s, in_place);
 }
 
 }  // namespace elemamd

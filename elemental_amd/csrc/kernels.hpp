@@ -85,7 +85,8 @@ hipError_t launch_syrk_diag_bf16_planes(int np, int ncol, int k, const unsigned 
 // tri: 0 all of C; 1 its lower triangle; 2 its upper triangle (1, 2: m == n).
 // Operand shapes mask the stored matrix: outside the triangle reads as zero,
 // a unit diagonal as one.  info (may be null): the launch does nothing when
-// *info != 0.  beta == 0: C is not read.
+// *info != 0.  beta == 0: C is not read.  in_place: 128 x 128 tiles, whose
+// workgroups have read their operands whole before they write.
 enum : int {
     kGemmShapeFull = 0,
     kGemmShapeLower = 1,
@@ -110,10 +111,10 @@ struct GemmJobs {
 hipError_t launch_gemm_jobs_f64(const GemmJobs& jobs, const int* info, hipStream_t s);
 hipError_t launch_gemm_f64(bool ta, bool tb, int m, int n, int k, double alpha, const double* A, i64 lda, int ashape,
                            const double* B, i64 ldb, int bshape, double beta, double* C, i64 ldc, int tri,
-                           const int* info, hipStream_t s);
+                           const int* info, hipStream_t s, bool in_place = false);
 // the TN form without masks (Trrk)
 hipError_t launch_gemm_tn_f64(int m, int n, int k, double alpha, const double* A, i64 lda, const double* B, i64 ldb,
-                              double beta, double* C, i64 ldc, int tri, hipStream_t s);
+                              double beta, double* C, i64 ldc, int tri, hipStream_t s, bool in_place = false);
 
 // inverse.hip -- n x n (n <= 128) blocks by one workgroup, bit-identical to
 // the reference's unblocked loops in IEEE double (no contraction).
