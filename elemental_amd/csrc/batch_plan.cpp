@@ -39,11 +39,12 @@ BatchArgs plan_args(const BatchPlan* P, bool with_skip) { return plan_args(P, 0,
 // The runs and their steps' work prefix sums, from the buckets and their
 // launch forms.  Buckets with the same block size share their steps' launches
 // (each of which lasts as long as its largest matrix's chain): 1024 matrices
-// of n = 16 ... 1024 in six buckets take 10 block steps instead of 17.
+// of n = 16 ... 1024 in six buckets take 10 block steps instead of 17.  On
+// failure the plan keeps the runs and the table that it has.
 int plan_runs(BatchPlan* P) {
-    P->runs.clear();
+    std::vector<BatchRun> runs;
     for (const BatchBucket& bk : P->buckets) {
-        BatchRun* last = P->runs.empty() ? nullptr : &P->runs.back();
+        BatchRun* last = runs.empty() ? nullptr : &runs.back();
         if (last != nullptr && bk.grid == 0 && last->grid == 0 && last->nb == bk.nb) {
             last->count += bk.count;
             continue;
@@ -53,12 +54,12 @@ int plan_runs(BatchPlan* P) {
         r.grid = bk.grid;
         r.first = bk.first;
         r.count = bk.count;
-        P->runs.push_back(r);
+        runs.push_back(r);
     }
     const int tile = P->precision == 2 ? 128 : 64;  // of the trailing update
     std::vector<int> prefix;
     auto size = [&](int p) { return P->n[P->order[p]]; };
-    for (BatchRun& r : P->runs) {
+    for (BatchRun& r : runs) {
         if (r.grid > 0) continue;
         const int nb = r.nb, steps = (size(r.first) + nb - 1) / nb;
         for (int j = 0; j < steps; ++j) {
@@ -83,12 +84,19 @@ int plan_runs(BatchPlan* P) {
     }
     std::vector<int> pr(P->count + 1, 0);
     for (int q = 0; q < P->count; ++q) pr[q + 1] = pr[q] + (size(q) + 63) / 64;
-    P->res_wgs = pr[P->count];
-    P->res_prefix_off = (int)prefix.size();
+    const int res_off = (int)prefix.size();
     prefix.insert(prefix.end(), pr.begin(), pr.end());
-    if (P->d_prefix != nullptr) (void)hipFree(P->d_prefix);
-    P->d_prefix = nullptr;
-    return upload(&P->d_prefix, prefix) == hipSuccess ? kOk : kErrHip;
+    int* table = nullptr;
+    if (upload(&table, prefix) != hipSuccess) {
+        if (table != nullptr) (void)hipFree(table);
+        return kErrHip;
+    }
+    if (P->d_prefix != nullptr) (void)hipFree(P->d_prefix);  // (waits for work that still reads it)
+    P->d_prefix = table;
+    P->runs.swap(runs);
+    P->res_wgs = pr[P->count];
+    P->res_prefix_off = res_off;
+    return kOk;
 }
 
 }  // namespace
@@ -203,17 +211,23 @@ int batch_set_launch(BatchPlan* P, const int* bucket_grid) {
     if (P == nullptr || bucket_grid == nullptr) return kErrArg;
     for (const BatchBucket& bk : P->buckets)
         if (bucket_grid[bk.index] < 0 || (bucket_grid[bk.index] > 0 && bk.nb > kPersistMaxNb)) return kErrArg;
+    const std::vector<BatchBucket> before = P->buckets;
     bool same = true;
     for (BatchBucket& bk : P->buckets) {
         same = same && bk.grid == bucket_grid[bk.index];
         bk.grid = bucket_grid[bk.index];
     }
     if (same) return kOk;
-    if (P->graph_exec) {  // captured with the previous launch forms
+    const int rc = plan_runs(P);
+    if (rc != kOk) {
+        P->buckets = before;
+        return rc;
+    }
+    if (P->graph_exec) {  // captured with the previous launch forms and table
         (void)hipGraphExecDestroy(P->graph_exec);
         P->graph_exec = nullptr;
     }
-    return plan_runs(P);
+    return kOk;
 }
 
 size_t batch_workspace_bytes(const BatchPlan* P) {
