@@ -128,10 +128,12 @@ __device__ __noinline__ void persist_factor_block(int b, T* L, int n, int* info,
     diag16::factor_block<T, false, 4>(*reinterpret_cast<diag16::Lds<false>*>(arena), b, L, n, nullptr, info, c0);
 }
 
-template <typename T>
+// (NT: eight tiles spill, 64 columns do with four: 1024 matrices of n = 16 ...
+// 1024 in blocks of 64, FP64: 7.3 ms, 11.0 with eight)
+template <typename T, int NT>
 __device__ __noinline__ void persist_panel(int m, int b, T* L, int n, char* arena) {
     for (int rb = 0; rb < (m + 63) / 64; ++rb) {
-        panel16::slab<T>(*reinterpret_cast<panel16::Lds*>(arena), m, b, L, n, L + b, n, L + b, n, rb);
+        panel16::slab<T, unsigned, false, NT>(*reinterpret_cast<panel16::Lds*>(arena), m, b, L, n, L + b, n, L + b, n, rb);
         __syncthreads();
     }
 }
@@ -186,7 +188,8 @@ __global__ __launch_bounds__(256, 2) void batch_persistent_kernel(BatchArgs a, T
             if (*info != 0) break;
             const int m = n - c0 - b;
             if (m <= 0) break;
-            persist_panel<T>(m, b, L, n, arena);
+            if (b <= 64) persist_panel<T, panel16::kTiles / 2>(m, b, L, n, arena);
+            else persist_panel<T, panel16::kTiles>(m, b, L, n, arena);
             persist_trailing<T, MODE>(m, b, L + b, M + (c0 + b) + (i64)(c0 + b) * n, n, arena);
         }
     }

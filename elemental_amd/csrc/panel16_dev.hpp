@@ -9,7 +9,7 @@
 namespace elemamd {
 namespace panel16 {
 
-constexpr int kTiles = 8;  // 16-column tiles of a panel of up to 128 columns
+constexpr int kTiles = 8;  // 16-column tiles of a panel of up to 128 columns (kTiles / 2: of up to 64)
 
 struct Lds {
     double M[kTiles][16][16];  // [tile][k][c]: multipliers l_ck / l_kk (k < c, else 0); [15]: 1 / l_cc
@@ -29,8 +29,8 @@ struct TileColumn {
 // Rows [64 slab, 64 slab + 64) of X := B L^{-T} (m x b, b <= 128; X may be B)
 // by the calling 256-thread workgroup, storage T (double, or float computed in
 // double).  Off: what holds the offset of three columns in bytes.  IDENT: B
-// is the identity.
-template <typename T, typename Off = unsigned, bool IDENT = false>
+// is the identity.  NT: tiles (b <= 16 NT).
+template <typename T, typename Off = unsigned, bool IDENT = false, int NT = kTiles>
 __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict__ L, i64 ldl, const T* B, i64 ldb, T* X,
                                      i64 ldx, int slab) {
     const int t = threadIdx.x, lane = t & 63, c = lane & 15, g = lane >> 4;
@@ -43,9 +43,9 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
     // the next (a wave alone on its SIMD pays 4 to 8 cycles for every scalar
     // or vector instruction: with a product and clamps per load, loading took
     // 14000 of 36000 cycles).
-    const bool full = b == 16 * kTiles;
-    // row c of the diagonal tile w (lanes with g < 2) or w + 4
-    const int d0 = 16 * (w + 4 * (g >> 1)), dr = min(d0 + c, b - 1);
+    const bool full = b == 16 * NT;
+    // row c of the diagonal tile w or, of eight and for lanes with g > 1, w + 4
+    const int dt = NT > 4 ? w + 4 * (g >> 1) : w, d0 = 16 * dt, dr = min(d0 + c, b - 1);
     double lm[15];
     {
         T raw[15];
@@ -72,22 +72,22 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
     // turned through LDS into lane (c, g): rows g + 4 v of column c.
     const T* Bw = B + min(rw, m - 1);
     const Off rowc = (Off)min(c, max(m - 1 - rw, 0));
-    T raw[kTiles][4];
+    T raw[NT][4];
     if constexpr (IDENT) {
 #pragma unroll
-        for (int q = 0; q < kTiles; ++q)
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) raw[q][v] = rw + c == 16 * q + g + 4 * v ? T(1) : T(0);
     } else if (full) {
         const T* p = Bw;
         const Off off = (Off)g * (Off)ldb + rowc;
 #pragma unroll
-        for (int q = 0; q < kTiles; ++q)
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v, p += 4 * ldb) raw[q][v] = at(p, off);
     } else {
 #pragma unroll
-        for (int q = 0; q < kTiles; ++q)
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 // (a partial tile's last column again in the place of missing ones)
@@ -98,31 +98,31 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
     // operands of the update of tile p by tile q: L(16 p + c, 16 q + 4 ks + g)
     // (a tile that updates others is full)
     const i64 ls = b >= 16 ? ldl : 0;
-    Off rowp[kTiles - 1];
+    Off rowp[NT - 1];
 #pragma unroll
-    for (int p = 1; p < kTiles; ++p) rowp[p - 1] = (Off)g * (Off)ls + (Off)min(16 * p + c, b - 1);
-    double y[kTiles - 1][4];
+    for (int p = 1; p < NT; ++p) rowp[p - 1] = (Off)g * (Off)ls + (Off)min(16 * p + c, b - 1);
+    double y[NT - 1][4];
     auto load_y = [&](int p, int q) __attribute__((always_inline)) {
         const T* Lq = L + (i64)(16 * q + 16 <= b ? 16 * q : 0) * ls;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) y[p - 1][ks] = (double)at(Lq + 4 * ks * ls, rowp[p - 1]);
     };
 #pragma unroll
-    for (int p = 1; p < kTiles; ++p) load_y(p, 0);
+    for (int p = 1; p < NT; ++p) load_y(p, 0);
     {
         const double r = 1.0 / dd;
         chain::Multipliers<double, 0>::run(lm, r, c);
-        if ((g & 1) == 0) {
-            double(*M)[16] = sh.M[w + 4 * (g >> 1)];
+        if (NT > 4 ? (g & 1) == 0 : g == 0) {
+            double(*M)[16] = sh.M[dt];
 #pragma unroll
             for (int k = 0; k < 15; ++k) M[k][c] = lm[k];
             M[15][c] = r;
         }
     }
-    d4_t a[kTiles];
+    d4_t a[NT];
     double(*sx)[16] = sh.X[w];  // (LDS serves a wave's accesses in order; the barriers keep the compiler's)
 #pragma unroll
-    for (int q = 0; q < kTiles; ++q) {
+    for (int q = 0; q < NT; ++q) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) sx[c][(g + 4 * v) ^ c] = (double)raw[q][v];
         __builtin_amdgcn_wave_barrier();
@@ -132,7 +132,7 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < kTiles; ++q) {
+    for (int q = 0; q < NT; ++q) {
         if (q >= np) break;
         double mk[15], x[4] = {a[q][0], a[q][1], a[q][2], a[q][3]};
 #pragma unroll
@@ -160,7 +160,7 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
             asm volatile("" : "+v"(fa[ks]));  // (made once)
         }
 #pragma unroll
-        for (int p = q + 1; p < kTiles; ++p) {
+        for (int p = q + 1; p < NT; ++p) {
             if (p < np) mfma_tile(a[p], fa, y[p - 1]);
             if (p > q + 1) load_y(p, q + 1);
         }
@@ -170,12 +170,12 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
         T* p = X + rw;
         const Off off = (Off)g * (Off)ldx + (Off)c;
 #pragma unroll
-        for (int q = 0; q < kTiles; ++q)
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v, p += 4 * ldx) *(T*)((char*)p + off * (Off)sizeof(T)) = raw[q][v];
     } else {
 #pragma unroll
-        for (int q = 0; q < kTiles; ++q)
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int r = rw + c, col = 16 * q + g + 4 * v;
