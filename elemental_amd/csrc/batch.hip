@@ -188,8 +188,13 @@ __global__ __launch_bounds__(256, 2) void batch_persistent_kernel(BatchArgs a, T
             if (*info != 0) break;
             const int m = n - c0 - b;
             if (m <= 0) break;
-            if (b <= 64) persist_panel<T, panel16::kTiles / 2>(m, b, L, n, arena);
-            else persist_panel<T, panel16::kTiles>(m, b, L, n, arena);
+            if (b <= 64) {
+                persist_panel<T, panel16::kTiles / 2>(m, b, L, n, arena);
+            } else {
+                int width = b;  // (opaque: FP32 lost 7 % at 128 columns with the range known inside)
+                asm volatile("" : "+s"(width));
+                persist_panel<T, panel16::kTiles>(m, width, L, n, arena);
+            }
             persist_trailing<T, MODE>(m, b, L + b, M + (c0 + b) + (i64)(c0 + b) * n, n, arena);
         }
     }

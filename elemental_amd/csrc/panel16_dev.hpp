@@ -45,7 +45,7 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
     // 14000 of 36000 cycles).
     const bool full = b == 16 * NT;
     // row c of the diagonal tile w or, of eight and for lanes with g > 1, w + 4
-    const int dt = NT > 4 ? w + 4 * (g >> 1) : w, d0 = 16 * dt, dr = min(d0 + c, b - 1);
+    const int d0 = 16 * (NT > 4 ? w + 4 * (g >> 1) : w), dr = min(d0 + c, b - 1);
     double lm[15];
     {
         T raw[15];
@@ -113,7 +113,7 @@ __device__ __forceinline__ void slab(Lds& sh, int m, int b, const T* __restrict_
         const double r = 1.0 / dd;
         chain::Multipliers<double, 0>::run(lm, r, c);
         if (NT > 4 ? (g & 1) == 0 : g == 0) {
-            double(*M)[16] = sh.M[dt];
+            double(*M)[16] = sh.M[NT > 4 ? w + 4 * (g >> 1) : w];
 #pragma unroll
             for (int k = 0; k < 15; ++k) M[k][c] = lm[k];
             M[15][c] = r;
