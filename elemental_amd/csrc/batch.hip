@@ -48,7 +48,7 @@ __global__ __launch_bounds__(diag16::kThreads, 4) void batch_potrf_kernel(BatchA
     if (c0 >= n) return;
     if (a.skip != nullptr && a.skip[p]) return;
     const int* info = a.info + p;
-    if (*info != 0 && *info <= c0) return;  // an earlier block failed: this one was not updated
+    if (step > 0 && *info != 0 && *info <= c0) return;  // an earlier block failed: this one was not updated
     const int b = min(nb, n - c0);
     diag16::factor_block<T, false>(sh, b, A + a.a_off[p] + c0 + (i64)c0 * n, n, nullptr, a.info + p, c0);
 }

@@ -104,6 +104,18 @@ constexpr int kNormal = 0x108, kInfinite = 0x204, kNotFinite = 0x207;
 __device__ __forceinline__ bool is_class(double x, int c) { return __builtin_amdgcn_class(x, c); }
 __device__ __forceinline__ bool is_class(float x, int c) { return __builtin_amdgcn_classf(x, c); }
 
+// Whether all of m are normal numbers, from the exponents alone.
+__device__ __forceinline__ unsigned magnitude(double x) { return (unsigned)__double2hiint(x) & 0x7fffffffu; }
+__device__ __forceinline__ unsigned magnitude(float x) { return (unsigned)__float_as_int(x) & 0x7fffffffu; }
+template <typename T>
+__device__ __forceinline__ bool all_normal(const T (&m)[15]) {
+    constexpr unsigned least = sizeof(T) == 8 ? 0x00100000u : 0x00800000u, inf = sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u;
+    unsigned lo = magnitude(m[0]), hi = lo;
+#pragma unroll
+    for (int k = 1; k < 15; ++k) lo = min(lo, magnitude(m[k])), hi = max(hi, magnitude(m[k]));
+    return (lo >= least) & (hi < inf);
+}
+
 // The tile's multipliers: m[k] := l_ck / l_kk for k < c, else 0 (lane c of
 // every 16-lane row holds row c's coefficients in m; r its reciprocal
 // diagonal).
@@ -130,14 +142,18 @@ struct Multipliers {
         m[K] = K < c ? m[K] * rk : T(0);
         if constexpr (K < 14) Multipliers<T, K + 1>::run(m, r, c);
     }
-    // the same from the coefficients l; true where a multiplier lost its value
-    // (with l_kk = 0 an infinite one has not)
-    static __device__ __forceinline__ bool checked(T (&m)[15], const T (&l)[15], T r, int c) {
+    // m := l_ck / l_kk without the mask
+    static __device__ __forceinline__ void products(T (&m)[15], const T (&l)[15], T r) {
+        m[K] = l[K] * row_lane<K>(r);
+        if constexpr (K < 14) Multipliers<T, K + 1>::products(m, l, r);
+    }
+    // whether one of row c's multipliers has lost its value (with l_kk = 0 an
+    // infinite one has not)
+    static __device__ __forceinline__ bool lost(const T (&m)[15], const T (&l)[15], T r, int c) {
         const T rk = row_lane<K>(r);
-        m[K] = K < c ? l[K] * rk : T(0);
-        const bool lost = (K < c) & (l[K] != T(0)) & !is_class(m[K], kNormal) & !is_class(rk, kInfinite);
-        if constexpr (K < 14) return lost | Multipliers<T, K + 1>::checked(m, l, r, c);
-        return lost;
+        const bool x = (K < c) & (l[K] != T(0)) & !is_class(m[K], kNormal) & !is_class(rk, kInfinite);
+        if constexpr (K < 14) return x | Multipliers<T, K + 1>::lost(m, l, r, c);
+        return x;
     }
 };
 
@@ -237,12 +253,20 @@ __device__ __forceinline__ void fetch_blocks(S& sh, const Rows<T, TRANS, CONTIG>
         // multipliers l_ck / l_kk of the tile's earlier columns
         const T r = in && !unit ? T(1) / dd : T(1);
         const int c16 = in ? lane & 15 : 0;
-        const bool lost = Multipliers<T, 0>::checked(m, l, r, c16) | (r != r);
-        // the whole tile takes the coefficients then
-        const bool careful = (__ballot(lost) >> (lane & 48) & 0xffff) != 0;
-        if (careful)
+        Multipliers<T, 0>::products(m, l, r);
+        // (a first look at all exponents, in two instructions a multiplier;
+        // tiles with a zero take the second look)
+        bool careful = false;
+        if (__ballot(!all_normal(m)) != 0) {
+            const bool lost = Multipliers<T, 0>::lost(m, l, r, c16) | (r != r);
+            // the whole tile takes the coefficients then
+            careful = (__ballot(lost) >> (lane & 48) & 0xffff) != 0;
+            if (careful)
 #pragma unroll
-            for (int k = 0; k < 15; ++k) m[k] = k < c16 ? l[k] : T(0);
+                for (int k = 0; k < 15; ++k) m[k] = l[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 15; ++k) m[k] = k < c16 ? m[k] : T(0);
         less(pos, ic, b);
         await(&sh.seq, 4 * (pos - RB + 1), limit, &sh.err);  // the slot's last block is solved
 #pragma unroll
@@ -297,7 +321,9 @@ __device__ __forceinline__ void hand_over(S& sh, int pos, int w, int lane, const
 // the chain comes here when a result is not finite, which the NaN of a tile
 // kept as coefficients sees to.  The rows pass through their places in sh.Y.
 // n = 4096, 16 columns, forward: 253 us, 1130 with every tile solved here; the
-// test alone costs 0.6 % (n = 8192, both solves: 1007 and 1013 us).
+// tests alone cost little (n = 8192, both solves: 1011 us with and without
+// them; n = 4100, forward, 285 and 289; 20000 matrices of n = 8 ... 16, FP64,
+// 0.97 and 1.01 ms).
 template <int NV, typename S, typename A>
 __device__ __forceinline__ void solve_tile_careful(S& sh, int pos, int w, int lane, bool in, const A& acc) {
     typedef typename S::value T;
