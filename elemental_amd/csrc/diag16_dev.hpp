@@ -253,7 +253,7 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
     const int np = (b + 15) / 16;
     const bool full = b == 16 * kWaves;
     if (tid == 0) sh.bad = 0;
-    __syncthreads();
+    if (np > 1) __syncthreads();  // (before another wave sets it)
     // tile row w, tiles 0 .. w (zero past b, the padded diagonal one; the
     // diagonal tile whole, mirrored).  16 rows by 4 columns per load, whole
     // lines (with lanes along columns every lane is an access of its own, 64
@@ -317,13 +317,15 @@ __device__ __forceinline__ void factor_block(Lds<INV>& sh, int b, T* __restrict_
                     if (i >= b || j >= b) t[r][J][v] = i == j ? 1.0 : 0.0;
                 }
     bool odd = false;
+    if (np > 1) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r)
+        for (int r = 0; r < NR; ++r)
 #pragma unroll
-        for (int J = 0; J < NW * (r + 1) - 1; ++J)
-            if (J < w0 + NW * r)
+            for (int J = 0; J < NW * (r + 1) - 1; ++J)
+                if (J < w0 + NW * r)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) odd = odd | __builtin_amdgcn_class(t[r][J][v], 0x207);
+                    for (int v = 0; v < 4; ++v) odd = odd | __builtin_amdgcn_class(t[r][J][v], 0x207);
+    }
     if (__ballot(odd) != 0 && lane == 0) atomicOr(&sh.bad, 2);
     if (w0 == 0) {
 #pragma unroll

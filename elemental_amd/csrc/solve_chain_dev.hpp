@@ -104,16 +104,18 @@ constexpr int kNormal = 0x108, kInfinite = 0x204, kNotFinite = 0x207;
 __device__ __forceinline__ bool is_class(double x, int c) { return __builtin_amdgcn_class(x, c); }
 __device__ __forceinline__ bool is_class(float x, int c) { return __builtin_amdgcn_classf(x, c); }
 
-// Whether all of m are normal numbers, from the exponents alone.
-__device__ __forceinline__ unsigned magnitude(double x) { return (unsigned)__double2hiint(x) & 0x7fffffffu; }
-__device__ __forceinline__ unsigned magnitude(float x) { return (unsigned)__float_as_int(x) & 0x7fffffffu; }
+// Whether all of m are normal numbers, from their leading bits x: 2 x less the
+// least normal number's is below the bound for these alone (zeros and
+// subnormal numbers wrap around to the top, where infinities and NaN are).
+__device__ __forceinline__ unsigned leading_bits(double x) { return (unsigned)__double2hiint(x); }
+__device__ __forceinline__ unsigned leading_bits(float x) { return (unsigned)__float_as_int(x); }
 template <typename T>
 __device__ __forceinline__ bool all_normal(const T (&m)[15]) {
-    constexpr unsigned least = sizeof(T) == 8 ? 0x00100000u : 0x00800000u, inf = sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u;
-    unsigned lo = magnitude(m[0]), hi = lo;
+    constexpr unsigned least = sizeof(T) == 8 ? 0x00200000u : 0x01000000u, bound = 0u - 2 * least;
+    unsigned worst = 0;
 #pragma unroll
-    for (int k = 1; k < 15; ++k) lo = min(lo, magnitude(m[k])), hi = max(hi, magnitude(m[k]));
-    return (lo >= least) & (hi < inf);
+    for (int k = 0; k < 15; ++k) worst = max(worst, (leading_bits(m[k]) << 1) - least);
+    return worst < bound;
 }
 
 // The tile's multipliers: m[k] := l_ck / l_kk for k < c, else 0 (lane c of
@@ -146,14 +148,6 @@ struct Multipliers {
     static __device__ __forceinline__ void products(T (&m)[15], const T (&l)[15], T r) {
         m[K] = l[K] * row_lane<K>(r);
         if constexpr (K < 14) Multipliers<T, K + 1>::products(m, l, r);
-    }
-    // whether one of row c's multipliers has lost its value (with l_kk = 0 an
-    // infinite one has not)
-    static __device__ __forceinline__ bool lost(const T (&m)[15], const T (&l)[15], T r, int c) {
-        const T rk = row_lane<K>(r);
-        const bool x = (K < c) & (l[K] != T(0)) & !is_class(m[K], kNormal) & !is_class(rk, kInfinite);
-        if constexpr (K < 14) return x | Multipliers<T, K + 1>::lost(m, l, r, c);
-        return x;
     }
 };
 
@@ -254,11 +248,17 @@ __device__ __forceinline__ void fetch_blocks(S& sh, const Rows<T, TRANS, CONTIG>
         const T r = in && !unit ? T(1) / dd : T(1);
         const int c16 = in ? lane & 15 : 0;
         Multipliers<T, 0>::products(m, l, r);
-        // (a first look at all exponents, in two instructions a multiplier;
-        // tiles with a zero take the second look)
+        // (a first look at all exponents; tiles with a zero take the second)
         bool careful = false;
         if (__ballot(!all_normal(m)) != 0) {
-            const bool lost = Multipliers<T, 0>::lost(m, l, r, c16) | (r != r);
+            // a multiplier that is not a normal number, of a coefficient other
+            // than zero, has lost its value; an infinite one with l_kk = 0 has not
+            bool lost = r != r;
+#pragma unroll 1
+            for (int k = 0; k < 15; ++k) {
+                const T lk = L.L[ic * L.rs + lesser(t0 + k, ic) * L.cs], rk = __shfl(r, (lane & 48) + k);
+                lost = lost | ((k < c16) & (lk != T(0)) & !is_class(lk * rk, kNormal) & !is_class(rk, kInfinite));
+            }
             // the whole tile takes the coefficients then
             careful = (__ballot(lost) >> (lane & 48) & 0xffff) != 0;
             if (careful)
@@ -321,9 +321,8 @@ __device__ __forceinline__ void hand_over(S& sh, int pos, int w, int lane, const
 // the chain comes here when a result is not finite, which the NaN of a tile
 // kept as coefficients sees to.  The rows pass through their places in sh.Y.
 // n = 4096, 16 columns, forward: 253 us, 1130 with every tile solved here; the
-// tests alone cost little (n = 8192, both solves: 1011 us with and without
-// them; n = 4100, forward, 285 and 289; 20000 matrices of n = 8 ... 16, FP64,
-// 0.97 and 1.01 ms).
+// tests alone cost little (n = 8192, both solves: 1008 us with and without
+// them; 20000 matrices of n = 8 ... 16, FP64, 0.97 and 1.00 ms).
 template <int NV, typename S, typename A>
 __device__ __forceinline__ void solve_tile_careful(S& sh, int pos, int w, int lane, bool in, const A& acc) {
     typedef typename S::value T;
