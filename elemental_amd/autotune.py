@@ -3,7 +3,7 @@
 For each size bucket it times the captured batch on a sample of matrices
 drawn log-uniformly inside the bucket, once per candidate shape -- the block
 size nb (the diagonal-block / panel width and the depth of the trailing
-update's 128 x 128 tiles) and the launch form: one potrf, panel and trailing
+update) and the launch form: one potrf, panel and trailing
 launch per block step, or one persistent launch of 256, 512 or 1024
 workgroups that each take whole matrices -- and keeps the
 fastest.  The result is cached as JSON (``batch.TUNING_FILE``), keyed by

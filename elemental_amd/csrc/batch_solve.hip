@@ -12,7 +12,7 @@
 // fill the CUs that the large ones leave.
 // Measured (1024 matrices, n = 16 ... 1024, up to 8 columns): 2.73 ms in six
 // launches of a kernel that staged every block between two barriers and
-// substituted 64 rows by wave broadcasts, 0.38 ms now; FP32 (four sweeps)
+// substituted 64 rows by wave broadcasts, 0.39 ms now; FP32 (four sweeps)
 // 6.81 and 0.66 ms.
 #include <algorithm>
 

@@ -368,8 +368,8 @@ int elemamd_hermitian_gen_definite_eig_f64(int type, char uplo, int n, double* A
 // ------------------------------------------------------- Matrix<float>
 // Cholesky / SolveAfter / HPDSolve with F = float: the float factorization
 // (FP64 diagonal blocks, FP32 panels by products with the diagonal pieces'
-// inverses, FP32 MFMA trailing updates) and float solves with the 64 x 64
-// diagonal-block inverses.
+// inverses, FP32 MFMA trailing updates) and float solves that substitute in
+// 16-row tiles.
 int elemamd_cholesky_f32(char uplo, int n, float* A, int64_t lda, int nb, int* dinfo, void* stream) {
     uplo = up(uplo);
     if (uplo != 'L' && uplo != 'U') return ELEMAMD_ERR_ARG;

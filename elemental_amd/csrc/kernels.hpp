@@ -34,9 +34,9 @@ hipError_t launch_panel_inverse_f64(int m, int b, const double* L, i64 ldl, cons
                                     double* R, i64 ldr, const int* info, hipStream_t s);
 
 // potrf_f32.hip -- panel step of the float-storage factor: the b x b
-// (b <= 128) diagonal block factored in place (FP64 on 32 x 32 pieces, whose
-// inverses go to Xd, 4 x 32 x 32 floats), and B (m x b) := B L^{-T} with the
-// factored block L and those inverses; planes (may be null): the result's np
+// (b <= 128) diagonal block factored in place (FP64 in 16-column pieces; the
+// inverses of its 32 x 32 pieces go to Xd, 4 x 32 x 32 floats), and B (m x b)
+// := B L^{-T} with the factored block L and those inverses; planes (may be null): the result's np
 // bf16 planes (launch_split_bf16's form) are also written, row r of B to
 // planes + p*ps + r*ldk (columns 0..b-1).  upd (may be null): B first takes
 // B -= P_B P_top^T over uk columns of the same np planes, P_top = upd rows

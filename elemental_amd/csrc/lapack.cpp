@@ -92,8 +92,8 @@ int cholesky_lower(int n, T* A, i64 lda, int nb, int trailing, int* dinfo, hipSt
     if (n == 0) return kOk;
     StreamPair* sp = stream_pair(s);
     if (sp == nullptr) return kErrHip;
-    // columns of the group that starts at column c (the float factor's groups
-    // are all of one width: its planes are laid out for it)
+    // columns of the group that starts at column c (with bf16 planes all groups
+    // are of one width: the planes are laid out for it)
     auto width = [&](int c) {
         const int G = std::max(1, update_depth<T>(trailing, n - c) / nb);
         return (int)std::min<i64>((i64)G * nb, n - c);

@@ -18,8 +18,9 @@ enum : int { kRefineIR = 0, kRefineCG = 1 };
 // the block size nb is used: max(1, depth / nb) panels).
 // FP64: 768 while more than 8192 columns are left (the trailing update sets
 // the pace), 256 below (the chain sets the pace, and a deeper group has more
-// of it); n = 16384 solve: 33.6 ms with 512, 33.1 with 768, 33.4 with 1024, 33.4
-// with 512 down to 4096 columns.  Where a pass is one launch on the caller's
+// of it); solves with 512 and 768, measured in turn: n = 8500 8.05 and 7.98 ms,
+// 10000 and 12000 the same (10.8, 16.0), 14000 23.1 and 22.9, 16384 33.9 and
+// 33.6.  Where a pass is one launch on the caller's
 // stream a group's inner updates cost more than the passes they save: 128 for
 // FP64 (n = 2048: 1098 us with 256, 1081; n = 3001: 1734, 1720) and, from 1024
 // columns on, for float (n = 4000: 2039 us with 512, 2011; from 2048 on 2000,

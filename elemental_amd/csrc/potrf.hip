@@ -40,7 +40,7 @@ hipError_t launch_potrf_unb(int n, T* A, i64 lda, int* info, int col_offset, hip
 }
 
 // The diagonal block of a blocked FP64 factorization (diag16_dev.hpp): same
-// result as LVar3Unb up to rounding order.  n = 128: 22.7 us alone and 45 us
+// result as LVar3Unb up to rounding order.  n = 128: 22.6 us alone and 51 us
 // beside the trailing update at n = 16384, against 78 and 128 us of
 // potrf_unb_kernel, which stays where the reference's rounding order is kept
 // bit for bit (a single block, n <= nb).

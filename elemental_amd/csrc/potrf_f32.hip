@@ -47,7 +47,7 @@ __device__ inline void tile_ab_t(f4_t (&acc)[2], const float (*P)[LP], int pr, i
 // One b x b (b <= 128) diagonal block at A (float storage): L11 overwrites
 // its lower triangle, the inverses of its four 32 x 32 diagonal pieces go to
 // Xd (4 x 32 x 32 floats, row-major).  A failing pivot records
-// col_offset + column in *info.  b = 128: 24.7 us alone, 35 us beside the
+// col_offset + column in *info.  b = 128: 25.0 us alone, 36 us beside the
 // trailing update at n = 16384; the form before it (the block as float in
 // LDS, 32-column pieces through LDS, 94 KB) took 56 and 70 us.
 __global__ __launch_bounds__(diag16::kThreads, 4) void potrf_f32_kernel(int b, float* __restrict__ A, i64 lda,

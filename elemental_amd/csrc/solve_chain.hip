@@ -40,11 +40,12 @@
 //   sum_{q <= pos - D - 1} M(pos, q) Y_q as the chain publishes those blocks
 //   and hands the partial sum to the chain: waves 0-3 the products (16 rows
 //   each), waves 8 and 9 bring the blocks into LDS, in turn.
-// Measured (FP64, n = 8192, 16 columns): 3.3 us per 64-row block forward, 3.9
+// Measured (FP64, n = 8192, 16 columns): 3.6 us per 64-row block forward, 4.0
 // backward (there every lane of an operand load reads another row, 64 cycles a
-// load, and the block's 120 loads of eight waves set the pace); a chain paced
-// by workgroup barriers with one load phase per block was 20.7 us (6.2 and 7.5
-// with products by inverted diagonal blocks in the substitutions' place).
+// load, and the block's 120 loads of eight waves set the pace); 3.4 and 4.0
+// with 8 columns.  A chain paced by workgroup barriers with one load phase per
+// block was 20.7 us (6.2 and 7.5 with products by inverted diagonal blocks in
+// the substitutions' place).
 // Both solves with an n = 8192 factor: 5.43 ms before, 1.00 ms now; the same
 // chain with conditional loads, whose waits the compiler cannot count: 1.35.
 // Cross-workgroup data (solved blocks, partial sums, flags) moves only

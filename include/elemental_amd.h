@@ -16,8 +16,8 @@
  *     whose pivot was <= 0 -- the column at which the reference's
  *     cholesky::LVar3Unb throws std::logic_error("A was not numerically HPD")
  *     (include/elemental/lapack-like/Cholesky/LVar3.hpp:37-38).  Work after a
- *     failing block is skipped, so A is left as the reference leaves it.  As
- *     in the reference, a NaN pivot is not detected.
+ *     failing block is skipped, so A is left as the reference leaves it.  A
+ *     NaN pivot, which the reference lets pass, is reported in the same way.
  *   - Character arguments follow the Fortran BLAS conventions the reference
  *     forwards to (src/core/imports/blas.cpp): uplo 'L'/'U', trans 'N'/'T'/'C'
  *     ('C' == 'T' for real data), side 'L'/'R', diag 'N'/'U'.
@@ -292,11 +292,12 @@ int elemamd_batch_plan_create(int count, const int *n, const int *k, int precisi
 int elemamd_batch_plan_destroy(elemamd_batch_plan *plan);
 /* Launch form of each size bucket (the create call's bucket order):
  * bucket_grid[b] = 0 runs bucket b as one potrf, one panel and one trailing
- * launch per block step (the default); g > 0 runs its whole factorization,
- * and for ELEMAMD_BATCH_F64 its solves, as ONE persistent launch of g
- * workgroups that take the bucket's matrices largest first.  Results are
- * the same bit for bit.  No reference counterpart
- * (for callers factoring many small matrices). */
+ * launch per block step (the default); g > 0 runs its whole factorization as
+ * ONE persistent launch of g workgroups that take the bucket's matrices
+ * largest first.  The solves of all buckets share their launches in either
+ * form.  Results are the same bit for bit, and so is what a matrix that is
+ * not HPD leaves behind.  On an error the plan keeps its launch forms.  No
+ * reference counterpart (for callers factoring many small matrices). */
 int elemamd_batch_set_launch(elemamd_batch_plan *plan, const int *bucket_grid);
 /* Element offsets of every A_i / B_i and the total element counts. */
 int elemamd_batch_plan_layout(const elemamd_batch_plan *plan, int64_t *a_off, int64_t *b_off, int64_t *a_total,
