@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <new>
 #include <numeric>
 #include <vector>
 
@@ -211,16 +212,21 @@ int batch_set_launch(BatchPlan* P, const int* bucket_grid) {
     if (P == nullptr || bucket_grid == nullptr) return kErrArg;
     for (const BatchBucket& bk : P->buckets)
         if (bucket_grid[bk.index] < 0 || (bucket_grid[bk.index] > 0 && bk.nb > kPersistMaxNb)) return kErrArg;
-    const std::vector<BatchBucket> before = P->buckets;
-    bool same = true;
-    for (BatchBucket& bk : P->buckets) {
-        same = same && bk.grid == bucket_grid[bk.index];
-        bk.grid = bucket_grid[bk.index];
+    std::vector<BatchBucket> before;
+    int rc = kErrHip;
+    try {  // (no exception leaves the C interface)
+        before = P->buckets;
+        bool same = true;
+        for (BatchBucket& bk : P->buckets) {
+            same = same && bk.grid == bucket_grid[bk.index];
+            bk.grid = bucket_grid[bk.index];
+        }
+        if (same) return kOk;
+        rc = plan_runs(P);
+    } catch (const std::bad_alloc&) {
     }
-    if (same) return kOk;
-    const int rc = plan_runs(P);
     if (rc != kOk) {
-        P->buckets = before;
+        if (!before.empty()) P->buckets.swap(before);
         return rc;
     }
     if (P->graph_exec) {  // captured with the previous launch forms and table
